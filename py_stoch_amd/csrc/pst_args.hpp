@@ -100,6 +100,7 @@ struct JobRef {
   static constexpr int kNP = NP, kMP = MP;
   static constexpr int kKP = MP;          // rates per row: one per reaction
   static constexpr bool kCustom = false;  // propensities from the mass-action table
+  static constexpr bool kTable = true;    // table entries are run-time values
   static constexpr int kOutLds = NP < 4 ? NP : 4;  // recorded species gathered in LDS (blocked layout)
   using Dev = JobDev<NP, MP>;
   static constexpr int NW = (NP * MP + 3) / 4;
@@ -142,6 +143,13 @@ struct JobRef {
   }
   __device__ __forceinline__ const JobParams& p() const { return P; }
   __device__ __forceinline__ int V(int i, int j) const { return sbyte(v, i * MP + j); }
+  // V(i, sel) for a run-time sel in [0, MP)
+  __device__ __forceinline__ int Vsel(int i, int sel) const {
+    uint32_t w = v[i * (MP / 4)];
+#pragma unroll
+    for (int r = 1; r < MP / 4; ++r) w = (sel >> 2) == r ? v[i * (MP / 4) + r] : w;
+    return __builtin_amdgcn_sbfe((int)w, (unsigned)(sel & 3) * 8u, 8u);
+  }
   __device__ __forceinline__ int Ord(int i, int j) const { return sbyte(ord, i * MP + j); }
   __device__ __forceinline__ int Stp(int i, int j) const { return sbyte(stp, i * MP + j); }
   __device__ __forceinline__ int Hv(int i) const { return sbyte(H, i); }
@@ -173,6 +181,7 @@ struct FixedRef {
   static constexpr int kNP = Net::N, kMP = Net::M;
   static constexpr int kKP = Net::n_rates;   // rates per row
   static constexpr bool kCustom = Net::custom;  // compiled hazard expressions
+  static constexpr bool kTable = false;         // table entries are constants
   static constexpr int kOutLds = Net::kappa < 4 ? Net::kappa : 4;  // recorded species gathered in LDS
   template <class R>
   __device__ __forceinline__ static void props(const int32_t (&x)[kNP], const R (&c)[kKP], R (&a)[kMP]) {
@@ -184,6 +193,20 @@ struct FixedRef {
   __device__ __forceinline__ void refresh() {}
   __device__ __forceinline__ const FixedParams<Net>& p() const { return P; }
   __device__ __forceinline__ static constexpr int V(int i, int j) { return Net::v[i * kMP + j]; }
+  // bytes V(i, 4 r) .. V(i, 4 r + 3) as one word
+  static constexpr uint32_t Vword(int i, int r) {
+    uint32_t w = 0;
+    for (int b = 0; b < 4; ++b)
+      if (4 * r + b < kMP) w |= ((uint32_t)Net::v[i * kMP + 4 * r + b] & 0xffu) << (8 * b);
+    return w;
+  }
+  // V(i, sel) for a run-time sel in [0, M): a bit-field extract from constants
+  __device__ __forceinline__ static int Vsel(int i, int sel) {
+    uint32_t w = Vword(i, 0);
+#pragma unroll
+    for (int r = 1; r < (kMP + 3) / 4; ++r) w = (sel >> 2) == r ? Vword(i, r) : w;
+    return __builtin_amdgcn_sbfe((int)w, (unsigned)(sel & 3) * 8u, 8u);
+  }
   __device__ __forceinline__ static constexpr int Ord(int i, int j) { return Net::ord[i * kMP + j]; }
   __device__ __forceinline__ static constexpr int Stp(int i, int j) { return Net::stp[i * kMP + j]; }
   __device__ __forceinline__ static constexpr int Hv(int i) { return Net::H[i]; }

@@ -117,6 +117,15 @@ struct Key {
     s_lo = (uint32_t)sim;
     s_hi = (uint32_t)(sim >> 32);
   }
+  // The same simulation's key with the job's seed in scalar registers: inside a
+  // loop the ten round keys are then loop-invariant scalars instead of 18
+  // vector adds per block.
+  __device__ __forceinline__ Key scalar_seed(uint64_t seed) const {
+    Key k = *this;
+    k.k0 = __builtin_amdgcn_readfirstlane((uint32_t)seed);
+    k.k1 = __builtin_amdgcn_readfirstlane((uint32_t)(seed >> 32));
+    return k;
+  }
   __device__ __forceinline__ Words4 block(uint64_t c, uint32_t it) const {
     return philox4x32_10((uint32_t)c, (uint32_t)(c >> 32) | (it << 16), s_lo, s_hi, k0, k1);
   }

@@ -210,9 +210,9 @@ struct StateIO {
 // Engine interface (see EngineF64 / EngineF32):
 //   int  start(job, sim)            -> initial mode, state loaded
 //   int  step<SSA_ONLY>(job, cnt, m) -> next mode (DONE may set flag)
+//   Draw1 ssa_draw(key, c), bool ssa_try(job, draw, tstop, sel, t1): one
+//     ordinary SSA step (ssa_run)
 //   int  flag
-constexpr int SSA_LANES_MIN = 1;
-
 template <class Engine, class Ref>
 __device__ __forceinline__ void finish_sim(const Ref& jr, const Engine& eng, int64_t sim, Counters& cnt,
                                            unsigned long long ev_start) {
@@ -270,6 +270,145 @@ __device__ __forceinline__ int range_stop(const Ref& jr, int f_end) {
   return f_end < jr.p().ita ? f_end : jr.p().ita;
 }
 
+// time of the last sample of the range
+template <class Ref>
+__device__ __forceinline__ double stop_time(const Ref& jr, int f_stop) {
+  return (double)glb(jr.p().I)[f_stop > 0 ? f_stop - 1 : 0];
+}
+
+// value of `v` in the lane with byte address `addr` (4 * lane)
+__device__ __forceinline__ float lane_get(float v, int addr) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(addr, __builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double lane_get(double v, int addr) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(addr, (int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(addr, (int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Ordinary SSA steps (P3.py:73-149, gillespie.py:70-149) of the lanes with
+// `on`, up to `cap` each, in batches of four steps without a branch.  A
+// step is computed from the state and committed by selects only if nothing
+// out of the ordinary happens in it.  A lane leaves the loop before a step
+// that ends the simulation or its range (absorbing state, last sample,
+// count limit, stuck clock, step budget, t_max): `general` is then set and
+// step<true> takes that step.  A lane whose step crosses a sample time stops
+// for the rest of its batch and records the state before that step.
+// The batch's Philox blocks and logarithms do not depend on the state; they
+// are independent chains beside the steps'.  On gfx950 a dependent vector
+// instruction issues every ~9 cycles, a branch on a lane mask costs 50-60: the
+// general step, with about ten of them, takes 1,300 cycles for a single lane.
+// All lanes of the wavefront call this together.
+
+template <class Engine, class Ref>
+__device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int mode, bool on, int cap, double tstop,
+                                       bool& general) {
+  using Out = typename Engine::Out;
+  constexpr int kBatch = 4;
+  const auto& P = jr.p();
+  int lim = cap;
+  if (P.method == 0) lim = eng.burst < lim ? eng.burst : lim;
+  if (P.max_steps != 0u) {
+    const uint32_t left = eng.nsteps < P.max_steps ? P.max_steps - eng.nsteps : 0u;
+    lim = left < (uint32_t)lim ? (int)left : lim;
+  }
+  if (P.method == 2) tstop = P.t_max < tstop ? P.t_max : tstop;
+  // a batch cannot reach the count limit from here
+  bool go = on & (lim > 0) & (eng.t < tstop);
+#pragma unroll
+  for (int i = 0; i < Engine::NP; ++i) go = go & (eng.x[i] < COUNT_LIMIT - 127 * 64);
+  bool stop = on & !go;  // the next step is not for this loop
+  const Key uk = eng.key.scalar_seed(P.seed);  // a lane without a simulation may hold any key
+  int n = 0;
+  while (wave_any(go)) {
+    jr.refresh();
+    typename Engine::Draw1 d[kBatch];
+#pragma unroll
+    for (int s = 0; s < kBatch; ++s) d[s] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + s));
+    bool act = go, crossed = false;
+    int csel = 0;
+#pragma unroll
+    for (int s = 0; s < kBatch; ++s) {
+      int sel;
+      double t1;
+      const bool ok = eng.ssa_try(jr, d[s], tstop, sel, t1);
+      const bool take = act & (n < lim);
+      const bool done = take & ok;
+      stop = stop | (take & !ok);
+      const bool cross = done & (t1 >= eng.tnext);
+      crossed = crossed | cross;
+      csel = cross ? sel : csel;
+#pragma unroll
+      for (int i = 0; i < Engine::NP; ++i) eng.x[i] += done ? jr.Vsel(i, sel) : 0;
+      eng.t = done ? t1 : eng.t;
+      n += done ? 1 : 0;
+      act = done & !cross;
+    }
+    if (wave_any(crossed)) {
+      if (crossed) {
+        do {
+#pragma unroll
+          for (int q = 0; q < Engine::NP; ++q) {
+            if (q < P.kappa) {
+              const int sp = jr.Ev(q);
+              int32_t v = 0;  // the state before the crossing step
+#pragma unroll
+              for (int i = 0; i < Engine::NP; ++i) v |= (eng.x[i] - jr.Vsel(i, csel)) & -(int32_t)(sp == i);
+              Out::put(P, eng.Ob, q, eng.F, v);
+            }
+          }
+          Out::row_done(P, eng.Ob, P.kappa, eng.F);
+          cnt.w.samples += 1;
+          eng.F = eng.F + 1;
+          eng.tnext = (double)glb(P.I)[eng.F];  // t < tstop: F stays below the range's last sample
+        } while (eng.t >= eng.tnext);
+      }
+    }
+    go = go & !stop & (n < lim);
+  }
+  eng.bc += (uint64_t)(uint32_t)n;
+  eng.nsteps += (uint32_t)n;
+  cnt.w.uniforms += 2u * (unsigned int)n;
+  cnt.ssa += (unsigned int)n;
+  cnt.events += (unsigned long long)n;
+  general = stop;
+  if (P.method == 0) {
+    eng.burst -= n;
+    if (on && eng.burst <= 0) mode = MODE_DECIDE;
+  }
+  return mode;
+}
+
+// Up to `cap` SSA steps of every lane in SSA mode: ordinary ones in ssa_run,
+// and the one it leaves over, if any, through step<true>.
+template <class Engine, class Ref>
+__device__ __forceinline__ int ssa_slice(Ref& jr, Engine& eng, int64_t sim, Counters& cnt,
+                                         unsigned long long ev_start, int mode, int cap, int f_stop, double t_stop) {
+  if constexpr (Ref::kTable && Ref::kNP * Ref::kMP > 64) {
+    // the 16 x 16 table: its step is dominated by the walk over the table's
+    // entries and too large to be unrolled (ssa_run: 51 -> 59 ms on six networks)
+    for (int s = 0; s < cap && wave_any(mode == MODE_SSA); ++s) {
+      jr.refresh();
+      if (mode == MODE_SSA) {
+        mode = eng.template step<true>(jr, cnt, mode);
+        mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
+      }
+    }
+    return mode;
+  }
+  bool general;
+  mode = ssa_run(jr, eng, cnt, mode, mode == MODE_SSA, cap, t_stop, general);
+  if (wave_any(general)) {
+    jr.refresh();
+    if (general) {
+      mode = eng.template step<true>(jr, cnt, MODE_SSA);
+      mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
+    }
+  }
+  return mode;
+}
+
 template <class Engine, class Ref>
 __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__ jobs, int n_jobs,
                                            unsigned int* __restrict__ queue, unsigned long long* __restrict__ stats,
@@ -286,6 +425,7 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
   Ref jr;
   jr.load(jobs);
   int f_stop = range_stop(jr, f_end);
+  double t_stop = stop_time(jr, f_stop);
 
   for (;;) {
     // ---- refill lanes whose simulation ended from the job's queue ----
@@ -314,6 +454,7 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
       if (job >= n_jobs) break;
       jr.load(jobs + job);
       f_stop = range_stop(jr, f_end);
+      t_stop = stop_time(jr, f_stop);
       exhausted = false;
       continue;
     }
@@ -325,28 +466,14 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
         mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
       }
       // SSA-only steps while lanes are inside a burst
-      const int slice = jr.p().ssa_slice;
-      for (int s = 0; s < slice; ++s) {
-        if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(mode == MODE_SSA)) < SSA_LANES_MIN) break;
-        jr.refresh();
-        if (mode == MODE_SSA) {
-          mode = eng.template step<true>(jr, cnt, mode);
-          mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-        }
-      }
+      if (wave_any(mode == MODE_SSA))
+        mode = ssa_slice(jr, eng, sim, cnt, ev_start, mode, jr.p().ssa_slice + 1, f_stop, t_stop);
     } else {
       // no lane decides (pure SSA, or every live lane inside a burst): up to
       // 1 + ssa_slice SSA steps before the next refill, 2 + 2 ssa_slice for
       // pure SSA, where no lane waits to decide
-      const int slice = jr.p().method == 2 ? 2 * jr.p().ssa_slice + 1 : jr.p().ssa_slice;
-      for (int s = 0; s <= slice; ++s) {
-        if (!wave_any(mode == MODE_SSA)) break;
-        if (s > 0) jr.refresh();
-        if (mode == MODE_SSA) {
-          mode = eng.template step<true>(jr, cnt, mode);
-          mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-        }
-      }
+      const int cap = jr.p().method == 2 ? 2 * jr.p().ssa_slice + 2 : jr.p().ssa_slice + 1;
+      mode = ssa_slice(jr, eng, sim, cnt, ev_start, mode, cap, f_stop, t_stop);
     }
   }
 
@@ -387,6 +514,7 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
 enum { MODE_AWAY = 3 };
 enum { SLOT_FREE = 0u, SLOT_SENT = 1u, SLOT_BACK = 2u };
 constexpr int PAIR_SLOTS = 256;  // decide lanes per workgroup
+constexpr int BURST_SLICE = 8;   // SSA steps of a burst wavefront between two looks at its slots
 
 __device__ __forceinline__ uint32_t lds_load_acquire(uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -521,6 +649,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     bool busy = false;
     int bjob = -1;
     int f_stop = 0x7fffffff;
+    double t_stop = 0.0;
     for (;;) {
       const bool pick = !busy && lds_load_acquire(&s_state[slot]) == SLOT_SENT;
       const unsigned long long pmask = __builtin_amdgcn_ballot_w64(pick);
@@ -531,6 +660,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
           jr.load(jobs + pj);
           bjob = pj;
           f_stop = range_stop(jr, f_end);
+          t_stop = stop_time(jr, f_stop);
         }
         if (pick) {
           unsigned long long ev;
@@ -545,9 +675,13 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         __builtin_amdgcn_s_sleep(4);
         continue;
       }
-      jr.refresh();
+      bool general;
+      int m = ssa_run(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, general);
+      if (wave_any(general)) {
+        jr.refresh();
+        if (general) m = eng.template step<true>(jr, cnt, MODE_SSA);
+      }
       if (busy) {
-        int m = eng.template step<true>(jr, cnt, MODE_SSA);
         if (m == MODE_DONE) m = settle(jr, eng, sim, cnt, ev_start, m, f_stop);
         // back to the decide lane at the burst's end, or at the range's
         // last sample (the decide lane saves it)

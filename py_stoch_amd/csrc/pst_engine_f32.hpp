@@ -452,6 +452,34 @@ struct EngineF32 {
     return MODE_DECIDE;
   }
 
+  // The random numbers of one SSA step: -ln(rho1) and rho2.
+  struct Draw1 {
+    float nl, u;
+  };
+  static __device__ __forceinline__ Draw1 ssa_draw(const Key& uk, uint64_t c) {
+    const Words4 w = uk.block(c, 0);
+    return {-fast_log(u24(w.w0)), u24(w.w1)};
+  }
+  static __device__ __forceinline__ Draw1 from_lane(const Draw1& d, int addr) { return {lane_get(d.nl, addr), lane_get(d.u, addr)}; }
+
+  // One SSA step from state (x, t) with draw d: the reaction and the new time;
+  // false if the step needs step<true> (see ssa_run).  step<true>'s
+  // arithmetic; a0 = 0 gives an infinite or undefined time, which fails.
+  __device__ __forceinline__ bool ssa_try(const Ref& tab, const Draw1& d, double tstop, int& sel, double& t1) const {
+    float a[MP];
+    propensities_f32<Ref>(tab, k, x, a);
+    double cum[MP];
+#pragma unroll
+    for (int j = 0; j < MP; ++j) cum[j] = (j > 0 ? cum[j > 0 ? j - 1 : 0] : 0.0) + (double)a[j];
+    const double asum = cum[MP - 1];
+    t1 = t + (double)(d.nl * fast_rcp((float)asum));
+    const double target = (double)d.u * asum;  // <= asum: the last sum always reaches it
+    sel = 0;
+#pragma unroll
+    for (int j = 0; j < MP - 1; ++j) sel += (cum[j] < target) ? 1 : 0;
+    return (t1 > t) & (t1 < tstop);
+  }
+
   // Poisson leap with tau halving (P1_P2.py:222-259,509-540).  Every draw is
   // an inversion of the Poisson CDF at one 24-bit uniform: reaction j reads
   // word j % 4 of block grp + j / 4 (so one block serves four reactions);

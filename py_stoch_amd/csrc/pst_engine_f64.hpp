@@ -400,6 +400,49 @@ struct EngineF64 {
     return MODE_DECIDE;
   }
 
+  // The random numbers of one SSA step: ln(1 / rho1) and rho2.
+  struct Draw1 {
+    double lr, rho;
+  };
+  static __device__ __forceinline__ Draw1 ssa_draw(const Key& uk, uint64_t c) {
+    const Words4 w = uk.block(c, 0);
+    return {log_f64(1.0 / u53(w.w0, w.w1)), u53(w.w2, w.w3)};
+  }
+  static __device__ __forceinline__ Draw1 from_lane(const Draw1& d, int addr) { return {lane_get(d.lr, addr), lane_get(d.rho, addr)}; }
+
+  // One SSA step from state (x, t) with draw d: the reaction and the new time;
+  // false if the step needs step<true> (see ssa_run).  The waiting time is
+  // step<true>'s expression; its reaction choice, the first j with
+  // sum_{r<=j} fl(a_r / asum) >= rho, is taken from the running sums against
+  // rho * asum instead of M divisions.  Both sums of up to 32 non-negative
+  // terms are within 1e-13 of the exact ones relative to asum, so outside a
+  // band of 1e-12 asum around a running sum both pick the same reaction; inside
+  // it (one step in ~10^11) step<true> decides.
+  __device__ __forceinline__ bool ssa_try(const Ref& tab, const Draw1& d, double tstop, int& sel, double& t1) const {
+    double a[MP];
+    propensities_f64<Ref>(tab, k, x, a);
+    double cum[MP];
+    uint32_t sign = 0u;  // of any propensity
+#pragma unroll
+    for (int j = 0; j < MP; ++j) {
+      cum[j] = (j > 0 ? cum[j > 0 ? j - 1 : 0] : 0.0) + a[j];
+      sign |= (uint32_t)(__builtin_bit_cast(uint64_t, a[j]) >> 32);
+    }
+    const double asum = cum[MP - 1];
+    t1 = t + (1.0 / asum) * d.lr;
+    const double target = d.rho * asum;
+    const double band = 1e-12 * asum;
+    bool ok = (t1 > t) & (t1 < tstop) & (asum > 1e-280) & (asum < 1e280) & ((int32_t)sign >= 0);
+    sel = 0;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) {
+      const double gap = cum[j] - target;
+      sel += (gap < 0.0) ? 1 : 0;
+      ok = ok & (__builtin_fabs(gap) > band);
+    }
+    return ok;
+  }
+
   // Poisson leap with tau halving (P1_P2.py:222-259,509-540).  K holds the
   // critical firing (if any) on entry and the accepted counts on return; tau
   // is halved in place, and the clock advances by the tau of the accepted
