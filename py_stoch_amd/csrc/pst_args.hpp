@@ -1,10 +1,10 @@
 // pst_args.hpp -- kernel argument blocks shared by the launch code and the kernels.
 //
-// A network is passed to the kernels as a dense, zero-padded species x reaction
-// table (NetTab) inside a job descriptor in device memory: every entry is the same for
-// all lanes of a launch, so the compiler reads it with scalar loads into SGPRs
-// and every branch on it is a scalar branch.  Per-simulation data (state, time,
-// sample cursor, Philox counter) lives in VGPRs for the whole run.
+// A network is passed to the table-driven kernels as lists of its non-zero
+// entries (NetTab) inside a job descriptor in device memory: every entry is the
+// same for all lanes of a wavefront, so every branch on it is a scalar branch.
+// Per-simulation data (state, time, sample cursor, Philox counter) lives in
+// VGPRs for the whole run.
 #pragma once
 #ifndef __HIPCC_RTC__
 #include <stdint.h>
@@ -13,18 +13,22 @@
 
 namespace pst {
 
-// Dense network table with capacity NP species x MP reactions.  Rows beyond N
-// and columns beyond M are zero, which makes them inert in every loop.
+#ifndef __HIPCC_RTC__  // (the table-driven kernels are built with the library)
+// Network table of a size class (capacity NP species x MP reactions) as lists
+// of its non-zero entries, species ascending within a reaction.
 template <int NP, int MP>
 struct NetTab {
-  int8_t v[NP * MP];    // net change V = Post - Pre, species-major (d_V, P1_P2.py:8)
-  int8_t ord[NP * MP];  // number of propensity factors of species i in reaction j
-  int8_t stp[NP * MP];  // factor step: 1 -> x(x-1)(x-2)..., 0 -> x^p
-  int8_t H[NP];         // highest order of reaction (d_H, P1_P2.py:9)
-  int8_t Ht[NP];        // d_H_type (P1_P2.py:10)
-  int8_t irs[NP];       // 1 if the species has any Pre entry (I_rs, P1_P2.py:338-346)
-  int8_t E[NP];         // recorded species (d_E, P1_P2.py:13)
+  uint16_t fac[NP * MP];   // propensity factors, reaction by reaction: species | step << 5 | last of
+                           // its reaction << 6 | order << 8 (order factors of the species, step 1:
+                           // x(x-1)(x-2)..., 0: x^order; order 0: a reaction without factors)
+  uint16_t vent[NP * MP];  // net changes V = Post - Pre (d_V, P1_P2.py:8): species | (uint8) value << 8
+  uint32_t vrange[MP];     // reaction j's net changes: first | end << 16
+  uint32_t species[NP];    // H (d_H, P1_P2.py:9) | H_type << 8 (P1_P2.py:10) | 1 << 16 if the species has any
+                           // Pre entry (I_rs, P1_P2.py:338-346) | recorded species E[i] << 24 (d_E, P1_P2.py:13)
+  int8_t vrow[MP * NP];    // V once more, dense and reaction-major: the change of every species by reaction j
 };
+
+#endif
 
 enum StatIdx {
   ST_EVENTS = 0, ST_LEAPS, ST_REJECTED, ST_SSA, ST_FLAGGED,
@@ -82,19 +86,35 @@ __device__ __forceinline__ void load_params_vgpr(JobParams* dst, const JobParams
   __builtin_memcpy(dst, w, sizeof(JobParams));
 }
 
+#ifndef __HIPCC_RTC__
 template <int NP, int MP>
 struct JobDev {
   NetTab<NP, MP> tab;
   JobParams p;
 };
 
-// Kernel-side view of the current job.  The table bytes are copied four to a
-// 32-bit word into SGPRs and hidden from the optimizer at the top of every
-// pass of the simulation loop (refresh(): an empty asm on a VGPR copy, then
-// readfirstlane), so the per-use byte extracts stay cheap scalar bit-field
-// extracts inside the loop instead of ~64 hoisted, long-lived SGPRs that
-// spill.  Scalar loads inside the loop are avoided: with one wavefront per
-// SIMD their latency is not hidden.
+#endif
+
+// v[i] for a wavefront-uniform i: a register picked by index (through a vector
+// value, so that the array itself stays in registers)
+template <class T, int N>
+__device__ __forceinline__ T at(const T (&v)[N], int i) {
+  typedef T Vec __attribute__((ext_vector_type(N)));
+  Vec w;
+#pragma unroll
+  for (int q = 0; q < N; ++q) w[q] = v[q];
+  return w[i];
+}
+
+#ifndef __HIPCC_RTC__
+// Kernel-side view of the current job of a table-driven kernel.  The lists are
+// held in vector registers, one word per lane, and read one word at a time
+// into a scalar register (v_readlane); loops over reactions and their entries
+// are rolled, so the code has the size of one entry, whatever the class.  (A
+// dense byte table in scalar registers with every loop unrolled came to 84 KB
+// of code for 4 x 4 and 300 KB for 16 x 16, beyond the 64 KB instruction
+// cache, and walked the zero entries too.)  The net changes of a reaction
+// chosen per lane are read from a dense copy in LDS.
 template <int NP, int MP>
 struct JobRef {
   static constexpr int kNP = NP, kMP = MP;
@@ -103,60 +123,173 @@ struct JobRef {
   static constexpr bool kTable = true;    // table entries are run-time values
   static constexpr int kOutLds = NP < 4 ? NP : 4;  // recorded species gathered in LDS (blocked layout)
   using Dev = JobDev<NP, MP>;
-  static constexpr int NW = (NP * MP + 3) / 4;
-  static constexpr int NS = (NP + 3) / 4;
-  uint32_t v[NW], ord[NW], stp[NW];
-  uint32_t H[NS], Ht[NS], irs[NS], E[NS];
+  static constexpr int EW = (NP * MP / 2 + 63) / 64;  // registers of an entry list
+  uint32_t fac[EW], vent[EW], vrange, species;
   JobParams P;
 
+  static __device__ __forceinline__ uint32_t* rows() {
+    __shared__ uint32_t buf[4 * NP * MP / 4];
+    return buf + (threadIdx.x >> 6) * (NP * MP / 4);
+  }
   __device__ __forceinline__ void load(const JobDev<NP, MP>* jd) {
-    __builtin_memcpy(v, jd->tab.v, sizeof(jd->tab.v));
-    __builtin_memcpy(ord, jd->tab.ord, sizeof(jd->tab.ord));
-    __builtin_memcpy(stp, jd->tab.stp, sizeof(jd->tab.stp));
-    __builtin_memcpy(H, jd->tab.H, sizeof(jd->tab.H));
-    __builtin_memcpy(Ht, jd->tab.Ht, sizeof(jd->tab.Ht));
-    __builtin_memcpy(irs, jd->tab.irs, sizeof(jd->tab.irs));
-    __builtin_memcpy(E, jd->tab.E, sizeof(jd->tab.E));
+    const int lane = (int)(threadIdx.x & 63u);
+    const uint32_t* f = reinterpret_cast<const uint32_t*>(jd->tab.fac);
+    const uint32_t* v = reinterpret_cast<const uint32_t*>(jd->tab.vent);
+#pragma unroll
+    for (int r = 0; r < EW; ++r) {
+      const int w = r * 64 + lane;
+      fac[r] = w < NP * MP / 2 ? f[w] : 0u;
+      vent[r] = w < NP * MP / 2 ? v[w] : 0u;
+    }
+    vrange = lane < MP ? jd->tab.vrange[lane] : 0u;
+    species = lane < NP ? jd->tab.species[lane] : 0u;
+    const uint32_t* d = reinterpret_cast<const uint32_t*>(jd->tab.vrow);
+    if (lane < NP * MP / 4) rows()[lane] = d[lane];  // NP * MP / 4 <= 64; read by this wavefront only
     load_params_vgpr(&P, &jd->p);
   }
-  static __device__ __forceinline__ uint32_t opaque(uint32_t w) {
-    asm volatile("" : "+v"(w));
-    return __builtin_amdgcn_readfirstlane(w);
-  }
-  __device__ __forceinline__ void refresh() {
+  static __device__ __forceinline__ uint32_t word(uint32_t v, int i) { return (uint32_t)__builtin_amdgcn_readlane((int)v, i); }
+  static __device__ __forceinline__ uint32_t entry(const uint32_t (&v)[EW], int e) {
+    uint32_t w = word(v[0], (e >> 1) & 63);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      v[w] = opaque(v[w]);
-      ord[w] = opaque(ord[w]);
-      stp[w] = opaque(stp[w]);
-    }
-#pragma unroll
-    for (int w = 0; w < NS; ++w) {
-      H[w] = opaque(H[w]);
-      Ht[w] = opaque(Ht[w]);
-      irs[w] = opaque(irs[w]);
-      E[w] = opaque(E[w]);
-    }
-  }
-  static __device__ __forceinline__ int sbyte(const uint32_t* w, int idx) {
-    return (int)(int8_t)(w[idx >> 2] >> (8 * (idx & 3)));
+    for (int r = 1; r < EW; ++r) w = (e >> 7) == r ? word(v[r], (e >> 1) & 63) : w;
+    return (e & 1) ? w >> 16 : w & 0xffffu;
   }
   __device__ __forceinline__ const JobParams& p() const { return P; }
-  __device__ __forceinline__ int V(int i, int j) const { return sbyte(v, i * MP + j); }
-  // V(i, sel) for a run-time sel in [0, MP)
-  __device__ __forceinline__ int Vsel(int i, int sel) const {
-    uint32_t w = v[i * (MP / 4)];
-#pragma unroll
-    for (int r = 1; r < MP / 4; ++r) w = (sel >> 2) == r ? v[i * (MP / 4) + r] : w;
-    return __builtin_amdgcn_sbfe((int)w, (unsigned)(sel & 3) * 8u, 8u);
+  __device__ __forceinline__ int n_reactions() const { return __builtin_amdgcn_readfirstlane(P.M); }
+  __device__ __forceinline__ int n_species() const { return __builtin_amdgcn_readfirstlane(P.N); }
+  __device__ __forceinline__ int n_recorded() const { return __builtin_amdgcn_readfirstlane(P.kappa); }
+  __device__ __forceinline__ int method() const { return __builtin_amdgcn_readfirstlane(P.method); }
+  __device__ __forceinline__ int Hv(int i) const { return (int)(word(species, i) & 0xffu); }
+  __device__ __forceinline__ int Htv(int i) const { return (int)((word(species, i) >> 8) & 0xffu); }
+  __device__ __forceinline__ bool Irs(int i) const { return (word(species, i) >> 16) & 1u; }
+  __device__ __forceinline__ int Ev(int q) const { return (int)(word(species, q) >> 24); }
+
+  // body(i) for every species, rolled (i is wavefront-uniform: index arrays with at())
+  template <class F>
+  __device__ __forceinline__ void for_species(F body) const {
+    const int n = n_species();
+#pragma unroll 1
+    for (int i = 0; i < n; ++i) body(i);
   }
-  __device__ __forceinline__ int Ord(int i, int j) const { return sbyte(ord, i * MP + j); }
-  __device__ __forceinline__ int Stp(int i, int j) const { return sbyte(stp, i * MP + j); }
-  __device__ __forceinline__ int Hv(int i) const { return sbyte(H, i); }
-  __device__ __forceinline__ int Htv(int i) const { return sbyte(Ht, i); }
-  __device__ __forceinline__ int Irs(int i) const { return sbyte(irs, i); }
-  __device__ __forceinline__ int Ev(int q) const { return sbyte(E, q); }
+  template <class F>
+  __device__ __forceinline__ void for_recorded(F body) const {
+    const int n = n_recorded();
+#pragma unroll 1
+    for (int q = 0; q < n; ++q) body(q);
+  }
+
+  // propensities a_j = k_j * product of factors (UpdatePropensities, parser.py:32-55)
+  template <class R>
+  __device__ __forceinline__ void props(const int32_t (&x)[NP], const R (&k)[MP], R (&a)[MP]) const {
+    typedef R RVec __attribute__((ext_vector_type(MP)));
+    RVec av;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) av[j] = (R)0;
+    const int n = n_reactions();
+    R v = k[0];
+    // one trip per listed factor
+#pragma unroll 1
+    for (int e = 0, j = 0; j < n; ++e) {
+      const uint32_t w = entry(fac, e);
+      const int order = (int)(w >> 8);
+      if (order > 0) {
+        const int32_t xi = at<int32_t, NP>(x, (int)(w & 31u));
+        v = v * (R)xi;
+        if (order > 1) {
+          const int step = (int)((w >> 5) & 1u);
+          for (int q = 1; q < order; ++q) v = v * (R)(xi - step * q);
+        }
+      }
+      if (w & 64u) {
+        av[j] = v;
+        j += 1;
+        v = at<R, MP>(k, j & (MP - 1));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < MP; ++j) a[j] = av[j];
+  }
+
+  // critical reactions (P1_P2.py:314-327, on V) as a bit mask; mu and sigma^2
+  // of every species over the non-critical reactions and whether it has any
+  // (P1_P2.py:330-383)
+  template <class R>
+  __device__ __forceinline__ void sums(const int32_t (&x)[NP], const R (&a)[MP], int n_c, unsigned& crit, R (&mu)[NP],
+                                       R (&s2)[NP], unsigned& any) const {
+    typedef R RVec __attribute__((ext_vector_type(NP)));
+    RVec m, s;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      m[i] = (R)0;
+      s[i] = (R)0;
+    }
+    crit = 0u;
+    any = 0u;
+    const int n = n_reactions();
+#pragma unroll 1
+    for (int j = 0; j < n; ++j) {
+      const uint32_t vr = word(vrange, j);
+      const int e0 = (int)(vr & 0xffffu), e1 = (int)(vr >> 16);
+      bool c = false;
+#pragma unroll 1
+      for (int e = e0; e < e1; ++e) {
+        const uint32_t w = entry(vent, e);
+        const int v = (int)(int8_t)(w >> 8);
+        if (v < 0) c = c | ((-v) * n_c > at<int32_t, NP>(x, (int)(w & 31u)));
+      }
+      crit |= c ? (1u << j) : 0u;
+      const R aj = at<R, MP>(a, j);
+#pragma unroll 1
+      for (int e = e0; e < e1; ++e) {
+        const uint32_t w = entry(vent, e);
+        const int i = (int)(w & 31u), v = (int)(int8_t)(w >> 8);
+        m[i] += c ? (R)0 : (R)v * aj;
+        s[i] += c ? (R)0 : (R)(v * v) * aj;
+        any |= c ? 0u : (1u << i);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      mu[i] = m[i];
+      s2[i] = s[i];
+    }
+  }
+
+  // s = x + V K
+  __device__ __forceinline__ void advance(const int32_t (&x)[NP], const int32_t (&K)[MP], int64_t (&s)[NP]) const {
+    typedef int64_t LVec __attribute__((ext_vector_type(NP)));
+    LVec t;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) t[i] = x[i];
+    const int n = n_reactions();
+#pragma unroll 1
+    for (int j = 0; j < n; ++j) {
+      const uint32_t vr = word(vrange, j);
+      const int e1 = (int)(vr >> 16);
+      const int64_t kj = at<int32_t, MP>(K, j);
+#pragma unroll 1
+      for (int e = (int)(vr & 0xffffu); e < e1; ++e) {
+        const uint32_t w = entry(vent, e);
+        t[(int)(w & 31u)] += kj * (int)(int8_t)(w >> 8);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) s[i] = t[i];
+  }
+
+  // d = V(., sel) for a per-lane sel in [0, MP)
+  __device__ __forceinline__ void row(int sel, int32_t (&d)[NP]) const {
+    const uint32_t* r = rows() + sel * (NP / 4);
+#pragma unroll
+    for (int w = 0; w < NP / 4; ++w) {
+      const int32_t b = (int32_t)r[w];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[4 * w + q] = __builtin_amdgcn_sbfe(b, 8 * q, 8);
+    }
+  }
 };
+
+#endif  // !__HIPCC_RTC__
 
 // Kernel-side view of a job whose network is compiled into the kernel (the
 // library generates `Net` and compiles it at run time, as the reference
@@ -183,16 +316,11 @@ struct FixedRef {
   static constexpr bool kCustom = Net::custom;  // compiled hazard expressions
   static constexpr bool kTable = false;         // table entries are constants
   static constexpr int kOutLds = Net::kappa < 4 ? Net::kappa : 4;  // recorded species gathered in LDS
-  template <class R>
-  __device__ __forceinline__ static void props(const int32_t (&x)[kNP], const R (&c)[kKP], R (&a)[kMP]) {
-    Net::template props<R>(x, c, a);
-  }
   using Dev = JobParams;
   FixedParams<Net> P;
   __device__ __forceinline__ void load(const JobParams* jp) { load_params_vgpr(&P, jp); }
-  __device__ __forceinline__ void refresh() {}
   __device__ __forceinline__ const FixedParams<Net>& p() const { return P; }
-  __device__ __forceinline__ static constexpr int V(int i, int j) { return Net::v[i * kMP + j]; }
+  __device__ __forceinline__ static constexpr int method() { return Net::method; }
   // bytes V(i, 4 r) .. V(i, 4 r + 3) as one word
   static constexpr uint32_t Vword(int i, int r) {
     uint32_t w = 0;
@@ -200,19 +328,91 @@ struct FixedRef {
       if (4 * r + b < kMP) w |= ((uint32_t)Net::v[i * kMP + 4 * r + b] & 0xffu) << (8 * b);
     return w;
   }
-  // V(i, sel) for a run-time sel in [0, M): a bit-field extract from constants
-  __device__ __forceinline__ static int Vsel(int i, int sel) {
-    uint32_t w = Vword(i, 0);
-#pragma unroll
-    for (int r = 1; r < (kMP + 3) / 4; ++r) w = (sel >> 2) == r ? Vword(i, r) : w;
-    return __builtin_amdgcn_sbfe((int)w, (unsigned)(sel & 3) * 8u, 8u);
-  }
-  __device__ __forceinline__ static constexpr int Ord(int i, int j) { return Net::ord[i * kMP + j]; }
-  __device__ __forceinline__ static constexpr int Stp(int i, int j) { return Net::stp[i * kMP + j]; }
+  __device__ __forceinline__ static constexpr int V(int i, int j) { return Net::v[i * kMP + j]; }
   __device__ __forceinline__ static constexpr int Hv(int i) { return Net::H[i]; }
   __device__ __forceinline__ static constexpr int Htv(int i) { return Net::Ht[i]; }
   __device__ __forceinline__ static constexpr int Irs(int i) { return Net::irs[i]; }
   __device__ __forceinline__ static constexpr int Ev(int q) { return Net::E[q]; }
+  template <class F>
+  __device__ __forceinline__ static void for_species(F body) {
+#pragma unroll
+    for (int i = 0; i < kNP; ++i) body(i);
+  }
+  template <class F>
+  __device__ __forceinline__ static void for_recorded(F body) {
+#pragma unroll
+    for (int q = 0; q < Net::kappa; ++q) body(q);
+  }
+  // the same operations as JobRef's, in straight-line code
+  template <class R>
+  __device__ __forceinline__ static void props(const int32_t (&x)[kNP], const R (&k)[kKP], R (&a)[kMP]) {
+    if constexpr (kCustom) {
+      Net::template props<R>(x, k, a);  // compiled hazard expressions
+    } else {
+#pragma unroll
+      for (int j = 0; j < kMP; ++j) {
+        R v = k[j];
+#pragma unroll
+        for (int i = 0; i < kNP; ++i)
+          for (int q = 0; q < Net::ord[i * kMP + j]; ++q) v = v * (R)(x[i] - Net::stp[i * kMP + j] * q);
+        a[j] = v;
+      }
+    }
+  }
+  template <class R>
+  __device__ __forceinline__ static void sums(const int32_t (&x)[kNP], const R (&a)[kMP], int n_c, unsigned& crit,
+                                              R (&mu)[kNP], R (&s2)[kNP], unsigned& any) {
+    crit = 0u;
+    any = 0u;
+    bool cr[kMP];
+#pragma unroll
+    for (int j = 0; j < kMP; ++j) {
+      bool c = false;
+#pragma unroll
+      for (int i = 0; i < kNP; ++i)
+        if (V(i, j) < 0) c = c | (-V(i, j) * n_c > x[i]);
+      cr[j] = c;
+      crit |= c ? (1u << j) : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kNP; ++i) {
+      R m = (R)0, s = (R)0;
+      bool some = false;
+#pragma unroll
+      for (int j = 0; j < kMP; ++j) {
+        const int v = V(i, j);
+        if (v != 0) {
+          const bool nc = !cr[j];
+          m += nc ? (R)v * a[j] : (R)0;
+          s += nc ? (R)(v * v) * a[j] : (R)0;
+          some = some | nc;
+        }
+      }
+      mu[i] = m;
+      s2[i] = s;
+      any |= some ? (1u << i) : 0u;
+    }
+  }
+  __device__ __forceinline__ static void advance(const int32_t (&x)[kNP], const int32_t (&K)[kMP], int64_t (&s)[kNP]) {
+#pragma unroll
+    for (int i = 0; i < kNP; ++i) {
+      int64_t t = x[i];
+#pragma unroll
+      for (int j = 0; j < kMP; ++j)
+        if (V(i, j) != 0) t += (int64_t)K[j] * V(i, j);
+      s[i] = t;
+    }
+  }
+  // bit-field extracts from constants
+  __device__ __forceinline__ static void row(int sel, int32_t (&d)[kNP]) {
+#pragma unroll
+    for (int i = 0; i < kNP; ++i) {
+      uint32_t w = Vword(i, 0);
+#pragma unroll
+      for (int r = 1; r < (kMP + 3) / 4; ++r) w = (sel >> 2) == r ? Vword(i, r) : w;
+      d[i] = __builtin_amdgcn_sbfe((int)w, (unsigned)(sel & 3) * 8u, 8u);
+    }
+  }
 };
 
 #ifndef __HIPCC_RTC__
@@ -233,36 +433,41 @@ constexpr int CLASS_MP[NUM_CLASSES] = {4, 8, 16};
 
 template <int NP, int MP>
 inline NetTab<NP, MP> make_tab(const HostNet& h) {
-  NetTab<NP, MP> t;
-  for (int i = 0; i < NP * MP; ++i) { t.v[i] = 0; t.ord[i] = 0; t.stp[i] = 0; }
-  for (int i = 0; i < NP; ++i) { t.H[i] = 0; t.Ht[i] = 0; t.irs[i] = 0; t.E[i] = 0; }
-  for (int i = 0; i < h.N; ++i) {
-    for (int j = 0; j < h.M; ++j) {
-      t.v[i * MP + j] = h.v[i * h.M + j];
-      t.ord[i * MP + j] = h.ord[i * h.M + j];
-      t.stp[i * MP + j] = h.stp[i * h.M + j];
+  NetTab<NP, MP> t = {};
+  int nf = 0, nv = 0;
+  for (int j = 0; j < h.M; ++j) {
+    const int v0 = nv;
+    int last = -1;
+    for (int i = 0; i < h.N; ++i) {
+      const int p = h.ord[i * h.M + j], v = h.v[i * h.M + j];
+      if (p > 0) t.fac[last = nf++] = (uint16_t)(i | (h.stp[i * h.M + j] ? 1 << 5 : 0) | (p << 8));
+      if (v != 0) t.vent[nv++] = (uint16_t)(i | (((unsigned)v & 0xffu) << 8));
+      t.vrow[j * NP + i] = (int8_t)v;
     }
-    t.H[i] = h.H[i];
-    t.Ht[i] = h.Ht[i];
-    t.irs[i] = h.irs[i];
+    if (last < 0) t.fac[last = nf++] = 0;
+    t.fac[last] |= 1 << 6;
+    t.vrange[j] = (uint32_t)v0 | ((uint32_t)nv << 16);
   }
-  for (int q = 0; q < h.kappa; ++q) t.E[q] = h.E[q];
+  for (int i = 0; i < h.N; ++i)
+    t.species[i] = (uint32_t)h.H[i] | ((uint32_t)h.Ht[i] << 8) | ((uint32_t)(h.irs[i] != 0) << 16) |
+                   (i < h.kappa ? (uint32_t)h.E[i] << 24 : 0u);
   return t;
 }
 
 // Launchers, one per translation unit (precision).  `jobs` is a device array
 // of JobDev<NP,MP> for the size class `cls`, `queue` n_jobs zeroed counters,
-// `waves` the number of wavefronts to launch.
+// `waves` the number of wavefronts to launch, `group` whether their jobs have
+// fewer than 64 simulations per wavefront (a group of lanes per simulation).
 int launch_fp64(int cls, const void* jobs, int n_jobs, unsigned int* queue, unsigned long long* stats,
-                int waves, Range range, hipStream_t stream);
+                int waves, Range range, bool group, hipStream_t stream);
 int launch_mixed(int cls, const void* jobs, int n_jobs, unsigned int* queue, unsigned long long* stats,
-                 int waves, Range range, hipStream_t stream);
+                 int waves, Range range, bool group, hipStream_t stream);
 // the mixed-precision Poisson sampler on given means and words (validation)
 int launch_poisson_probe(const float* lam, const uint32_t* words, int64_t n, int32_t* k, int32_t* path,
                          hipStream_t stream);
 // resident 256-lane blocks per CU for a class (occupancy)
-int blocks_per_cu_fp64(int cls);
-int blocks_per_cu_mixed(int cls);
+int blocks_per_cu_fp64(int cls, bool group);
+int blocks_per_cu_mixed(int cls, bool group);
 
 // the large-network kernel (one wavefront per simulation, mixed precision):
 // `jobs` is a device array of WaveJob
@@ -271,6 +476,10 @@ int launch_wave(const void* jobs, int n_jobs, unsigned int* queue, unsigned long
                 hipStream_t stream);
 int blocks_per_cu_wave();
 bool make_wave_tab(const HostNet& h, WaveTab* t, char* why, size_t why_len);
+
+// kernel of a size class: 2 cls, or 2 cls + 1 for the group form (the 16 x 16
+// table has none: its code for one simulation per lane is large already)
+inline int table_form(int cls, bool group) { return 2 * cls + (group && cls < 2 ? 1 : 0); }
 
 // smallest compiled size class holding (N, M, kappa), or -1
 inline int size_class(int N, int M, int kappa) {

@@ -368,17 +368,21 @@ constexpr int kOccupancyWaves = 3;
 // counters, and no result depends on the order.
 constexpr int kSideStreams = 3;
 
+// builds of a specialised kernel: one simulation per lane, the same for
+// kOccupancyWaves wavefronts per SIMD, decide + burst wavefronts, a group of
+// lanes per simulation
+enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_PAIR, BUILD_GROUP, NUM_BUILDS };
+struct FixedBuild {
+  std::string source;
+  pst::RtcForm form = pst::RTC_PLAIN;
+  pst::RtcKernel k;  // compiled on first need
+  bool tried = false;
+};
+
 // jobs sharing one specialised kernel (same network and constant settings)
 struct FixedGroup {
-  pst::RtcKernel k;
-  std::string occ_source;   // source of the occupancy build
-  pst::RtcKernel k_occ;     // compiled on first need
-  bool occ_tried = false;
-  bool use_occ = false;     // this execute launches k_occ
-  std::string pair_source;  // source of the paired build (decide + burst wavefronts)
-  pst::RtcKernel k_pair;    // compiled on first need
-  bool pair_tried = false;
-  bool use_pair = false;    // this execute launches k_pair
+  FixedBuild build[NUM_BUILDS];
+  int use = BUILD_PLAIN;  // the build this execute launches
   std::vector<int> jobs;
   void* d_jobs = nullptr;
   size_t d_bytes = 0;
@@ -417,6 +421,17 @@ struct pst_plan {
   hipEvent_t join[kSideStreams] = {};
 };
 
+// the build's kernel, compiled on first need
+static int fixed_kernel(FixedBuild& b, int precision, const char* what) {
+  if (!b.tried) {
+    std::string err;
+    const int rc = pst::rtc_kernel(b.source, precision, &b.k, &err, b.form);
+    if (rc != PST_OK) return fail(rc, "%s%s", what, err.c_str());
+    b.tried = true;
+  }
+  return PST_OK;
+}
+
 // resident 256-lane blocks per CU for a kernel whose occupancy limit is bpc,
 // after the plan's waves_trim (one block = one wavefront per SIMD)
 static int trimmed(int bpc, int trim) { return std::max(1, bpc - trim); }
@@ -445,15 +460,19 @@ static int enqueue_launches(pst_plan* p, const int* count, int n_wave, int64_t w
     if (count[c] == 0) continue;
     const hipStream_t ls = next_stream();
     int64_t need = 0;
-    for (const PlanJob& pj : p->jobs)
-      if (pj.cls == c) need += ((int64_t)pj.p.n_sims + pj.p.lanes - 1) / pj.p.lanes;
-    const int bpc = (p->precision == PST_PRECISION_MIXED) ? pst::blocks_per_cu_mixed(c) : pst::blocks_per_cu_fp64(c);
+    bool group = false;  // one lane count per class
+    for (const PlanJob& pj : p->jobs) {
+      if (pj.cls != c) continue;
+      need += ((int64_t)pj.p.n_sims + pj.p.lanes - 1) / pj.p.lanes;
+      group = pj.p.lanes < 64;
+    }
+    const bool mixed = p->precision == PST_PRECISION_MIXED;
+    const int bpc = mixed ? pst::blocks_per_cu_mixed(c, group) : pst::blocks_per_cu_fp64(c, group);
     const int64_t resident = (int64_t)trimmed(bpc, p->waves_trim) * p->cu_count * 4;
     const int waves = (int)(need < resident ? need : resident);
     // the queue counters of this class's jobs are queue[qoff .. qoff + count)
-    const int rc = (p->precision == PST_PRECISION_MIXED)
-                       ? pst::launch_mixed(c, p->d_jobs[c], count[c], p->d_queue + qoff, p->d_stats, waves, range, ls)
-                       : pst::launch_fp64(c, p->d_jobs[c], count[c], p->d_queue + qoff, p->d_stats, waves, range, ls);
+    const auto launch = mixed ? pst::launch_mixed : pst::launch_fp64;
+    const int rc = launch(c, p->d_jobs[c], count[c], p->d_queue + qoff, p->d_stats, waves, range, group, ls);
     if (rc < 0) return fail(PST_ETOOLARGE, "no compiled kernel for size class %d", c);
     if (rc != 0) return hip_fail((hipError_t)rc, "simulation kernel launch");
     qoff += count[c];
@@ -461,7 +480,7 @@ static int enqueue_launches(pst_plan* p, const int* count, int n_wave, int64_t w
   for (FixedGroup& g : p->fixed) {
     int64_t need = 0;
     for (int q : g.jobs) need += ((int64_t)p->jobs[q].p.n_sims + p->jobs[q].p.lanes - 1) / p->jobs[q].p.lanes;
-    const pst::RtcKernel* k = g.use_pair ? &g.k_pair : g.use_occ ? &g.k_occ : &g.k;
+    const pst::RtcKernel* k = &g.build[g.use].k;
     const int64_t resident = (int64_t)trimmed(k->blocks_per_cu, p->waves_trim) * p->cu_count * 4;
     const int waves = (int)(need < resident ? need : resident);
     const int cnt = (int)g.jobs.size();
@@ -693,23 +712,33 @@ int pst_batch_plan_create(const pst_job* jobs, int32_t n_jobs, pst_plan** out) {
     P.x0 = pj.d_x0;
     P.I = pj.d_I;
     if (kinds[q] == KIND_FIXED) {
-      pst::RtcKernel k;
-      std::string err;
-      const int rc2 = pst::rtc_kernel(pst::rtc_source(pj.net, P, p->precision, pj.hazards), p->precision, &k, &err);
-      if (rc2 != PST_OK) {
-        pst_plan_destroy(p);
-        return fail(rc2, "job %d: %s", q, err.c_str());
-      }
+      std::string src = pst::rtc_source(pj.net, P, p->precision, pj.hazards);
       int g = 0;
-      while (g < (int)p->fixed.size() && p->fixed[g].k.fn != k.fn) ++g;
+      while (g < (int)p->fixed.size() && p->fixed[g].build[BUILD_PLAIN].source != src) ++g;
       if (g == (int)p->fixed.size()) {
         p->fixed.emplace_back();
-        p->fixed[g].k = k;
-        p->fixed[g].occ_source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, kOccupancyWaves);
-        p->fixed[g].pair_source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, true);
+        FixedBuild* b = p->fixed[g].build;
+        b[BUILD_PLAIN].source = std::move(src);
+        b[BUILD_OCC].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, kOccupancyWaves);
+        b[BUILD_PAIR].form = pst::RTC_PAIRED;
+        b[BUILD_PAIR].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_PAIRED);
+        b[BUILD_GROUP].form = pst::RTC_GROUP;
+        b[BUILD_GROUP].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_GROUP);
       }
       p->fixed[g].jobs.push_back(q);
       pj.fixed = g;
+    }
+  }
+  // compile what the default launch shape runs, so that a kinetic law the
+  // compiler refuses is refused here
+  for (FixedGroup& g : p->fixed) {
+    const int b = lanes_for(p->jobs, g.jobs, cu * 4) < 64 ? BUILD_GROUP : BUILD_PLAIN;
+    char what[32];
+    std::snprintf(what, sizeof(what), "job %d: ", g.jobs[0]);
+    const int rc2 = fixed_kernel(g.build[b], p->precision, what);
+    if (rc2 != PST_OK) {
+      pst_plan_destroy(p);
+      return rc2;
     }
   }
   if ((e = hipMalloc(&p->d_queue, sizeof(unsigned int) * n_jobs)) != hipSuccess ||
@@ -776,33 +805,27 @@ static int prepare_plan(pst_plan* p, int32_t* const* O_dev, const int64_t* o_str
     for (int q : g.jobs) p->jobs[q].p.lanes = L;
   }
   for (PlanJob& pj : p->jobs) pj.p.ssa_slice = p->ssa_slice;
-  // network kernels: the occupancy build for launches the plain build cannot
-  // hold resident at once
+  // The build of each network kernel: SSA bursts of tau-leaping jobs on paired
+  // wavefronts if the launch shape says so; a group of lanes per simulation if
+  // a wavefront has fewer than 64; else one simulation per lane, in the
+  // occupancy build if the plain build cannot hold the launch resident at once.
   for (FixedGroup& g : p->fixed) {
+    const pst::JobParams& P0 = p->jobs[g.jobs[0]].p;
+    int rc;
+    if (p->burst_waves && P0.method == PST_METHOD_TAU_LEAPING) {
+      g.use = BUILD_PAIR;
+      if ((rc = fixed_kernel(g.build[BUILD_PAIR], p->precision, "network kernel (paired build): ")) != PST_OK) return rc;
+      continue;
+    }
+    g.use = P0.lanes < 64 ? BUILD_GROUP : BUILD_PLAIN;
+    if ((rc = fixed_kernel(g.build[g.use], p->precision, "network kernel: ")) != PST_OK) return rc;
+    if (g.use == BUILD_GROUP) continue;
     int64_t need = 0;
     for (int q : g.jobs) need += ((int64_t)p->jobs[q].p.n_sims + p->jobs[q].p.lanes - 1) / p->jobs[q].p.lanes;
-    g.use_occ = false;
-    if (need <= (int64_t)g.k.blocks_per_cu * simds) continue;
-    if (!g.occ_tried) {
-      g.occ_tried = true;
-      std::string err;
-      const int rc = pst::rtc_kernel(g.occ_source, p->precision, &g.k_occ, &err);
-      if (rc != PST_OK) return fail(rc, "network kernel (occupancy build): %s", err.c_str());
-    }
-    g.use_occ = g.k_occ.fn != nullptr && g.k_occ.blocks_per_cu > g.k.blocks_per_cu;
-  }
-  // network kernels of tau-leaping jobs: SSA bursts on paired wavefronts
-  for (FixedGroup& g : p->fixed) {
-    g.use_pair = false;
-    if (!p->burst_waves || p->jobs[g.jobs[0]].p.method != PST_METHOD_TAU_LEAPING) continue;
-    if (!g.pair_tried) {
-      g.pair_tried = true;
-      std::string err;
-      const int rc = pst::rtc_kernel(g.pair_source, p->precision, &g.k_pair, &err, true);
-      if (rc != PST_OK) return fail(rc, "network kernel (paired build): %s", err.c_str());
-    }
-    if (!g.k_pair.fn) return fail(PST_EHIP, "network kernel (paired build) is not available");
-    g.use_pair = true;
+    const int plain = g.build[BUILD_PLAIN].k.blocks_per_cu;
+    if (need <= (int64_t)plain * simds) continue;
+    if ((rc = fixed_kernel(g.build[BUILD_OCC], p->precision, "network kernel (occupancy build): ")) != PST_OK) return rc;
+    if (g.build[BUILD_OCC].k.blocks_per_cu > plain) g.use = BUILD_OCC;
   }
   // job descriptors, one device array per size class
   for (int c = 0; c < pst::NUM_CLASSES; ++c) count[c] = 0;
@@ -1407,15 +1430,16 @@ int pst_run_noalloc(const pst_network* net, const pst_config* cfg, const double*
   else e = noalloc_enqueue<16, 16>(h, P, base, s);
   if (e != hipSuccess) return hip_fail(e, "descriptor kernel launch");
   const bool mixed = c.precision == PST_PRECISION_MIXED;
-  const int bpc = mixed ? pst::blocks_per_cu_mixed(cls) : pst::blocks_per_cu_fp64(cls);
+  const bool group = L < 64;
+  const int bpc = mixed ? pst::blocks_per_cu_mixed(cls, group) : pst::blocks_per_cu_fp64(cls, group);
   const int64_t need = ((int64_t)c.n_sims + L - 1) / L;
   const int64_t resident = (int64_t)bpc * simds;
   const int waves = (int)(need < resident ? need : resident);
   const void* jobs = base + kNoAllocJob;
   unsigned int* queue = (unsigned int*)(base + kNoAllocQueue);
   unsigned long long* counters = (unsigned long long*)base;
-  rc = mixed ? pst::launch_mixed(cls, jobs, 1, queue, counters, waves, pst::FULL_RUN, s)
-             : pst::launch_fp64(cls, jobs, 1, queue, counters, waves, pst::FULL_RUN, s);
+  const auto launch = mixed ? pst::launch_mixed : pst::launch_fp64;
+  rc = launch(cls, jobs, 1, queue, counters, waves, pst::FULL_RUN, group, s);
   if (rc != 0) return hip_fail((hipError_t)rc, "simulation kernel launch");
   if (stats) {
     unsigned long long hs[pst::ST_COUNT];

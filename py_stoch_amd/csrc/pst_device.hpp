@@ -89,7 +89,8 @@ __device__ __forceinline__ Words4 philox4x32_10(uint32_t c0, uint32_t c1, uint32
 
 // Per-lane work counters feeding the work model of the roofline figure.
 struct Work {
-  unsigned int uniforms;   // uniforms drawn
+  unsigned int uniforms;   // uniforms drawn, but for the Poisson draws
+  unsigned int draws;      // uniforms of the Poisson draws (by the lane that owns the reaction)
   unsigned int ptrs;       // PTRS rejection-loop iterations
   unsigned int inv;        // inversion search steps
   unsigned int decisions;  // tau-leap decisions (P1_P2 bodies with a0 > 0)
@@ -150,15 +151,7 @@ constexpr double SQRT2 = 1.4142135623730951;
 
 // ln x = e ln2 + 2 atanh(s), s = (m-1)/(m+1), m in [sqrt(2)/2, sqrt(2)),
 // odd series to z^10/21 with z = s^2.
-__device__ __forceinline__ double log_f64(double x) {
-  if (!(x > 0.0)) return (x == 0.0) ? -__builtin_inf() : __builtin_nan("");
-  if (x == __builtin_inf()) return x;
-  int e_adj = 0;
-  if (x < 0x1p-1022) {
-    x = x * 0x1p54;
-    e_adj = -54;
-  }
-  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+__device__ __forceinline__ double log_core_f64(uint64_t b, int e_adj) {
   int e = (int)((b >> 52) & 0x7ff) - 1023 + e_adj;
   double m = __builtin_bit_cast(double, (b & 0x000fffffffffffffull) | 0x3ff0000000000000ull);
   if (m > SQRT2) {
@@ -183,12 +176,21 @@ __device__ __forceinline__ double log_f64(double x) {
   const double de = (double)e;
   return de * LN2_HI + (lm + de * LN2_LO);
 }
+__device__ __forceinline__ double log_f64(double x) {
+  if (!(x > 0.0)) return (x == 0.0) ? -__builtin_inf() : __builtin_nan("");
+  if (x == __builtin_inf()) return x;
+  int e_adj = 0;
+  if (x < 0x1p-1022) {
+    x = x * 0x1p54;
+    e_adj = -54;
+  }
+  return log_core_f64(__builtin_bit_cast(uint64_t, x), e_adj);
+}
+// the same for a positive, finite, normal x (no special cases, no branches)
+__device__ __forceinline__ double log_normal_f64(double x) { return log_core_f64(__builtin_bit_cast(uint64_t, x), 0); }
 
 // exp x = 2^k exp(r), x = k ln2 + r (Cody-Waite), Taylor to r^13/13!.
-__device__ __forceinline__ double exp_f64(double x) {
-  if (x != x) return x;
-  if (x > 709.0) return __builtin_inf();
-  if (x < -708.0) return 0.0;
+__device__ __forceinline__ double exp_core_f64(double x) {  // -708 <= x <= 709
   const double k = floor(x * INV_LN2 + 0.5);
   const double r = (x - k * LN2_HI) - k * LN2_LO;
   double p = 1.0 / 6227020800.0;
@@ -207,6 +209,12 @@ __device__ __forceinline__ double exp_f64(double x) {
   p = p * r + 1.0;
   const int ki = (int)k;
   return p * __builtin_bit_cast(double, (uint64_t)(ki + 1023) << 52);
+}
+__device__ __forceinline__ double exp_f64(double x) {
+  if (x != x) return x;
+  if (x > 709.0) return __builtin_inf();
+  if (x < -708.0) return 0.0;
+  return exp_core_f64(x);
 }
 
 // ln(k!) for k = 0..9 (exact values rounded to double), Stirling's series above.

@@ -58,6 +58,42 @@ __device__ __forceinline__ int32_t pick_i(const int32_t (&x)[NP], int idx) {
   return r;
 }
 
+template <int NP>
+__device__ __forceinline__ float pick_f(const float (&x)[NP], int idx) {
+  int32_t r = 0;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) r |= __builtin_bit_cast(int32_t, x[i]) & -(int32_t)(idx == i);
+  return __builtin_bit_cast(float, r);
+}
+
+// Lane groups (GROUP builds): the 64 lanes of a wavefront hold 64 / G
+// simulations, each replicated over G adjacent lanes that run in lock-step on
+// the same registers; lane r of the group computes what can be split (the
+// random blocks of the next SSA steps, the Poisson draws of reactions r, r +
+// G, ...) and the results are exchanged.  GROUP = false: G = 1.
+template <bool GROUP>
+struct LaneGroup {
+  int G, r, base;  // size, position in the group, the group's first lane
+  __device__ __forceinline__ void set(int lane, int sims_per_wave) {
+    G = GROUP ? 64 / sims_per_wave : 1;
+    r = GROUP ? (lane & (G - 1)) : 0;
+    base = GROUP ? (lane & ~(G - 1)) : lane;
+  }
+  __device__ __forceinline__ bool lead() const { return !GROUP || r == 0; }
+  __device__ __forceinline__ bool mine(int j) const { return !GROUP || (j & (G - 1)) == r; }
+  // p in any lane of the group
+  __device__ __forceinline__ unsigned long long mask() const { return (G == 64 ? ~0ull : (1ull << G) - 1ull) << base; }
+  __device__ __forceinline__ bool any(bool p) const {
+    if constexpr (!GROUP) return p;
+    return (__builtin_amdgcn_ballot_w64(p) & mask()) != 0ull;
+  }
+  // reaction j's value, from the lane that owns it
+  __device__ __forceinline__ int32_t owners(int32_t v, int j) const {
+    if constexpr (!GROUP) return v;
+    return __builtin_amdgcn_ds_bpermute((base + (j & (G - 1))) * 4, v);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Trajectory output.  JobParams::layout selects
 //   LAYOUT_ROWS    O[q][f][o_stride], the reference's [kappa][ita][U]
@@ -209,7 +245,8 @@ struct StateIO {
 
 // Engine interface (see EngineF64 / EngineF32):
 //   int  start(job, sim)            -> initial mode, state loaded
-//   int  step<SSA_ONLY>(job, cnt, m) -> next mode (DONE may set flag)
+//   int  decide<GROUP>(job, cnt, on, group), int ssa_step(job, cnt) -> next
+//     mode (DONE may set flag)
 //   Draw1 ssa_draw(key, c), bool ssa_try(job, draw, tstop, sel, t1): one
 //     ordinary SSA step (ssa_run)
 //   int  flag
@@ -293,7 +330,7 @@ __device__ __forceinline__ double lane_get(double v, int addr) {
 // out of the ordinary happens in it.  A lane leaves the loop before a step
 // that ends the simulation or its range (absorbing state, last sample,
 // count limit, stuck clock, step budget, t_max): `general` is then set and
-// step<true> takes that step.  A lane whose step crosses a sample time stops
+// Engine::ssa_step takes that step.  A lane whose step crosses a sample time stops
 // for the rest of its batch and records the state before that step.
 // The batch's Philox blocks and logarithms do not depend on the state; they
 // are independent chains beside the steps'.  On gfx950 a dependent vector
@@ -301,9 +338,9 @@ __device__ __forceinline__ double lane_get(double v, int addr) {
 // general step, with about ten of them, takes 1,300 cycles for a single lane.
 // All lanes of the wavefront call this together.
 
-template <class Engine, class Ref>
+template <bool GROUP, class Engine, class Ref>
 __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int mode, bool on, int cap, double tstop,
-                                       bool& general) {
+                                       bool& general, const LaneGroup<GROUP>& g) {
   using Out = typename Engine::Out;
   constexpr int kBatch = 4;
   const auto& P = jr.p();
@@ -322,10 +359,22 @@ __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int 
   const Key uk = eng.key.scalar_seed(P.seed);  // a lane without a simulation may hold any key
   int n = 0;
   while (wave_any(go)) {
-    jr.refresh();
     typename Engine::Draw1 d[kBatch];
+    if constexpr (GROUP) {
+      // lane r of the group draws for step (n + r) % kBatch of the batch
+      const int q = g.G >= kBatch ? (g.r & (kBatch - 1)) : g.r;
+      typename Engine::Draw1 own = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + q));
+      typename Engine::Draw1 own2 = own;
+      if (g.G < kBatch) own2 = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + q + 2));
 #pragma unroll
-    for (int s = 0; s < kBatch; ++s) d[s] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + s));
+      for (int s = 0; s < kBatch; ++s) {
+        const int src = (g.base + (g.G >= kBatch ? s : (s & 1))) * 4;
+        d[s] = Engine::from_lane(g.G < kBatch && s >= 2 ? own2 : own, src);
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < kBatch; ++s) d[s] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + s));
+    }
     bool act = go, crossed = false;
     int csel = 0;
 #pragma unroll
@@ -339,25 +388,22 @@ __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int 
       const bool cross = done & (t1 >= eng.tnext);
       crossed = crossed | cross;
       csel = cross ? sel : csel;
+      int32_t dx[Engine::NP];
+      jr.row(sel, dx);
 #pragma unroll
-      for (int i = 0; i < Engine::NP; ++i) eng.x[i] += done ? jr.Vsel(i, sel) : 0;
+      for (int i = 0; i < Engine::NP; ++i) eng.x[i] += done ? dx[i] : 0;
       eng.t = done ? t1 : eng.t;
       n += done ? 1 : 0;
       act = done & !cross;
     }
     if (wave_any(crossed)) {
       if (crossed) {
+        int32_t before[Engine::NP];  // the state before the crossing step
+        jr.row(csel, before);
+#pragma unroll
+        for (int i = 0; i < Engine::NP; ++i) before[i] = eng.x[i] - before[i];
         do {
-#pragma unroll
-          for (int q = 0; q < Engine::NP; ++q) {
-            if (q < P.kappa) {
-              const int sp = jr.Ev(q);
-              int32_t v = 0;  // the state before the crossing step
-#pragma unroll
-              for (int i = 0; i < Engine::NP; ++i) v |= (eng.x[i] - jr.Vsel(i, csel)) & -(int32_t)(sp == i);
-              Out::put(P, eng.Ob, q, eng.F, v);
-            }
-          }
+          jr.for_recorded([&](int q) { Out::put(P, eng.Ob, q, eng.F, pick_i<Engine::NP>(before, jr.Ev(q))); });
           Out::row_done(P, eng.Ob, P.kappa, eng.F);
           cnt.w.samples += 1;
           eng.F = eng.F + 1;
@@ -381,35 +427,56 @@ __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int 
 }
 
 // Up to `cap` SSA steps of every lane in SSA mode: ordinary ones in ssa_run,
-// and the one it leaves over, if any, through step<true>.
-template <class Engine, class Ref>
+// and the one it leaves over, if any, through ssa_step.
+template <bool GROUP, class Engine, class Ref>
 __device__ __forceinline__ int ssa_slice(Ref& jr, Engine& eng, int64_t sim, Counters& cnt,
-                                         unsigned long long ev_start, int mode, int cap, int f_stop, double t_stop) {
-  if constexpr (Ref::kTable && Ref::kNP * Ref::kMP > 64) {
-    // the 16 x 16 table: its step is dominated by the walk over the table's
-    // entries and too large to be unrolled (ssa_run: 51 -> 59 ms on six networks)
-    for (int s = 0; s < cap && wave_any(mode == MODE_SSA); ++s) {
-      jr.refresh();
-      if (mode == MODE_SSA) {
-        mode = eng.template step<true>(jr, cnt, mode);
-        mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-      }
-    }
-    return mode;
-  }
+                                         unsigned long long ev_start, int mode, int cap, int f_stop, double t_stop,
+                                         const LaneGroup<GROUP>& g) {
   bool general;
-  mode = ssa_run(jr, eng, cnt, mode, mode == MODE_SSA, cap, t_stop, general);
+  mode = ssa_run<GROUP>(jr, eng, cnt, mode, mode == MODE_SSA, cap, t_stop, general, g);
   if (wave_any(general)) {
-    jr.refresh();
     if (general) {
-      mode = eng.template step<true>(jr, cnt, MODE_SSA);
+      mode = eng.ssa_step(jr, cnt);
       mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
     }
   }
   return mode;
 }
 
-template <class Engine, class Ref>
+// One leap decision of every lane in DECIDE mode.
+template <bool GROUP, class Engine, class Ref>
+__device__ __forceinline__ int decide_pass(Ref& jr, Engine& eng, int64_t sim, Counters& cnt,
+                                           unsigned long long ev_start, int mode, int f_stop,
+                                           const LaneGroup<GROUP>& g) {
+  const bool on = mode == MODE_DECIDE;
+  const int next = eng.template decide<GROUP>(jr, cnt, on, g);
+  mode = on ? next : mode;
+  if (wave_any(on & ((mode == MODE_DONE) | (eng.F >= f_stop)))) {
+    if (on) mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
+  }
+  return mode;
+}
+
+// Adds a wavefront's counters to the launch's.  Lanes of a group count the
+// same events: only the first lane's count, except for the Poisson draws,
+// which each lane counts for the reactions it drew.
+template <bool GROUP>
+__device__ __forceinline__ void add_stats(const Counters& cnt, const LaneGroup<GROUP>& g, int lane,
+                                          unsigned long long* __restrict__ stats) {
+  const unsigned long long m = g.lead() ? ~0ull : 0ull;
+  const unsigned long long vals[ST_EXACT + 1] = {cnt.events & m, cnt.leaps & m, cnt.rejected & m, cnt.ssa & m,
+                                                 cnt.flagged & m, (cnt.w.uniforms & m) + cnt.w.draws, cnt.w.ptrs,
+                                                 cnt.w.inv, cnt.w.decisions & m, cnt.w.samples & m, cnt.fevents & m,
+                                                 cnt.w.asym, cnt.w.exact};
+  // (32-bit per-lane counters: a lane's share of one launch stays far below 2^32)
+#pragma unroll
+  for (int i = 0; i <= ST_EXACT; ++i) {
+    const unsigned long long sum = wave_sum(vals[i]);
+    if (lane == 0) atomicAdd(&stats[i], sum);
+  }
+}
+
+template <class Engine, class Ref, bool GROUP>
 __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__ jobs, int n_jobs,
                                            unsigned int* __restrict__ queue, unsigned long long* __restrict__ stats,
                                            int f_end, int resume) {
@@ -426,11 +493,14 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
   jr.load(jobs);
   int f_stop = range_stop(jr, f_end);
   double t_stop = stop_time(jr, f_stop);
+  LaneGroup<GROUP> g;
+  g.set(lane, jr.p().lanes);
 
   for (;;) {
-    // ---- refill lanes whose simulation ended from the job's queue ----
-    const bool want = (mode == MODE_DONE) && !exhausted && lane < jr.p().lanes;
-    const unsigned long long wmask = __builtin_amdgcn_ballot_w64(want);
+    // ---- refill lanes whose simulation ended from the job's queue (the lanes
+    // of a group are in lock-step: they end together and take one simulation) ----
+    const bool want = (mode == MODE_DONE) && !exhausted && (GROUP || lane < jr.p().lanes);
+    const unsigned long long wmask = __builtin_amdgcn_ballot_w64(want & g.lead());
     if (wmask != 0ull) {
       const int n = __builtin_popcountll(wmask);
       const int leader = __builtin_ctzll(wmask);
@@ -440,7 +510,7 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
       const int n_sims = jr.p().n_sims;
       if ((int64_t)base + n >= (int64_t)n_sims) exhausted = true;
       if (want) {
-        const int rank = __builtin_popcountll(wmask & ((1ull << lane) - 1ull));
+        const int rank = __builtin_popcountll(wmask & ((1ull << g.base) - 1ull));
         const int64_t s = (int64_t)base + rank;
         if (s < n_sims) {
           sim = s;
@@ -455,37 +525,27 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
       jr.load(jobs + job);
       f_stop = range_stop(jr, f_end);
       t_stop = stop_time(jr, f_stop);
+      g.set(lane, jr.p().lanes);
       exhausted = false;
       continue;
     }
 
-    jr.refresh();
-    if (wave_any(mode == MODE_DECIDE)) {
-      if (mode != MODE_DONE) {
-        mode = eng.template step<false>(jr, cnt, mode);
-        mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-      }
+    // (only tau-leaping decides: a compile-time fact in network kernels)
+    if (jr.method() == 0 && wave_any(mode == MODE_DECIDE)) {
+      mode = decide_pass<GROUP>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
       // SSA-only steps while lanes are inside a burst
       if (wave_any(mode == MODE_SSA))
-        mode = ssa_slice(jr, eng, sim, cnt, ev_start, mode, jr.p().ssa_slice + 1, f_stop, t_stop);
+        mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, jr.p().ssa_slice + 1, f_stop, t_stop, g);
     } else {
       // no lane decides (pure SSA, or every live lane inside a burst): up to
       // 1 + ssa_slice SSA steps before the next refill, 2 + 2 ssa_slice for
       // pure SSA, where no lane waits to decide
       const int cap = jr.p().method == 2 ? 2 * jr.p().ssa_slice + 2 : jr.p().ssa_slice + 1;
-      mode = ssa_slice(jr, eng, sim, cnt, ev_start, mode, cap, f_stop, t_stop);
+      mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, cap, f_stop, t_stop, g);
     }
   }
 
-  const unsigned long long vals[ST_EXACT + 1] = {cnt.events, cnt.leaps, cnt.rejected, cnt.ssa, cnt.flagged,
-                                                 cnt.w.uniforms, cnt.w.ptrs, cnt.w.inv, cnt.w.decisions,
-                                                 cnt.w.samples, cnt.fevents, cnt.w.asym, cnt.w.exact};
-  // (32-bit per-lane counters: a lane's share of one launch stays far below 2^32)
-#pragma unroll
-  for (int i = 0; i <= ST_EXACT; ++i) {
-    const unsigned long long sum = wave_sum(vals[i]);
-    if (lane == 0) atomicAdd(&stats[i], sum);
-  }
+  add_stats(cnt, g, lane, stats);
 }
 
 // ---------------------------------------------------------------------------
@@ -581,6 +641,8 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
   int64_t sim = -1;
   unsigned long long ev_start = 0;  // cnt.events when this lane's simulation began (here)
   Ref jr;
+  LaneGroup<false> g;
+  g.set(lane, 64);
 
   if (wave < 4) {
     // ---- decide wavefront ----
@@ -626,11 +688,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         continue;
       }
       if (wave_any(mode == MODE_DECIDE)) {
-        jr.refresh();
-        if (mode == MODE_DECIDE) {
-          mode = eng.template step<false>(jr, cnt, mode);
-          mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-        }
+            mode = decide_pass<false>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
       } else if (!wave_any(mode == MODE_SSA)) {
         __builtin_amdgcn_s_sleep(2);  // every live lane is away: wait for a burst to come back
       }
@@ -676,10 +734,9 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         continue;
       }
       bool general;
-      int m = ssa_run(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, general);
+      int m = ssa_run<false>(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, general, g);
       if (wave_any(general)) {
-        jr.refresh();
-        if (general) m = eng.template step<true>(jr, cnt, MODE_SSA);
+            if (general) m = eng.ssa_step(jr, cnt);
       }
       if (busy) {
         if (m == MODE_DONE) m = settle(jr, eng, sim, cnt, ev_start, m, f_stop);
@@ -694,14 +751,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     }
   }
 
-  const unsigned long long vals[ST_EXACT + 1] = {cnt.events, cnt.leaps, cnt.rejected, cnt.ssa, cnt.flagged,
-                                                 cnt.w.uniforms, cnt.w.ptrs, cnt.w.inv, cnt.w.decisions,
-                                                 cnt.w.samples, cnt.fevents, cnt.w.asym, cnt.w.exact};
-#pragma unroll
-  for (int i = 0; i <= ST_EXACT; ++i) {
-    const unsigned long long sum = wave_sum(vals[i]);
-    if (lane == 0) atomicAdd(&stats[i], sum);
-  }
+  add_stats(cnt, g, lane, stats);
 }
 
 }  // namespace pst

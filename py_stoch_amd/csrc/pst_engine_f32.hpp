@@ -19,26 +19,6 @@
 
 namespace pst {
 
-template <class Ref, int NP = Ref::kNP, int MP = Ref::kMP>
-__device__ __forceinline__ void propensities_f32(const Ref& tab, const float (&k)[Ref::kKP],
-                                                 const int32_t (&x)[NP], float (&a)[MP]) {
-  if constexpr (Ref::kCustom) {
-    Ref::template props<float>(x, k, a);  // compiled hazard expressions
-  } else {
-#pragma unroll
-    for (int j = 0; j < MP; ++j) {
-      float v = k[j];
-#pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        const int p = tab.Ord(i, j);
-        const int st = tab.Stp(i, j);
-        for (int q = 0; q < p; ++q) v = v * (float)(x[i] - st * q);
-      }
-      a[j] = v;
-    }
-  }
-}
-
 // CalculateG (P1_P2.py:447-486) in FP32
 __device__ __forceinline__ float calc_g_f32(int h, int ht, int xi) {
   const float xf = (float)xi;
@@ -168,6 +148,13 @@ __device__ __noinline__ Draw ptrs_wide(uint32_t k0, uint32_t k1, uint32_t s_lo, 
 template <class Ref>
 struct EngineF32 {
   static constexpr int NP = Ref::kNP, MP = Ref::kMP;
+  static constexpr int NB = (MP + 3) / 4;  // Philox blocks of a leap attempt
+  // The larger tables take their draws one after the other through one copy
+  // of the sampler: one copy per reaction came to 320 KB of code for 16 x 16.
+  static constexpr bool kWorklist = Ref::kTable && MP > 4;
+  // blocks generated beside the decision (the one-by-one draws generate theirs)
+  template <bool GROUP>
+  static constexpr int ahead() { return (GROUP || kWorklist) && NB > 1 ? 1 : NB; }
   float k[Ref::kKP];  // rates row: per-reaction constants, or hazard parameters
   int32_t x[NP];
   Key key;
@@ -181,23 +168,25 @@ struct EngineF32 {
 
   using Out = SampleOut<Ref::kOutLds>;
 
+  // v[i]: i is a constant in network kernels, wavefront-uniform in table-driven ones
+  template <class T>
+  static __device__ __forceinline__ T species_of(const T (&v)[NP], int i) {
+    if constexpr (Ref::kTable) return at<T, NP>(v, i);
+    else return v[i];
+  }
+
   __device__ __forceinline__ void fill_rest(const Ref& tab, bool zero, Counters& cnt) const {
     const auto& P = tab.p();
     cnt.w.samples += (unsigned int)(P.ita - F);
     if (P.layout != LAYOUT_BLOCKS) {
-#pragma unroll
-      for (int q = 0; q < NP; ++q) {
-        if (q < P.kappa) {
-          const int32_t val = zero ? 0 : pick_i<NP>(x, tab.Ev(q));
-          for (int f = F; f < P.ita; ++f) glb(Ob)[((int64_t)q * P.ita + f) * P.o_stride] = val;
-        }
-      }
+      tab.for_recorded([&](int q) {
+        const int32_t val = zero ? 0 : pick_i<NP>(x, tab.Ev(q));
+        for (int f = F; f < P.ita; ++f) glb(Ob)[((int64_t)q * P.ita + f) * P.o_stride] = val;
+      });
       return;
     }
     for (int f = F; f < P.ita; ++f) {
-#pragma unroll
-      for (int q = 0; q < NP; ++q)
-        if (q < P.kappa) Out::put(P, Ob, q, f, zero ? 0 : pick_i<NP>(x, tab.Ev(q)));
+      tab.for_recorded([&](int q) { Out::put(P, Ob, q, f, zero ? 0 : pick_i<NP>(x, tab.Ev(q))); });
       Out::row_done(P, Ob, P.kappa, f);
     }
   }
@@ -221,16 +210,12 @@ struct EngineF32 {
     return P.method == 0 ? MODE_DECIDE : MODE_SSA;
   }
 
-  // One step: leap decision and leap (P1_P2.py:96-294), or one SSA step
-  // (P3.py:73-149, gillespie.py:70-149) -- see EngineF64::step for the
-  // structure; the arithmetic is FP32 except the clock and the cumulative
-  // sum of the reaction choice.
-  template <bool SSA_ONLY>
-  __device__ __forceinline__ int step(const Ref& tab, Counters& cnt, int mode) {
+  // One direct-method SSA step in its general form -- see EngineF64::ssa_step;
+  // the arithmetic is FP32 except the clock and the cumulative sum of the
+  // reaction choice.
+  __device__ __forceinline__ int ssa_step(const Ref& tab, Counters& cnt) {
     const auto& P = tab.p();
-    const int M = P.M;
-    bool ssa = SSA_ONLY || (mode == MODE_SSA);
-    if (ssa && P.method == 2 && !(t < P.t_max)) {
+    if (P.method == 2 && !(t < P.t_max)) {
       fill_rest(tab, true, cnt);
       return MODE_DONE;
     }
@@ -241,24 +226,8 @@ struct EngineF32 {
       return MODE_DONE;
     }
     nsteps += 1;
-    // Philox blocks bc .. bc + NB - 1, generated together as independent
-    // chains: block bc serves the one-block draw (SSA step, or tau2 and the
-    // critical reaction) and the first Poisson attempt takes NB consecutive
-    // blocks after it, or from bc when there is no one-block draw; block
-    // bc + NB is generated at the leap, only if a lane of the wavefront made
-    // a one-block draw.
-    constexpr int NB = (MP + 3) / 4;
-    const uint64_t bc0 = bc;
-    Words4 B[NB + 1];
-    B[0] = key.block(bc, 0);
-    B[NB] = Words4{0u, 0u, 0u, 0u};
-    if (!SSA_ONLY) {
-#pragma unroll
-      for (int r = 1; r < NB; ++r)
-        if (4 * (r - 1) < M) B[r] = key.block(bc + (uint64_t)r, 0);
-    }
     float a[MP];
-    propensities_f32<Ref>(tab, k, x, a);
+    tab.template props<float>(x, k, a);
     float a0 = 0.0f;
 #pragma unroll
     for (int j = 0; j < MP; ++j) a0 += a[j];
@@ -266,142 +235,19 @@ struct EngineF32 {
       fill_rest(tab, false, cnt);
       return MODE_DONE;
     }
-    bool crit[MP];
-#pragma unroll
-    for (int j = 0; j < MP; ++j) crit[j] = false;
-    float tau1 = __builtin_inff();
-    if (!SSA_ONLY && !ssa) {
-      cnt.w.decisions += 1;
-      // critical reactions (P1_P2.py:314-327)
-#pragma unroll
-      for (int j = 0; j < MP; ++j) {
-        bool c = false;
-#pragma unroll
-        for (int i = 0; i < NP; ++i) {
-          const int v = tab.V(i, j);
-          if (v < 0) c = c | ((-v) * P.n_c > x[i]);
-        }
-        crit[j] = c;
-      }
-      const float eta = (float)P.eta;
-#pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        if (tab.Irs(i)) {
-          float mu = 0.0f, s2 = 0.0f;
-          bool any = false;
-#pragma unroll
-          for (int j = 0; j < MP; ++j) {
-            const int v = tab.V(i, j);
-            if (v != 0) {
-              const bool nc = !crit[j];
-              mu += nc ? (float)v * a[j] : 0.0f;
-              s2 += nc ? (float)(v * v) * a[j] : 0.0f;
-              any = any | nc;
-            }
-          }
-          const float g_i = calc_g_f32(tab.Hv(i), tab.Htv(i), x[i]);
-          const float num = fmaxf(eta * (float)x[i] * fast_rcp(g_i), 1.0f);
-          const float cand = fminf(num * fast_rcp(fabsf(mu)), num * num * fast_rcp(s2));
-          tau1 = any ? fminf(tau1, cand) : tau1;
-        }
-      }
-      if (tau1 < 10.0f * fast_rcp(a0)) {
-        ssa = true;
-        burst = P.ssa_burst;
-        if (P.max_steps != 0u && nsteps >= P.max_steps) {
-          fill_rest(tab, true, cnt);
-          flag = FLAG_STEPS;
-          return MODE_DONE;
-        }
-        nsteps += 1;
-      }
-    }
-    bool msk[MP];
     double asum = 0.0;
 #pragma unroll
-    for (int j = 0; j < MP; ++j) {
-      msk[j] = ssa ? (j < M) : crit[j];
-      asum += msk[j] ? (double)a[j] : 0.0;
-    }
-    float tauX = __builtin_inff();
+    for (int j = 0; j < MP; ++j) asum += (double)a[j];
+    float tau = __builtin_inff();
     uint32_t cw1 = 0;
-    const bool one = asum > 0.0;
-    if (one) {
-      const Words4 bw = B[0];
+    if (asum > 0.0) {
+      const Words4 bw = key.block(bc, 0);
       bc += 1;
-      cnt.w.uniforms += ssa ? 2 : 1;
+      cnt.w.uniforms += 2;
       cw1 = bw.w1;
-      tauX = -fast_log(u24(bw.w0)) * fast_rcp((float)asum);
+      tau = -fast_log(u24(bw.w0)) * fast_rcp((float)asum);
     }
-    const float tau_f = ssa ? tauX : fminf(tau1, tauX);
-    int sel = -1;
-    if (ssa || tau1 > tauX) {
-      if (!ssa) cnt.w.uniforms += 1;
-      // first j of the mask with sum_{r<=j} a_r >= rho2 * asum, summed in FP64
-      const double target = (double)u24(cw1) * asum;
-      double cum = 0.0;
-      int last = -1;
-      if constexpr (SSA_ONLY) {
-        // The running sum never decreases and rho2 * asum > 0, so that j is
-        // the number of positions whose sum is still below the target (a
-        // masked-out position repeats its predecessor's sum and is never the
-        // first to reach it): no branches in the SSA-only steps (Schlogl pure
-        // SSA 68 -> 59 ms; the leap step keeps the loop, which measured faster
-        // there).  The last positive masked reaction covers a sum that ends
-        // below the target.
-        int below = 0;
-#pragma unroll
-        for (int j = 0; j < MP; ++j) {
-          cum += msk[j] ? (double)a[j] : 0.0;
-          last = (msk[j] && a[j] > 0.0f) ? j : last;
-          below += (cum < target) ? 1 : 0;
-        }
-        sel = below < MP ? below : last;
-      } else {
-#pragma unroll
-        for (int j = 0; j < MP; ++j) {
-          if (msk[j] && sel < 0) {
-            if (a[j] > 0.0f) last = j;
-            cum += (double)a[j];
-            if (cum >= target) sel = j;
-          }
-        }
-        if (sel < 0) sel = last;
-      }
-    }
-    int32_t xn[NP];
-    float tau = tau_f;
-    if (ssa) {
-#pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        int dx = 0;
-#pragma unroll
-        for (int j = 0; j < MP; ++j)
-          if (sel == j) dx = tab.V(i, j);
-        xn[i] = x[i] + dx;
-      }
-    } else if (!SSA_ONLY) {
-      if (!(tau < __builtin_inff())) {
-        fill_rest(tab, true, cnt);
-        flag = FLAG_TAU_INF;
-        return MODE_DONE;
-      }
-      int32_t K[MP];
-#pragma unroll
-      for (int j = 0; j < MP; ++j) K[j] = (sel == j) ? 1 : 0;
-      if (wave_any(one)) B[NB] = key.block(bc0 + (uint64_t)NB, 0);
-      const int st = leap(tab, cnt, a, crit, tau, K, xn, B, one);
-      if (st != 0) {
-        fill_rest(tab, true, cnt);
-        flag = st;
-        return MODE_DONE;
-      }
-      unsigned long long ev = 0;
-#pragma unroll
-      for (int j = 0; j < MP; ++j) ev += (unsigned long long)K[j];
-      cnt.events += ev;
-      cnt.leaps += 1;
-    }
+    const int sel = pick_reaction(a, asum, u24(cw1), [](int) { return true; });
     const double t0 = t;
     t = t + (double)tau;
     if (t == t0 && tau > 0.0f) {  // tau == 0 (a draw of u = 1) is a valid event
@@ -409,47 +255,191 @@ struct EngineF32 {
       flag = FLAG_STALL;
       return MODE_DONE;
     }
-    if (t >= tnext) {
-      const float inv_gap = fast_rcp((float)(t - t0));
-      while (t >= tnext) {
-        // sample-and-hold for an SSA step: a zero fraction keeps the pre-step state
-        const float frac = ssa ? 0.0f : (float)(tnext - t0) * inv_gap;
+    // sample-and-hold of the pre-step state
+    while (t >= tnext) {
+      tab.for_recorded([&](int q) { Out::put(P, Ob, q, F, pick_i<NP>(x, tab.Ev(q))); });
+      Out::row_done(P, Ob, P.kappa, F);
+      cnt.w.samples += 1;
+      F = F + 1;
+      if (F == P.ita) return MODE_DONE;
+      tnext = (double)glb(P.I)[F];
+    }
+    bool over = false;
+    int32_t d[NP];
+    tab.row(sel >= 0 ? sel : 0, d);
 #pragma unroll
-        for (int q = 0; q < NP; ++q) {
-          if (q < P.kappa) {
+    for (int i = 0; i < NP; ++i) {
+      x[i] += sel >= 0 ? d[i] : 0;
+      over = over | (x[i] >= COUNT_LIMIT);
+    }
+    cnt.ssa += 1;
+    cnt.events += 1;
+    if (over) {
+      fill_rest(tab, true, cnt);
+      flag = FLAG_OVERFLOW;
+      return MODE_DONE;
+    }
+    if (P.method != 0) return MODE_SSA;
+    burst -= 1;
+    return burst > 0 ? MODE_SSA : MODE_DECIDE;
+  }
+
+  // First j of the mask with sum_{r<=j} a_r >= rho * asum, summed in FP64; the
+  // running sum never decreases and the target is positive, so that is the
+  // number of positions whose sum is still below it (a masked-out position
+  // repeats its predecessor's sum and is never the first to reach it).  A sum
+  // that ends below the target takes the last positive masked reaction.
+  template <class Mask>
+  static __device__ __forceinline__ int pick_reaction(const float (&a)[MP], double asum, float rho, Mask in) {
+    const double target = (double)rho * asum;
+    double cum = 0.0;
+    int below = 0, last = -1;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) {
+      cum += in(j) ? (double)a[j] : 0.0;
+      last = (in(j) & (a[j] > 0.0f)) ? j : last;
+      below += (cum < target) ? 1 : 0;
+    }
+    return below < MP ? below : last;
+  }
+
+  // One P1_P2 body (P1_P2.py:96-294) of the lanes with `on` -- see
+  // EngineF64::decide.
+  template <bool GROUP>
+  __device__ __forceinline__ int decide(Ref& tab, Counters& cnt, bool on, const LaneGroup<GROUP>& g) {
+    const auto& P = tab.p();
+    constexpr int ABSORBED = -1;
+    int end = 0;  // ABSORBED, or the flag that ends the simulation
+    bool live = on;
+    if (P.max_steps != 0u) {
+      end = (live & (nsteps >= P.max_steps)) ? FLAG_STEPS : 0;
+      live = live & (end == 0);
+    }
+    nsteps += live ? 1u : 0u;
+    // Philox blocks bc .. bc + NB - 1, independent of the state: chains beside
+    // the decision's.  The first Poisson attempt takes the NB blocks from bc,
+    // or those from bc + 1 when the critical draw took block bc.
+    const Key uk = key.scalar_seed(P.seed);
+    constexpr int NA = ahead<GROUP>();
+    Words4 B[NB];
+#pragma unroll
+    for (int r = 0; r < NA; ++r) B[r] = uk.block(bc + (uint64_t)r, 0);
+    float a[MP];
+    tab.template props<float>(x, k, a);
+    float a0 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) a0 += a[j];
+    // (products already rounded to FP32: not to be contracted into the sums below)
+#pragma unroll
+    for (int j = 0; j < MP; ++j) asm("" : "+v"(a[j]));
+    end = (live & (a0 == 0.0f)) ? ABSORBED : end;
+    live = live & !(a0 == 0.0f);
+    cnt.w.decisions += live ? 1u : 0u;
+    // critical reactions, mu and sigma^2, and the Cao bound (P1_P2.py:314-445)
+    unsigned crit, any;
+    float mu[NP], s2[NP];
+    tab.template sums<float>(x, a, P.n_c, crit, mu, s2, any);
+    float tau1 = __builtin_inff();
+    const float eta = (float)P.eta;
+    tab.for_species([&](int i) {
+      if (tab.Irs(i)) {
+        const int32_t xi = species_of<int32_t>(x, i);
+        const float g_i = calc_g_f32(tab.Hv(i), tab.Htv(i), xi);
+        const float num = fmaxf(eta * (float)xi * fast_rcp(g_i), 1.0f);
+        const float cand = fminf(num * fast_rcp(fabsf(species_of<float>(mu, i))),
+                                 num * num * fast_rcp(species_of<float>(s2, i)));
+        tau1 = ((any >> i) & 1u) ? fminf(tau1, cand) : tau1;
+      }
+    });
+    // SSA switch (P1_P2.py:157-173)
+    const bool fall = live & (tau1 < 10.0f * fast_rcp(a0));
+    burst = fall ? P.ssa_burst : burst;
+    live = live & !fall;
+    // tau2 and the critical reaction (P1_P2.py:175-220)
+    double asum = 0.0;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) asum += ((crit >> j) & 1u) ? (double)a[j] : 0.0;
+    float tau = tau1;
+    int sel = -1;
+    const bool one = live & (asum > 0.0);
+    if (wave_any(one)) {
+      const float tauX = -fast_log(u24(B[0].w0)) * fast_rcp((float)asum);
+      const bool fire = one & (tau1 > tauX);
+      cnt.w.uniforms += (one ? 1u : 0u) + (fire ? 1u : 0u);
+      tau = one ? fminf(tau1, tauX) : tau;
+      const int c = pick_reaction(a, asum, u24(B[0].w1), [&](int j) { return ((crit >> j) & 1u) != 0u; });
+      sel = fire ? c : -1;
+      const Words4 e = NA == NB ? uk.block(bc + (uint64_t)NB, 0) : B[0];
+#pragma unroll
+      for (int r = 0; r < NA; ++r) {
+        const Words4 n = r + 1 < NA ? B[r + 1 < NA ? r + 1 : 0] : e;
+        B[r].w0 = one ? n.w0 : B[r].w0;
+        B[r].w1 = one ? n.w1 : B[r].w1;
+        B[r].w2 = one ? n.w2 : B[r].w2;
+        B[r].w3 = one ? n.w3 : B[r].w3;
+      }
+      bc += one ? 1u : 0u;
+    }
+    end = (live & !(tau < __builtin_inff())) ? FLAG_TAU_INF : end;
+    live = live & (tau < __builtin_inff());
+    // the leap, with tau halving (P1_P2.py:222-259)
+    int32_t xn[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) xn[i] = 0;
+    unsigned long long ev = 0;
+    bool again = live;
+    for (int h = 0;; ++h) {
+      const int st = attempt<GROUP>(tab, cnt, again, a, crit, tau, sel, B, xn, ev, uk, g);
+      end = (again & (st > 0)) ? st : end;
+      again = again & (st < 0);
+      if (!wave_any(again)) break;
+      cnt.rejected += again ? 1u : 0u;
+      tau = again ? tau * 0.5f : tau;
+      end = (again & (h + 1 >= MAX_HALVINGS)) ? FLAG_HALVING : end;
+      again = again & (h + 1 < MAX_HALVINGS);
+#pragma unroll
+      for (int r = 0; r < NA; ++r) B[r] = uk.block(bc + (uint64_t)r, 0);
+    }
+    live = live & (end == 0);
+    cnt.events += live ? ev : 0ull;
+    cnt.leaps += live ? 1u : 0u;
+    // time advance and interpolated samples
+    const double t0 = t;
+    const double t1 = t + (double)tau;
+    t = live ? t1 : t;
+    const bool stall = live & (t1 == t0) & (tau > 0.0f);  // tau == 0 is a valid event
+    end = stall ? FLAG_STALL : end;
+    live = live & !stall;
+    bool last = false;
+    if (wave_any(live & (t >= tnext))) {
+      if (live) {
+        const float inv_gap = fast_rcp((float)(t - t0));
+        while (t >= tnext) {
+          const float frac = (float)(tnext - t0) * inv_gap;
+          tab.for_recorded([&](int q) {
             const int s = tab.Ev(q);
             const int32_t xs = pick_i<NP>(x, s);
             const int diff = pick_i<NP>(xn, s) - xs;
             Out::put(P, Ob, q, F, xs + rn_f32_to_int((float)diff * frac));
-          }
+          });
+          Out::row_done(P, Ob, P.kappa, F);
+          cnt.w.samples += 1;
+          F = F + 1;
+          last = F == P.ita;
+          if (last) break;
+          tnext = (double)glb(P.I)[F];
         }
-        Out::row_done(P, Ob, P.kappa, F);
-        cnt.w.samples += 1;
-        F = F + 1;
-        if (F == P.ita) return MODE_DONE;
-        tnext = (double)glb(P.I)[F];
       }
     }
-    if (ssa) {
-      bool over = false;
-#pragma unroll
-      for (int i = 0; i < NP; ++i) over = over | (xn[i] >= COUNT_LIMIT);
-      cnt.ssa += 1;
-      cnt.events += 1;
-#pragma unroll
-      for (int i = 0; i < NP; ++i) x[i] = xn[i];
-      if (over) {
-        fill_rest(tab, true, cnt);
-        flag = FLAG_OVERFLOW;
-        return MODE_DONE;
+    if (wave_any(end != 0)) {
+      if (end != 0) {
+        fill_rest(tab, end != ABSORBED, cnt);
+        flag = end != ABSORBED ? end : 0;
       }
-      if (P.method != 0) return MODE_SSA;
-      burst -= 1;
-      return burst > 0 ? MODE_SSA : MODE_DECIDE;
     }
 #pragma unroll
-    for (int i = 0; i < NP; ++i) x[i] = xn[i];
-    return MODE_DECIDE;
+    for (int i = 0; i < NP; ++i) x[i] = live ? xn[i] : x[i];
+    return ((end != 0) | last) ? MODE_DONE : fall ? MODE_SSA : MODE_DECIDE;
   }
 
   // The random numbers of one SSA step: -ln(rho1) and rho2.
@@ -467,7 +457,7 @@ struct EngineF32 {
   // arithmetic; a0 = 0 gives an infinite or undefined time, which fails.
   __device__ __forceinline__ bool ssa_try(const Ref& tab, const Draw1& d, double tstop, int& sel, double& t1) const {
     float a[MP];
-    propensities_f32<Ref>(tab, k, x, a);
+    tab.template props<float>(x, k, a);
     double cum[MP];
 #pragma unroll
     for (int j = 0; j < MP; ++j) cum[j] = (j > 0 ? cum[j > 0 ? j - 1 : 0] : 0.0) + (double)a[j];
@@ -480,150 +470,220 @@ struct EngineF32 {
     return (t1 > t) & (t1 < tstop);
   }
 
-  // Poisson leap with tau halving (P1_P2.py:222-259,509-540).  Every draw is
-  // an inversion of the Poisson CDF at one 24-bit uniform: reaction j reads
-  // word j % 4 of block grp + j / 4 (so one block serves four reactions);
-  // lambda < 10 by sequential search, 10 <= lambda < 2^16 by the asymptotic
-  // inversion with exact FP64 decisions near integer boundaries (both are
-  // inversions, so no draw is rejected and repeated); lambda >= 2^16 by
-  // PTRS on blocks of its own (ptrs_wide).  tau is halved in place: the clock
-  // advances by the tau of the accepted draw (P1_P2.py:258-261).  Returns 0
-  // or a flag.
-  __device__ __forceinline__ int leap(const Ref& tab, Counters& cnt,
-                                      const float (&a)[MP], const bool (&crit)[MP], float& tau,
-                                      int32_t (&K)[MP], int32_t (&xn)[NP], const Words4 (&B)[(MP + 3) / 4 + 1],
-                                      bool shifted) {
-    constexpr int NB = (MP + 3) / 4;
+  // One attempt of the leap for the lanes with `on` -- see EngineF64::attempt
+  // for what it returns.  Every draw is an inversion of the Poisson CDF at one
+  // 24-bit uniform: reaction j reads word j % 4 of block W[j / 4]; lambda < 10
+  // by sequential search, 10 <= lambda < 2^16 by the asymptotic inversion with
+  // exact FP64 decisions near integer boundaries (both are inversions, so no
+  // draw is rejected and repeated); lambda >= 2^16 by PTRS on blocks of its own
+  // (ptrs_wide).
+  template <bool GROUP>
+  __device__ __forceinline__ int attempt(Ref& tab, Counters& cnt, bool on, const float (&a)[MP],
+                                         unsigned crit, float tau, int sel, const Words4 (&W)[NB],
+                                         int32_t (&xn)[NP], unsigned long long& ev, const Key& uk,
+                                         const LaneGroup<GROUP>& g) {
     const auto& P = tab.p();
     const int M = P.M;
-    const int nblk = (M + 3) >> 2;
-    for (int h = 0; h < MAX_HALVINGS; ++h) {
-      const uint64_t grp = bc;
-      bc += (uint64_t)nblk;
-      // first attempt: the blocks generated with the step's; retries: new ones
-      Words4 W[NB];
+    const uint64_t grp = bc;
+    bc += on ? (uint64_t)((M + 3) >> 2) : 0ull;
+    float lam[MP];
+    int32_t K[MP];
+    bool bad = false, fail = false;
 #pragma unroll
-      for (int r = 0; r < NB; ++r) {
-        if (4 * r < M) {
-          if (h == 0) {
-            W[r].w0 = shifted ? B[r + 1].w0 : B[r].w0;
-            W[r].w1 = shifted ? B[r + 1].w1 : B[r].w1;
-            W[r].w2 = shifted ? B[r + 1].w2 : B[r].w2;
-            W[r].w3 = shifted ? B[r + 1].w3 : B[r].w3;
-          } else {
-            W[r] = key.block(grp + (uint64_t)r, 0);
-          }
-        }
+    for (int j = 0; j < MP; ++j) {
+      lam[j] = (on & (j < M) & !((crit >> j) & 1u)) ? a[j] * tau : 0.0f;
+      K[j] = (sel == j) ? 1 : 0;
+      bad = bad | (lam[j] >= (float)LAMBDA_LIMIT);
+    }
+    if constexpr (GROUP || kWorklist) {
+      // the lane's own reactions, one after the other
+      unsigned todo = 0;
+#pragma unroll
+      for (int j = 0; j < MP; ++j) todo |= (g.mine(j) & (lam[j] > 0.0f)) ? (1u << j) : 0u;
+      todo = bad ? 0u : todo;
+      while (wave_any(todo != 0u)) {
+        const bool has = todo != 0u;
+        const int j = has ? __builtin_ctz(todo) : 0;
+        const float l = pick_f<MP>(lam, j);
+        const uint64_t c = grp + (uint64_t)(uint32_t)(j >> 2);
+        Words4 w;
+        if constexpr (NB == 1) w = W[0];
+        else w = uk.block(c, 0);
+        const int32_t kk = draw(cnt, has, l, u24(word_of(w, j)), c, j & 3, fail);
+#pragma unroll
+        for (int r = 0; r < MP; ++r) K[r] = (has & (r == j)) ? kk : K[r];
+        todo = todo & (todo - 1u);
       }
-      float lam[MP], u[MP];
-      unsigned inv = 0, exact = 0, wide = 0, nasym = 0;
-      int32_t mb[MP];
-      bool bad = false;
+#pragma unroll
+      for (int j = 0; j < MP; ++j) K[j] = g.owners(K[j], j);
+      fail = g.any(fail);
+    } else {
+      float u[MP];
+#pragma unroll
+      for (int j = 0; j < MP; ++j) u[j] = u24(word_of(W[j >> 2], j));
+      draw_all(cnt, bad, lam, u, grp, K, fail);
+    }
+    bool ok = true, big = false;
+    int64_t s[NP];
+    tab.advance(x, K, s);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      ok = ok & (s[i] >= 0);
+      big = big | (s[i] >= COUNT_LIMIT);
+      xn[i] = on ? (int32_t)s[i] : xn[i];
+    }
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) sum += (unsigned long long)K[j];
+    ev = on ? sum : ev;
+    return bad ? FLAG_OVERFLOW : fail ? FLAG_PTRS : !ok ? -1 : big ? FLAG_OVERFLOW : 0;
+  }
+
+  // word j % 4 of a block
+  static __device__ __forceinline__ uint32_t word_of(const Words4& w, int j) {
+    const uint32_t odd = 0u - (uint32_t)(j & 1), up = 0u - (uint32_t)((j >> 1) & 1);
+    const uint32_t lo = w.w0 ^ ((w.w0 ^ w.w1) & odd), hi = w.w2 ^ ((w.w2 ^ w.w3) & odd);
+    return lo ^ ((lo ^ hi) & up);
+  }
+
+  // One Poisson draw of mean l at the uniform u for the lanes with `has`.
+  __device__ __forceinline__ int32_t draw(Counters& cnt, bool has, float l, float u, uint64_t c, int slot,
+                                          bool& fail) const {
+    int32_t kk = 0;
+    const bool asym = has & (l >= POIS_ASYM_MIN) & (l < POIS_ASYM_MAX);
+    if (wave_any(asym)) {
+      bool ex = false;
+      int32_t m = -1;
+      const int32_t ka = poisson_asym_f32(__builtin_fmaxf(l, POIS_ASYM_MIN), u, ex, m);
+      kk = asym ? ka : 0;
+      cnt.w.asym += asym ? 1u : 0u;
+      cnt.w.draws += asym ? 1u : 0u;
+      const bool exact = asym & ex;
+      if (wave_any(exact)) {
+        cnt.w.exact += exact ? 1u : 0u;
+        if (exact) kk = poisson_exact_f64((double)l, (double)u, m);
+      }
+    }
+    const bool inv = has & (l < POIS_ASYM_MIN);
+    if (wave_any(inv)) {
+      // the search of draw_all for one reaction
+      float p = fast_exp(-l), Fc = p;
+      bool live = inv & (u > Fc);
+      for (int it = 0; it < INV_MAX_K && wave_any(live); it += 2) {
+        const float r1 = fast_rcp((float)(it + 1));
+        const float r2 = fast_rcp((float)(it + 2));
+        const float q1 = p * l;
+        const float p1 = r1 * q1;
+        const float F1 = __builtin_fmaf(r1, q1, Fc);
+        const float q2 = p1 * l;
+        const float F2 = __builtin_fmaf(r2, q2, F1);
+        kk = live ? ((u > F1) ? it + 2 : it + 1) : kk;
+        live = live & (u > F2) & (F2 > Fc);
+        p = r2 * q2;
+        Fc = F2;
+      }
+      cnt.w.draws += inv ? 1u : 0u;
+      cnt.w.inv += inv ? (unsigned int)kk : 0u;
+    }
+    const bool wide = has & (l >= POIS_ASYM_MAX);
+    if (wave_any(wide)) {
+      if (wide) {
+        const Draw dr = ptrs_wide(key.k0, key.k1, key.s_lo, key.s_hi, c, slot, l);
+        cnt.w.ptrs += dr.iters;
+        cnt.w.draws += 2 * dr.iters;
+        fail = fail | (dr.k < 0);
+        kk = (int32_t)dr.k;
+      }
+    }
+    return kk;
+  }
+
+  // Every reaction's draw by the simulation's own lane.
+  __device__ __forceinline__ void draw_all(Counters& cnt, bool bad, const float (&lam)[MP], const float (&u)[MP],
+                                           uint64_t grp, int32_t (&K)[MP], bool& fail) const {
+    unsigned inv = 0, exact = 0, wide = 0, nasym = 0;
+    int32_t mb[MP];
+#pragma unroll
+    for (int j = 0; j < MP; ++j) {
+      const float l = lam[j];
+      const bool asym = !bad & (l >= POIS_ASYM_MIN) & (l < POIS_ASYM_MAX);
+      bool ex = false;
+      int32_t m = -1;
+      int32_t k = 0;
+      if (wave_any(asym)) k = poisson_asym_f32(__builtin_fmaxf(l, POIS_ASYM_MIN), u[j], ex, m);
+      K[j] = asym ? k : K[j];
+      mb[j] = m;
+      exact |= (asym & ex) ? (1u << j) : 0u;
+      nasym += asym ? 1u : 0u;
+      inv |= (!bad & (l > 0.0f) & (l < POIS_ASYM_MIN)) ? (1u << j) : 0u;
+      wide |= (!bad & (l >= POIS_ASYM_MAX)) ? (1u << j) : 0u;
+    }
+    cnt.w.asym += nasym;
+    cnt.w.draws += nasym;
+    // near an integer boundary, or in a far tail: decide exactly in FP64
+    if (wave_any(exact != 0u)) {
+      cnt.w.exact += (unsigned int)__builtin_popcount(exact);
+#pragma unroll
+      for (int j = 0; j < MP; ++j)
+        if ((exact >> j) & 1u) K[j] = poisson_exact_f64((double)lam[j], (double)u[j], mb[j]);
+    }
+    // sequential-search inversion (0 < lambda < 10) for all such reactions
+    // in lock-step, two search steps per trip: a live search at k = it
+    // steps to it + 1 and it + 2 and stops at the first k with u <= F(k);
+    // p and F past a search's end are computed but never read
+    if (wave_any(inv != 0u)) {
+      float p[MP], Fc[MP];
+      bool live[MP];
+      bool any_live = false;
 #pragma unroll
       for (int j = 0; j < MP; ++j) {
-        const float l = (j < M && !crit[j]) ? a[j] * tau : 0.0f;
-        lam[j] = l;
-        const Words4& wd = W[j >> 2];
-        const uint32_t word = (j & 3) == 0 ? wd.w0 : (j & 3) == 1 ? wd.w1 : (j & 3) == 2 ? wd.w2 : wd.w3;
-        u[j] = u24(word);
-        const bool asym = (l >= POIS_ASYM_MIN) & (l < POIS_ASYM_MAX);
-        bool ex = false;
-        int32_t m = -1;
-        int32_t k = 0;
-        if (wave_any(asym)) k = poisson_asym_f32(__builtin_fmaxf(l, POIS_ASYM_MIN), u[j], ex, m);
-        if (!crit[j]) K[j] = asym ? k : 0;
-        mb[j] = m;
-        exact |= (asym & ex) ? (1u << j) : 0u;
-        nasym += asym ? 1u : 0u;
-        inv |= ((l > 0.0f) & (l < POIS_ASYM_MIN)) ? (1u << j) : 0u;
-        wide |= (l >= POIS_ASYM_MAX) ? (1u << j) : 0u;
-        bad = bad | (l >= (float)LAMBDA_LIMIT);
+        const bool on = (inv >> j) & 1u;
+        p[j] = fast_exp(-lam[j]);
+        Fc[j] = p[j];
+        live[j] = on && u[j] > Fc[j];
+        if (on) K[j] = 0;
+        any_live = any_live | live[j];
       }
-      if (bad) return FLAG_OVERFLOW;
-      cnt.w.asym += nasym;
-      cnt.w.uniforms += nasym;
-      // near an integer boundary, or in a far tail: decide exactly in FP64
-      if (wave_any(exact != 0u)) {
-        cnt.w.exact += (unsigned int)__builtin_popcount(exact);
-#pragma unroll
-        for (int j = 0; j < MP; ++j)
-          if ((exact >> j) & 1u) K[j] = poisson_exact_f64((double)lam[j], (double)u[j], mb[j]);
-      }
-      // sequential-search inversion (0 < lambda < 10) for all such reactions
-      // in lock-step, two search steps per trip: a live search at k = it
-      // steps to it + 1 and it + 2 and stops at the first k with u <= F(k);
-      // p and F past a search's end are computed but never read
-      if (wave_any(inv != 0u)) {
-        float p[MP], Fc[MP];
-        bool live[MP];
-        bool any_live = false;
+      cnt.w.draws += (unsigned int)__builtin_popcount(inv);
+      for (int it = 0; it < INV_MAX_K && wave_any(any_live); it += 2) {
+        const float r1 = fast_rcp((float)(it + 1));
+        const float r2 = fast_rcp((float)(it + 2));
+        any_live = false;
 #pragma unroll
         for (int j = 0; j < MP; ++j) {
-          const bool on = (inv >> j) & 1u;
-          p[j] = fast_exp(-lam[j]);
-          Fc[j] = p[j];
-          live[j] = on && u[j] > Fc[j];
-          if (on) K[j] = 0;
+          const float q1 = p[j] * lam[j];
+          const float p1 = r1 * q1;
+          const float F1 = __builtin_fmaf(r1, q1, Fc[j]);
+          const float q2 = p1 * lam[j];
+          const float F2 = __builtin_fmaf(r2, q2, F1);
+          K[j] = live[j] ? ((u[j] > F1) ? it + 2 : it + 1) : K[j];
+          // a search also ends where the FP32 sum stops growing: past the
+          // mode every later term is smaller still, and a u above that sum
+          // (u24 can be 1.0, the sum can end a few ulps below it) would
+          // otherwise run to INV_MAX_K
+          live[j] = live[j] && (u[j] > F2) && (F2 > Fc[j]);
           any_live = any_live | live[j];
-        }
-        cnt.w.uniforms += (unsigned int)__builtin_popcount(inv);
-        for (int it = 0; it < INV_MAX_K && wave_any(any_live); it += 2) {
-          const float r1 = fast_rcp((float)(it + 1));
-          const float r2 = fast_rcp((float)(it + 2));
-          any_live = false;
-#pragma unroll
-          for (int j = 0; j < MP; ++j) {
-            const float p1 = p[j] * lam[j] * r1;
-            const float F1 = Fc[j] + p1;
-            const float p2 = p1 * lam[j] * r2;
-            const float F2 = F1 + p2;
-            K[j] = live[j] ? ((u[j] > F1) ? it + 2 : it + 1) : K[j];
-            // a search also ends where the FP32 sum stops growing: past the
-            // mode every later term is smaller still, and a u above that sum
-            // (u24 can be 1.0, the sum can end a few ulps below it) would
-            // otherwise run to INV_MAX_K
-            live[j] = live[j] && (u[j] > F2) && (F2 > Fc[j]);
-            any_live = any_live | live[j];
-            p[j] = p2;
-            Fc[j] = F2;
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < MP; ++j)
-          if ((inv >> j) & 1u) cnt.w.inv += (unsigned int)K[j];
-      }
-      // means of 2^16 and above (rare): PTRS, one reaction at a time
-      if (wave_any(wide != 0u)) {
-#pragma unroll
-        for (int j = 0; j < MP; ++j) {
-          if ((wide >> j) & 1u) {
-            const Draw dr = ptrs_wide(key.k0, key.k1, key.s_lo, key.s_hi, grp + (uint64_t)(j >> 2), j & 3,
-                                      lam[j]);
-            cnt.w.ptrs += dr.iters;
-            cnt.w.uniforms += 2 * dr.iters;
-            if (dr.k < 0) return FLAG_PTRS;
-            K[j] = (int32_t)dr.k;
-          }
+          p[j] = r2 * q2;
+          Fc[j] = F2;
         }
       }
-      bool ok = true, big = false;
 #pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        int64_t sacc = x[i];
-#pragma unroll
-        for (int j = 0; j < MP; ++j) {
-          const int v = tab.V(i, j);
-          if (v != 0) sacc += (int64_t)K[j] * v;
-        }
-        ok = ok & (sacc >= 0);
-        big = big | (sacc >= COUNT_LIMIT);
-        xn[i] = (int32_t)sacc;
-      }
-      if (ok) return big ? FLAG_OVERFLOW : 0;
-      cnt.rejected += 1;
-      tau = tau * 0.5f;
+      for (int j = 0; j < MP; ++j)
+        if ((inv >> j) & 1u) cnt.w.inv += (unsigned int)K[j];
     }
-    return FLAG_HALVING;
+    // means of 2^16 and above (rare): PTRS, one reaction at a time
+    if (wave_any(wide != 0u)) {
+#pragma unroll
+      for (int j = 0; j < MP; ++j) {
+        if ((wide >> j) & 1u) {
+          const Draw dr = ptrs_wide(key.k0, key.k1, key.s_lo, key.s_hi, grp + (uint64_t)(j >> 2), j & 3, lam[j]);
+          cnt.w.ptrs += dr.iters;
+          cnt.w.draws += 2 * dr.iters;
+          fail = fail | (dr.k < 0);
+          K[j] = (int32_t)dr.k;
+        }
+      }
+    }
   }
 };
 

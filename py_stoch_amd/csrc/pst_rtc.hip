@@ -29,6 +29,8 @@ const char* const kOptsFp64[] = {"--offload-arch=gfx950", "-O3", "-std=c++17",
                                  "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                                  "-ffp-contract=off"};
 
+const char* const kSuffix[] = {"", "_paired", "_group"};  // kernel name suffix per RtcForm
+
 void arr(std::string& s, const char* name, const int8_t* v, int n) {
   s += "  static constexpr int8_t ";
   s += name;
@@ -133,7 +135,8 @@ int compile(const std::string& source, int precision, std::vector<char>* code, s
 }  // namespace
 
 std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
-                       const std::vector<std::string>& hazards, int waves_per_eu, bool paired) {
+                       const std::vector<std::string>& hazards, int waves_per_eu, RtcForm form) {
+  const bool paired = form == RTC_PAIRED;
   const int N = net.N, M = net.M;
   std::vector<int8_t> v(N * M), ord(N * M), stp(N * M), E(N, 0);
   for (int i = 0; i < N * M; ++i) {
@@ -172,19 +175,20 @@ std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
   s += "  }\n};\n}  // namespace pst\n";
   s += precision == PST_PRECISION_FP64 ? "#define PST_ENGINE EngineF64\n" : "#define PST_ENGINE EngineF32\n";
   s += std::string("#define PST_KERNEL_NAME ") + (precision == PST_PRECISION_FP64 ? "pst_net_fp64" : "pst_net_mixed") +
-       (paired ? "_paired" : "") + "\n";
+       kSuffix[form] + "\n";
   s += paired ? "extern \"C\" __global__ void __launch_bounds__(512)" : "extern \"C\" __global__ void __launch_bounds__(256)";
   if (waves_per_eu > 0) s += " __attribute__((amdgpu_waves_per_eu(" + std::to_string(waves_per_eu) + ")))";
   s += "\n"
        "PST_KERNEL_NAME(const pst::JobParams* __restrict__ jobs, int n_jobs, unsigned int* __restrict__ queue,\n"
        "                 unsigned long long* __restrict__ stats, pst::Range range) {\n";
   s += std::string("  pst::") + (paired ? "run_driver_paired" : "run_driver") +
-       "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>>(jobs, n_jobs, queue, stats, "
+       "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>" +
+       (paired ? "" : form == RTC_GROUP ? ", true" : ", false") + ">(jobs, n_jobs, queue, stats, "
        "range.f_end, range.resume);\n}\n";
   return s;
 }
 
-int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::string* err, bool paired) {
+int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::string* err, RtcForm form) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) {
@@ -233,12 +237,12 @@ int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::st
   }
   RtcKernel k;
   const std::string name = std::string(precision == PST_PRECISION_FP64 ? "pst_net_fp64" : "pst_net_mixed") +
-                           (paired ? "_paired" : "");
+                           kSuffix[form];
   if ((e = hipModuleGetFunction(&k.fn, mod, name.c_str())) != hipSuccess) {
     *err = std::string("hipModuleGetFunction: ") + hipGetErrorString(e);
     return PST_EHIP;
   }
-  k.block = paired ? 512 : 256;
+  k.block = form == RTC_PAIRED ? 512 : 256;
   int blocks = 0;
   if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k.fn, k.block, 0) == hipSuccess && blocks > 0)
     k.blocks_per_cu = blocks;

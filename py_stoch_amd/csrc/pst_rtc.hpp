@@ -36,15 +36,18 @@ struct RtcKernel {
 // C expression per reaction (X(i), C(k), R(v), see pst_network.hazards).
 // waves_per_eu > 0 asks the compiler for register use that fits that many
 // wavefronts per SIMD (the kernel's arithmetic, and so its results, do not
-// change).  paired: the kernel runs run_driver_paired (workgroups of 512
-// lanes: four decide and four burst wavefronts), named pst_net_*_paired.
+// change).  RTC_PAIRED: the kernel runs run_driver_paired (workgroups of 512
+// lanes: four decide and four burst wavefronts), named pst_net_*_paired;
+// RTC_GROUP: run_driver with a group of lanes per simulation (fewer than 64
+// simulations per wavefront), named pst_net_*_group.
+enum RtcForm { RTC_PLAIN = 0, RTC_PAIRED = 1, RTC_GROUP = 2 };
 std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
-                       const std::vector<std::string>& hazards, int waves_per_eu = 0, bool paired = false);
+                       const std::vector<std::string>& hazards, int waves_per_eu = 0, RtcForm form = RTC_PLAIN);
 
 // Compile (or fetch from the cache) the kernel for `source` on the current
-// device (`paired` as given to rtc_source).  Returns 0, or a PST_* status
+// device (`form` as given to rtc_source).  Returns 0, or a PST_* status
 // with a message in err.
-int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::string* err, bool paired = false);
+int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::string* err, RtcForm form = RTC_PLAIN);
 
 // Launch a specialised kernel: `jobs` is a device array of n_jobs JobParams;
 // `waves` simulation wavefronts, four per workgroup.
