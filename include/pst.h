@@ -238,7 +238,8 @@ int pst_batch_plan_execute(pst_plan* plan, int32_t* const* O_dev, const int64_t*
  */
 typedef struct pst_launch {
   int32_t lanes_shift;        /* simulations per wavefront = library choice >> lanes_shift */
-  int32_t ssa_slice;          /* SSA-only steps per pass (pure SSA: 2 ssa_slice + 1) */
+  int32_t ssa_slice;          /* SSA steps per pass while lanes decide: 1 + ssa_slice, more the more
+                                 lanes are in a burst than deciding (up to 8 times as many) */
   int32_t waves_trim;         /* resident wavefronts per SIMD held back from the kernel's
                                  occupancy limit (at least one stays): with fewer lanes
                                  than simulations, the work queue refills lanes and a
@@ -247,9 +248,11 @@ typedef struct pst_launch {
   int32_t burst_waves;        /* 1: tau-leaping network kernels run in workgroups of four
                                  decide and four burst wavefronts; a simulation's SSA
                                  fallback burst (P3.py:71-151) moves through LDS to the
-                                 paired burst wavefront and back */
+                                 paired burst wavefront and back.  0: they do not.  A plan
+                                 without a launch shape of its own pairs while one wavefront
+                                 per SIMD holds all its simulations */
   double kernel_ms;           /* kernel time of the chosen shape on the tuning horizon */
-  double default_ms;          /* same for the library's default shape (0, 7) */
+  double default_ms;          /* same for the library's default shape */
 } pst_launch;
 int pst_plan_autotune(pst_plan* plan, int32_t* const* O_dev, const int64_t* o_strides,
                       int32_t* const* flags_dev, void* stream, double fraction, pst_launch* chosen);

@@ -300,21 +300,52 @@ void pack_jobs(const std::vector<PlanJob>& jobs, int cls, std::vector<unsigned c
   *count = (int)v.size();
 }
 
-// Simulations per wavefront for one launch (jobs `ids`): 64 unless the launch
-// holds fewer than 64 simulations per SIMD, then the smallest power of two
-// that still needs no more wavefronts than the chip has SIMDs.  A wavefront
-// issues the same instructions whatever its lane count, so spreading a small
-// launch over every SIMD costs nothing per wavefront and leaves each one with
-// fewer divergent paths and a shorter slowest-lane tail.
-int lanes_for(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int simds) {
-  auto need = [&](int L) {
-    int64_t n = 0;
-    for (int q : ids) n += ((int64_t)jobs[q].p.n_sims + L - 1) / L;
-    return n;
-  };
+// Simulations per wavefront when `need(L)` wavefronts hold L each: 64 unless
+// the launch holds fewer than 64 simulations per SIMD, then the smallest power
+// of two that needs (up to a tenth more) no more wavefronts than the chip has
+// SIMDs.  A wavefront issues the same instructions whatever its lane count, so
+// spreading a small launch over every SIMD costs nothing per wavefront and
+// leaves each with fewer divergent paths, a shorter slowest-lane tail and
+// lanes that share one simulation's work.  The tenth keeps a launch just
+// beyond a power of two from running on half the SIMDs: Lotka-Volterra,
+// 16,411 simulations, 32 -> 16 per wavefront (513 -> 1026 wavefronts on 1024
+// SIMDs): FP64 72 -> 53 ms, mixed 35.6 -> 27.6 ms; at twice as many wavefronts
+// as SIMDs the second one per SIMD costs as much as it hides (Schloegl SSA,
+// 8192 simulations, 8 -> 4: 3.6 -> 4.1 ms).
+template <class Need>
+int spread_lanes(Need need, int simds) {
   int L = 64;
-  while (L > 1 && need(L / 2) <= (int64_t)simds) L /= 2;
+  while (L > 1 && need(L / 2) * 10 <= (int64_t)simds * 11) L /= 2;
   return L;
+}
+
+// wavefronts of the jobs `ids` at L simulations each
+int64_t waves_at(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int L) {
+  int64_t n = 0;
+  for (int q : ids) n += ((int64_t)jobs[q].p.n_sims + L - 1) / L;
+  return n;
+}
+
+int lanes_for(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int simds) {
+  return spread_lanes([&](int L) { return waves_at(jobs, ids, L); }, simds);
+}
+
+// Whether a launch of a tau-leaping network kernel runs its SSA bursts on
+// paired wavefronts when the launch shape leaves it open: yes while one
+// wavefront per SIMD holds every simulation (the burst wavefront then takes
+// issue slots that would stay empty) and a wavefront holds several simulations
+// (alone it never waits for another's burst), if the hand-off slots fit LDS.
+// Measured, one role / paired: Schloegl mixed 2048 simulations 5.3 / 4.5 ms,
+// 20,000 8.6 / 6.4, 65,536 10.9 / 7.8, 262,144 (four wavefronts per SIMD)
+// 31.0 / 33.5; Lotka-Volterra FP64 16,411 53 / 43, 65,536 107 / 93, 131,072 (to
+// t = 6) 60 / 65; 128 Schloegl simulations, one per wavefront, 3.1 / 3.9.
+bool pair_by_default(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int L, int simds, int precision) {
+  const pst::JobParams& P = jobs[ids[0]].p;
+  if (P.method != PST_METHOD_TAU_LEAPING || L < 2 || waves_at(jobs, ids, L) * 10 > (int64_t)simds * 11) return false;
+  // engine words: rates, counts and 17 more; 6 words around it in a slot
+  const int rates = std::max(1, P.n_rates) * (precision == PST_PRECISION_FP64 ? 2 : 1);
+  const int words = rates + P.N + 17 + 6 + 8 * std::min(P.kappa, 4);
+  return words * 256 * (int)sizeof(uint32_t) <= 60 * 1024;
 }
 
 }  // namespace
@@ -371,7 +402,7 @@ constexpr int kSideStreams = 3;
 // builds of a specialised kernel: one simulation per lane, the same for
 // kOccupancyWaves wavefronts per SIMD, decide + burst wavefronts, a group of
 // lanes per simulation
-enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_PAIR, BUILD_GROUP, NUM_BUILDS };
+enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_PAIR, BUILD_GROUP, BUILD_PAIR_GROUP, NUM_BUILDS };
 struct FixedBuild {
   std::string source;
   pst::RtcForm form = pst::RTC_PLAIN;
@@ -383,6 +414,8 @@ struct FixedBuild {
 struct FixedGroup {
   FixedBuild build[NUM_BUILDS];
   int use = BUILD_PLAIN;  // the build this execute launches
+  bool pair = false;      // ... with SSA bursts on paired wavefronts
+  bool pair_failed = false;
   std::vector<int> jobs;
   void* d_jobs = nullptr;
   size_t d_bytes = 0;
@@ -409,7 +442,8 @@ struct pst_plan {
   int lanes_shift = 0;        // launch shape (pst_plan_autotune)
   int ssa_slice = kSsaSlice;
   int waves_trim = 0;
-  int burst_waves = 0;        // 1: tau-leaping network kernels run bursts on paired wavefronts
+  int burst_waves = -1;       // 1: tau-leaping network kernels run bursts on paired wavefronts; 0: they do
+                              // not; -1: pair_by_default
   int range_pos = 0;          // samples every simulation has recorded in the pending ranges (0: none)
   uint64_t generation = 0;    // changes whenever the descriptors or the launch shape change
   hipGraph_t graph = nullptr; // sample-range chunks captured by pst_plan_graph_create
@@ -429,6 +463,35 @@ static int fixed_kernel(FixedBuild& b, int precision, const char* what) {
     if (rc != PST_OK) return fail(rc, "%s%s", what, err.c_str());
     b.tried = true;
   }
+  return PST_OK;
+}
+
+// The build of a network kernel for a launch at the jobs' lane counts: SSA
+// bursts of tau-leaping jobs on paired wavefronts if the launch shape says so
+// (or leaves it open and pair_by_default); a group of lanes per simulation if a
+// wavefront has fewer than 64; the occupancy build if the plain build cannot
+// hold the launch resident at once.
+static int choose_build(pst_plan* p, FixedGroup& g, int simds) {
+  const int L = p->jobs[g.jobs[0]].p.lanes;
+  int rc;
+  g.pair = p->jobs[g.jobs[0]].p.method == PST_METHOD_TAU_LEAPING &&
+           (p->burst_waves == 1 ||
+            (p->burst_waves < 0 && !g.pair_failed && pair_by_default(p->jobs, g.jobs, L, simds, p->precision)));
+  if (g.pair) {
+    g.use = L < 64 ? BUILD_PAIR_GROUP : BUILD_PAIR;
+    rc = fixed_kernel(g.build[g.use], p->precision, "network kernel (paired build): ");
+    if (rc == PST_OK || p->burst_waves == 1) return rc;
+    g.pair_failed = true;  // not to be had for this network: one role
+    g.pair = false;
+    g_err[0] = 0;
+  }
+  g.use = L < 64 ? BUILD_GROUP : BUILD_PLAIN;
+  if ((rc = fixed_kernel(g.build[g.use], p->precision, "network kernel: ")) != PST_OK) return rc;
+  if (g.use == BUILD_GROUP) return PST_OK;
+  const int plain = g.build[BUILD_PLAIN].k.blocks_per_cu;
+  if (waves_at(p->jobs, g.jobs, L) <= (int64_t)plain * simds) return PST_OK;
+  if ((rc = fixed_kernel(g.build[BUILD_OCC], p->precision, "network kernel (occupancy build): ")) != PST_OK) return rc;
+  if (g.build[BUILD_OCC].k.blocks_per_cu > plain) g.use = BUILD_OCC;
   return PST_OK;
 }
 
@@ -478,8 +541,7 @@ static int enqueue_launches(pst_plan* p, const int* count, int n_wave, int64_t w
     qoff += count[c];
   }
   for (FixedGroup& g : p->fixed) {
-    int64_t need = 0;
-    for (int q : g.jobs) need += ((int64_t)p->jobs[q].p.n_sims + p->jobs[q].p.lanes - 1) / p->jobs[q].p.lanes;
+    const int64_t need = waves_at(p->jobs, g.jobs, p->jobs[g.jobs[0]].p.lanes);
     const pst::RtcKernel* k = &g.build[g.use].k;
     const int64_t resident = (int64_t)trimmed(k->blocks_per_cu, p->waves_trim) * p->cu_count * 4;
     const int waves = (int)(need < resident ? need : resident);
@@ -724,6 +786,8 @@ int pst_batch_plan_create(const pst_job* jobs, int32_t n_jobs, pst_plan** out) {
         b[BUILD_PAIR].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_PAIRED);
         b[BUILD_GROUP].form = pst::RTC_GROUP;
         b[BUILD_GROUP].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_GROUP);
+        b[BUILD_PAIR_GROUP].form = pst::RTC_PAIRED_GROUP;
+        b[BUILD_PAIR_GROUP].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_PAIRED_GROUP);
       }
       p->fixed[g].jobs.push_back(q);
       pj.fixed = g;
@@ -732,13 +796,14 @@ int pst_batch_plan_create(const pst_job* jobs, int32_t n_jobs, pst_plan** out) {
   // compile what the default launch shape runs, so that a kinetic law the
   // compiler refuses is refused here
   for (FixedGroup& g : p->fixed) {
-    const int b = lanes_for(p->jobs, g.jobs, cu * 4) < 64 ? BUILD_GROUP : BUILD_PLAIN;
-    char what[32];
-    std::snprintf(what, sizeof(what), "job %d: ", g.jobs[0]);
-    const int rc2 = fixed_kernel(g.build[b], p->precision, what);
+    const int L = lanes_for(p->jobs, g.jobs, cu * 4);
+    for (int q : g.jobs) p->jobs[q].p.lanes = L;
+    const int rc2 = choose_build(p, g, cu * 4);
     if (rc2 != PST_OK) {
       pst_plan_destroy(p);
-      return rc2;
+      char msg[sizeof(g_err)];
+      std::snprintf(msg, sizeof(msg), "%s", g_err);
+      return fail(rc2, "job %d: %.480s", g.jobs[0], msg);
     }
   }
   if ((e = hipMalloc(&p->d_queue, sizeof(unsigned int) * n_jobs)) != hipSuccess ||
@@ -805,27 +870,9 @@ static int prepare_plan(pst_plan* p, int32_t* const* O_dev, const int64_t* o_str
     for (int q : g.jobs) p->jobs[q].p.lanes = L;
   }
   for (PlanJob& pj : p->jobs) pj.p.ssa_slice = p->ssa_slice;
-  // The build of each network kernel: SSA bursts of tau-leaping jobs on paired
-  // wavefronts if the launch shape says so; a group of lanes per simulation if
-  // a wavefront has fewer than 64; else one simulation per lane, in the
-  // occupancy build if the plain build cannot hold the launch resident at once.
   for (FixedGroup& g : p->fixed) {
-    const pst::JobParams& P0 = p->jobs[g.jobs[0]].p;
-    int rc;
-    if (p->burst_waves && P0.method == PST_METHOD_TAU_LEAPING) {
-      g.use = BUILD_PAIR;
-      if ((rc = fixed_kernel(g.build[BUILD_PAIR], p->precision, "network kernel (paired build): ")) != PST_OK) return rc;
-      continue;
-    }
-    g.use = P0.lanes < 64 ? BUILD_GROUP : BUILD_PLAIN;
-    if ((rc = fixed_kernel(g.build[g.use], p->precision, "network kernel: ")) != PST_OK) return rc;
-    if (g.use == BUILD_GROUP) continue;
-    int64_t need = 0;
-    for (int q : g.jobs) need += ((int64_t)p->jobs[q].p.n_sims + p->jobs[q].p.lanes - 1) / p->jobs[q].p.lanes;
-    const int plain = g.build[BUILD_PLAIN].k.blocks_per_cu;
-    if (need <= (int64_t)plain * simds) continue;
-    if ((rc = fixed_kernel(g.build[BUILD_OCC], p->precision, "network kernel (occupancy build): ")) != PST_OK) return rc;
-    if (g.build[BUILD_OCC].k.blocks_per_cu > plain) g.use = BUILD_OCC;
+    const int rc = choose_build(p, g, simds);
+    if (rc != PST_OK) return rc;
   }
   // job descriptors, one device array per size class
   for (int c = 0; c < pst::NUM_CLASSES; ++c) count[c] = 0;
@@ -1203,21 +1250,27 @@ int pst_plan_autotune(pst_plan* p, int32_t* const* O_dev, const int64_t* o_strid
     return PST_OK;
   };
   double ms = 0.0, def_ms = 0.0, best_ms = 0.0;
-  int best_shift = 0, best_slice = kSsaSlice, best_trim = 0, best_bw = 0;
-  int rc = timed(0, kSsaSlice, 0, 0, &ms);  // warm-up (first launch of each kernel)
-  if (rc == PST_OK) rc = timed(0, kSsaSlice, 0, 0, &def_ms);
+  int best_shift = 0, best_slice = kSsaSlice, best_trim = 0, best_bw = -1;
+  int rc = timed(0, kSsaSlice, 0, -1, &ms);  // warm-up (first launch of each kernel)
+  if (rc == PST_OK) rc = timed(0, kSsaSlice, 0, -1, &def_ms);
   best_ms = def_ms;
-  // paired wavefronts apply to network kernels of tau-leaping jobs; the SSA
-  // slice then matters only to the plan's other launches
-  bool pairable = false, others = false;
-  for (const FixedGroup& g : p->fixed) pairable = pairable || p->jobs[g.jobs[0]].p.method == PST_METHOD_TAU_LEAPING;
+  // paired wavefronts apply to network kernels of tau-leaping jobs (the SSA
+  // slice then matters only to the plan's other launches); `paired` / `single`:
+  // whether the default shape ran any of them with / without
+  bool paired = false, single = false, others = false;
+  for (const FixedGroup& g : p->fixed) {
+    if (p->jobs[g.jobs[0]].p.method != PST_METHOD_TAU_LEAPING) continue;
+    paired = paired || g.pair;
+    single = single || !g.pair;
+  }
+  const int def_bw = paired ? 1 : 0;
   for (const PlanJob& pj : p->jobs) others = others || pj.fixed < 0;
   const int slices[3] = {3, 7, 15};
-  for (int bw = 0; bw <= (pairable ? 1 : 0) && rc == PST_OK; ++bw) {
+  for (int bw = 0; bw <= (paired || single ? 1 : 0) && rc == PST_OK; ++bw) {
     for (int trim = 0; trim <= 1 && rc == PST_OK; ++trim) {
       for (int shift = 0; shift <= 1 && rc == PST_OK; ++shift) {
         for (int k = 0; k < 3 && rc == PST_OK; ++k) {
-          if (bw == 0 && trim == 0 && shift == 0 && slices[k] == kSsaSlice) continue;  // the default, timed above
+          if (trim == 0 && shift == 0 && slices[k] == kSsaSlice && !(bw ? single : paired)) continue;  // the default
           if (bw == 1 && !others && slices[k] != kSsaSlice) continue;
           rc = timed(shift, slices[k], trim, bw, &ms);
           if (rc != PST_OK && bw == 1) {  // no paired build for this network (e.g. its state does not fit LDS)
@@ -1252,7 +1305,7 @@ int pst_plan_autotune(pst_plan* p, int32_t* const* O_dev, const int64_t* o_strid
   chosen->lanes_shift = best_shift;
   chosen->ssa_slice = best_slice;
   chosen->waves_trim = best_trim;
-  chosen->burst_waves = best_bw;
+  chosen->burst_waves = best_bw >= 0 ? best_bw : def_bw;
   chosen->kernel_ms = best_ms;
   chosen->default_ms = def_ms;
   return PST_OK;
@@ -1395,8 +1448,8 @@ int pst_run_noalloc(const pst_network* net, const pst_config* cfg, const double*
   if ((rc = scratch_on_device(dev, &base)) != PST_OK) return rc;
 
   const int simds = cu * 4;
-  int L = 64;  // simulations per wavefront, as for a plan (lanes_for)
-  while (L > 1 && ((int64_t)c.n_sims + L / 2 - 1) / (L / 2) <= (int64_t)simds) L /= 2;
+  // simulations per wavefront, as for a plan
+  const int L = spread_lanes([&](int l) { return ((int64_t)c.n_sims + l - 1) / l; }, simds);
   pst::JobParams P;
   std::memset(&P, 0, sizeof(P));
   P.N = h.N;

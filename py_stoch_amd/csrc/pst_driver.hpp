@@ -81,11 +81,15 @@ struct LaneGroup {
   }
   __device__ __forceinline__ bool lead() const { return !GROUP || r == 0; }
   __device__ __forceinline__ bool mine(int j) const { return !GROUP || (j & (G - 1)) == r; }
-  // p in any lane of the group
+  // p in any lane / in every lane of the group
   __device__ __forceinline__ unsigned long long mask() const { return (G == 64 ? ~0ull : (1ull << G) - 1ull) << base; }
   __device__ __forceinline__ bool any(bool p) const {
     if constexpr (!GROUP) return p;
     return (__builtin_amdgcn_ballot_w64(p) & mask()) != 0ull;
+  }
+  __device__ __forceinline__ bool all(bool p) const {
+    if constexpr (!GROUP) return p;
+    return (~__builtin_amdgcn_ballot_w64(p) & mask()) == 0ull;
   }
   // reaction j's value, from the lane that owns it
   __device__ __forceinline__ int32_t owners(int32_t v, int j) const {
@@ -533,15 +537,20 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
     // (only tau-leaping decides: a compile-time fact in network kernels)
     if (jr.method() == 0 && wave_any(mode == MODE_DECIDE)) {
       mode = decide_pass<GROUP>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
-      // SSA-only steps while lanes are inside a burst
-      if (wave_any(mode == MODE_SSA))
-        mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, jr.p().ssa_slice + 1, f_stop, t_stop, g);
+      // SSA steps of the lanes inside a burst: more of them the more lanes are
+      // in one than deciding (a burst of 100 steps taken 8 at a time waits
+      // through 13 decisions of the others)
+      const unsigned long long ssa = __builtin_amdgcn_ballot_w64(mode == MODE_SSA);
+      if (ssa != 0ull) {
+        const int n_ssa = __builtin_popcountll(ssa);
+        const int n_dec = __builtin_popcountll(__builtin_amdgcn_ballot_w64(mode == MODE_DECIDE));
+        const int times = n_ssa >= 8 * n_dec ? 8 : n_ssa >= 4 * n_dec ? 4 : n_ssa >= 2 * n_dec ? 2 : 1;
+        mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, times * (jr.p().ssa_slice + 1), f_stop, t_stop, g);
+      }
     } else {
       // no lane decides (pure SSA, or every live lane inside a burst): up to
-      // 1 + ssa_slice SSA steps before the next refill, 2 + 2 ssa_slice for
-      // pure SSA, where no lane waits to decide
-      const int cap = jr.p().method == 2 ? 2 * jr.p().ssa_slice + 2 : jr.p().ssa_slice + 1;
-      mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, cap, f_stop, t_stop, g);
+      // 8 (1 + ssa_slice) SSA steps before the next refill
+      mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, 8 * (jr.p().ssa_slice + 1), f_stop, t_stop, g);
     }
   }
 
@@ -619,7 +628,7 @@ struct SlotIO {
   }
 };
 
-template <class Engine, class Ref>
+template <class Engine, class Ref, bool GROUP>
 __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __restrict__ jobs, int n_jobs,
                                                   unsigned int* __restrict__ queue,
                                                   unsigned long long* __restrict__ stats, int f_end, int resume) {
@@ -641,8 +650,8 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
   int64_t sim = -1;
   unsigned long long ev_start = 0;  // cnt.events when this lane's simulation began (here)
   Ref jr;
-  LaneGroup<false> g;
-  g.set(lane, 64);
+  LaneGroup<GROUP> g;
+  g.set(lane, 1);
 
   if (wave < 4) {
     // ---- decide wavefront ----
@@ -651,17 +660,19 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     bool exhausted = false;
     jr.load(jobs);
     int f_stop = range_stop(jr, f_end);
+    g.set(lane, jr.p().lanes);
     for (;;) {
-      // a burst handed back (ended simulations were recorded by the burst lane)
-      if (mode == MODE_AWAY && lds_load_acquire(&s_state[slot]) == SLOT_BACK) {
+      // a burst handed back (ended simulations were recorded by the burst
+      // lane); the lanes of a group take it together
+      if (g.all(mode == MODE_AWAY && lds_load_acquire(&s_state[slot]) == SLOT_BACK)) {
         unsigned long long ev;
         IO::get(s_data, slot, eng, sim, ev, mode);
         ev_start = cnt.events - ev;
         s_state[slot] = SLOT_FREE;
         if (mode != MODE_DONE) mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
       }
-      const bool want = (mode == MODE_DONE) && !exhausted && lane < jr.p().lanes;
-      const unsigned long long wmask = __builtin_amdgcn_ballot_w64(want);
+      const bool want = (mode == MODE_DONE) && !exhausted && (GROUP || lane < jr.p().lanes);
+      const unsigned long long wmask = __builtin_amdgcn_ballot_w64(want & g.lead());
       if (wmask != 0ull) {
         const int n = __builtin_popcountll(wmask);
         const int leader = __builtin_ctzll(wmask);
@@ -671,7 +682,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         const int n_sims = jr.p().n_sims;
         if ((int64_t)base + n >= (int64_t)n_sims) exhausted = true;
         if (want) {
-          const int rank = __builtin_popcountll(wmask & ((1ull << lane) - 1ull));
+          const int rank = __builtin_popcountll(wmask & ((1ull << g.base) - 1ull));
           const int64_t s = (int64_t)base + rank;
           if (s < n_sims) {
             sim = s;
@@ -684,11 +695,12 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         if (job >= n_jobs) break;
         jr.load(jobs + job);
         f_stop = range_stop(jr, f_end);
+        g.set(lane, jr.p().lanes);
         exhausted = false;
         continue;
       }
       if (wave_any(mode == MODE_DECIDE)) {
-            mode = decide_pass<false>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
+            mode = decide_pass<GROUP>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
       } else if (!wave_any(mode == MODE_SSA)) {
         __builtin_amdgcn_s_sleep(2);  // every live lane is away: wait for a burst to come back
       }
@@ -709,17 +721,24 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     int f_stop = 0x7fffffff;
     double t_stop = 0.0;
     for (;;) {
-      const bool pick = !busy && lds_load_acquire(&s_state[slot]) == SLOT_SENT;
-      const unsigned long long pmask = __builtin_amdgcn_ballot_w64(pick);
-      if (pmask != 0ull) {
+      // (the slots of a group are filled by one store of the partner, but may
+      // be read while it is under way)
+      const bool sent = !busy && lds_load_acquire(&s_state[slot]) == SLOT_SENT;
+      const unsigned long long smask = __builtin_amdgcn_ballot_w64(sent);
+      if (smask != 0ull) {
         // all simulations the partner sends belong to its current job
-        const int pj = __builtin_amdgcn_readlane(IO::job(s_data, slot), __builtin_ctzll(pmask));
+        const int pj = __builtin_amdgcn_readlane(IO::job(s_data, slot), __builtin_ctzll(smask));
         if (pj != bjob) {
           jr.load(jobs + pj);
           bjob = pj;
           f_stop = range_stop(jr, f_end);
           t_stop = stop_time(jr, f_stop);
+          g.set(lane, jr.p().lanes);
         }
+      }
+      const bool pick = g.all(sent);
+      const unsigned long long pmask = __builtin_amdgcn_ballot_w64(pick);
+      if (pmask != 0ull) {
         if (pick) {
           unsigned long long ev;
           int m;
@@ -734,7 +753,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         continue;
       }
       bool general;
-      int m = ssa_run<false>(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, general, g);
+      int m = ssa_run<GROUP>(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, general, g);
       if (wave_any(general)) {
             if (general) m = eng.ssa_step(jr, cnt);
       }

@@ -29,7 +29,7 @@ const char* const kOptsFp64[] = {"--offload-arch=gfx950", "-O3", "-std=c++17",
                                  "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                                  "-ffp-contract=off"};
 
-const char* const kSuffix[] = {"", "_paired", "_group"};  // kernel name suffix per RtcForm
+const char* const kSuffix[] = {"", "_paired", "_group", "_paired_group"};  // kernel name suffix per RtcForm
 
 void arr(std::string& s, const char* name, const int8_t* v, int n) {
   s += "  static constexpr int8_t ";
@@ -136,7 +136,8 @@ int compile(const std::string& source, int precision, std::vector<char>* code, s
 
 std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
                        const std::vector<std::string>& hazards, int waves_per_eu, RtcForm form) {
-  const bool paired = form == RTC_PAIRED;
+  const bool paired = form == RTC_PAIRED || form == RTC_PAIRED_GROUP;
+  const bool group = form == RTC_GROUP || form == RTC_PAIRED_GROUP;
   const int N = net.N, M = net.M;
   std::vector<int8_t> v(N * M), ord(N * M), stp(N * M), E(N, 0);
   for (int i = 0; i < N * M; ++i) {
@@ -183,7 +184,7 @@ std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
        "                 unsigned long long* __restrict__ stats, pst::Range range) {\n";
   s += std::string("  pst::") + (paired ? "run_driver_paired" : "run_driver") +
        "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>" +
-       (paired ? "" : form == RTC_GROUP ? ", true" : ", false") + ">(jobs, n_jobs, queue, stats, "
+       (group ? ", true" : ", false") + ">(jobs, n_jobs, queue, stats, "
        "range.f_end, range.resume);\n}\n";
   return s;
 }
@@ -242,7 +243,7 @@ int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::st
     *err = std::string("hipModuleGetFunction: ") + hipGetErrorString(e);
     return PST_EHIP;
   }
-  k.block = form == RTC_PAIRED ? 512 : 256;
+  k.block = (form == RTC_PAIRED || form == RTC_PAIRED_GROUP) ? 512 : 256;
   int blocks = 0;
   if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k.fn, k.block, 0) == hipSuccess && blocks > 0)
     k.blocks_per_cu = blocks;

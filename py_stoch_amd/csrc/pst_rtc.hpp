@@ -39,8 +39,8 @@ struct RtcKernel {
 // change).  RTC_PAIRED: the kernel runs run_driver_paired (workgroups of 512
 // lanes: four decide and four burst wavefronts), named pst_net_*_paired;
 // RTC_GROUP: run_driver with a group of lanes per simulation (fewer than 64
-// simulations per wavefront), named pst_net_*_group.
-enum RtcForm { RTC_PLAIN = 0, RTC_PAIRED = 1, RTC_GROUP = 2 };
+// simulations per wavefront), named pst_net_*_group; RTC_PAIRED_GROUP: both.
+enum RtcForm { RTC_PLAIN = 0, RTC_PAIRED = 1, RTC_GROUP = 2, RTC_PAIRED_GROUP = 3 };
 std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
                        const std::vector<std::string>& hazards, int waves_per_eu = 0, RtcForm form = RTC_PLAIN);
 
