@@ -73,6 +73,18 @@ struct Range {
 };
 constexpr Range FULL_RUN = {0x7fffffff, 0};
 
+// A job's settings re-read from its descriptor, for the rarely used ones (a
+// simulation's start and end, the saved-state record): the pointer is hidden
+// from the optimizer, so the scalar loads stay where they are used instead of
+// holding a register through the simulation loop.
+__device__ __forceinline__ const JobParams& cold_params(const JobParams* jp) {
+  uint64_t a = (uint64_t)jp;
+  a = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+  asm volatile("" : "+s"(a));
+  return *(const JobParams*)(__attribute__((address_space(4))) const JobParams*)a;
+}
+
 // Copy a job's settings into VGPRs (an empty asm on each 32-bit word hides
 // their uniformity).  They are read only by per-lane arithmetic (addresses,
 // sample cursor, queue bounds), and held in SGPRs they would exceed the
@@ -126,6 +138,8 @@ struct JobRef {
   static constexpr int EW = (NP * MP / 2 + 63) / 64;  // registers of an entry list
   uint32_t fac[EW], vent[EW], vrange, species;
   JobParams P;
+  const JobParams* jp;
+  __device__ __forceinline__ const JobParams& cold() const { return cold_params(jp); }
 
   static __device__ __forceinline__ uint32_t* rows() {
     __shared__ uint32_t buf[4 * NP * MP / 4];
@@ -145,7 +159,8 @@ struct JobRef {
     species = lane < NP ? jd->tab.species[lane] : 0u;
     const uint32_t* d = reinterpret_cast<const uint32_t*>(jd->tab.vrow);
     if (lane < NP * MP / 4) rows()[lane] = d[lane];  // NP * MP / 4 <= 64; read by this wavefront only
-    load_params_vgpr(&P, &jd->p);
+    jp = &jd->p;
+    load_params_vgpr(&P, jp);
   }
   static __device__ __forceinline__ uint32_t word(uint32_t v, int i) { return (uint32_t)__builtin_amdgcn_readlane((int)v, i); }
   static __device__ __forceinline__ uint32_t entry(const uint32_t (&v)[EW], int e) {
@@ -318,9 +333,15 @@ struct FixedRef {
   static constexpr int kOutLds = Net::kappa < 4 ? Net::kappa : 4;  // recorded species gathered in LDS
   using Dev = JobParams;
   FixedParams<Net> P;
-  __device__ __forceinline__ void load(const JobParams* jp) { load_params_vgpr(&P, jp); }
+  const JobParams* jp;
+  __device__ __forceinline__ void load(const JobParams* p) {
+    jp = p;
+    load_params_vgpr(&P, p);
+  }
+  __device__ __forceinline__ const JobParams& cold() const { return cold_params(jp); }
   __device__ __forceinline__ const FixedParams<Net>& p() const { return P; }
   __device__ __forceinline__ static constexpr int method() { return Net::method; }
+  __device__ __forceinline__ static constexpr int n_reactions() { return kMP; }
   // bytes V(i, 4 r) .. V(i, 4 r + 3) as one word
   static constexpr uint32_t Vword(int i, int r) {
     uint32_t w = 0;
@@ -456,7 +477,7 @@ inline NetTab<NP, MP> make_tab(const HostNet& h) {
 
 // Launchers, one per translation unit (precision).  `jobs` is a device array
 // of JobDev<NP,MP> for the size class `cls`, `queue` n_jobs zeroed counters,
-// `waves` the number of wavefronts to launch, `group` whether their jobs have
+// `waves` the number of wavefronts to launch, `group` whether the jobs have
 // fewer than 64 simulations per wavefront (a group of lanes per simulation).
 int launch_fp64(int cls, const void* jobs, int n_jobs, unsigned int* queue, unsigned long long* stats,
                 int waves, Range range, bool group, hipStream_t stream);
@@ -476,10 +497,6 @@ int launch_wave(const void* jobs, int n_jobs, unsigned int* queue, unsigned long
                 hipStream_t stream);
 int blocks_per_cu_wave();
 bool make_wave_tab(const HostNet& h, WaveTab* t, char* why, size_t why_len);
-
-// kernel of a size class: 2 cls, or 2 cls + 1 for the group form (the 16 x 16
-// table has none: its code for one simulation per lane is large already)
-inline int table_form(int cls, bool group) { return 2 * cls + (group && cls < 2 ? 1 : 0); }
 
 // smallest compiled size class holding (N, M, kappa), or -1
 inline int size_class(int N, int M, int kappa) {

@@ -341,7 +341,7 @@ int lanes_for(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int
 // t = 6) 60 / 65; 128 Schloegl simulations, one per wavefront, 3.1 / 3.9.
 bool pair_by_default(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int L, int simds, int precision) {
   const pst::JobParams& P = jobs[ids[0]].p;
-  if (P.method != PST_METHOD_TAU_LEAPING || L < 2 || waves_at(jobs, ids, L) * 10 > (int64_t)simds * 11) return false;
+  if (P.method != PST_METHOD_TAU_LEAPING || L < 2 || waves_at(jobs, ids, L) > 2 * (int64_t)simds) return false;
   // engine words: rates, counts and 17 more; 6 words around it in a slot
   const int rates = std::max(1, P.n_rates) * (precision == PST_PRECISION_FP64 ? 2 : 1);
   const int words = rates + P.N + 17 + 6 + 8 * std::min(P.kappa, 4);
@@ -399,10 +399,10 @@ constexpr int kOccupancyWaves = 3;
 // counters, and no result depends on the order.
 constexpr int kSideStreams = 3;
 
-// builds of a specialised kernel: one simulation per lane, the same for
-// kOccupancyWaves wavefronts per SIMD, decide + burst wavefronts, a group of
-// lanes per simulation
-enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_PAIR, BUILD_GROUP, BUILD_PAIR_GROUP, NUM_BUILDS };
+// builds of a specialised kernel: one simulation per lane, the same compiled
+// for kOccupancyWaves wavefronts per SIMD, a group of lanes per simulation, and
+// decide + burst wavefronts with one simulation or a group
+enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_GROUP, BUILD_PAIR, BUILD_PAIR_GROUP, NUM_BUILDS };
 struct FixedBuild {
   std::string source;
   pst::RtcForm form = pst::RTC_PLAIN;
@@ -468,9 +468,8 @@ static int fixed_kernel(FixedBuild& b, int precision, const char* what) {
 
 // The build of a network kernel for a launch at the jobs' lane counts: SSA
 // bursts of tau-leaping jobs on paired wavefronts if the launch shape says so
-// (or leaves it open and pair_by_default); a group of lanes per simulation if a
-// wavefront has fewer than 64; the occupancy build if the plain build cannot
-// hold the launch resident at once.
+// (or leaves it open and pair_by_default); the occupancy build if the plain
+// build cannot hold the launch resident at once.
 static int choose_build(pst_plan* p, FixedGroup& g, int simds) {
   const int L = p->jobs[g.jobs[0]].p.lanes;
   int rc;
@@ -782,12 +781,11 @@ int pst_batch_plan_create(const pst_job* jobs, int32_t n_jobs, pst_plan** out) {
         FixedBuild* b = p->fixed[g].build;
         b[BUILD_PLAIN].source = std::move(src);
         b[BUILD_OCC].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, kOccupancyWaves);
-        b[BUILD_PAIR].form = pst::RTC_PAIRED;
-        b[BUILD_PAIR].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_PAIRED);
-        b[BUILD_GROUP].form = pst::RTC_GROUP;
-        b[BUILD_GROUP].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_GROUP);
-        b[BUILD_PAIR_GROUP].form = pst::RTC_PAIRED_GROUP;
-        b[BUILD_PAIR_GROUP].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, pst::RTC_PAIRED_GROUP);
+        const pst::RtcForm forms[] = {pst::RTC_GROUP, pst::RTC_PAIRED, pst::RTC_PAIRED_GROUP};
+        for (int i = 0; i < 3; ++i) {
+          b[BUILD_GROUP + i].form = forms[i];
+          b[BUILD_GROUP + i].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, 0, forms[i]);
+        }
       }
       p->fixed[g].jobs.push_back(q);
       pj.fixed = g;

@@ -30,7 +30,7 @@
 
 namespace pst {
 
-enum Mode { MODE_DECIDE = 0, MODE_SSA = 1, MODE_DONE = 2 };
+enum Mode { MODE_DECIDE = 0, MODE_SSA = 1, MODE_DONE = 2, MODE_AWAY = 3 /* paired driver: with the burst lane */ };
 
 struct Counters {
   unsigned long long events;
@@ -39,13 +39,26 @@ struct Counters {
   Work w;
 };
 
-__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
-
-__device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+// The workgroup's counters, in LDS: wavefronts add theirs (once per job, group
+// size and at their end), lanes add the rarely counted events themselves, and
+// the last wavefront to leave adds the sums to the launch's.
+struct WgStats {
+  unsigned long long v[ST_EXACT + 1];
+  uint32_t waves;  // still running
+};
+__device__ __forceinline__ WgStats& wg_stats() {
+  __shared__ WgStats s;
+  return s;
 }
+__device__ __forceinline__ void init_stats() {  // every wavefront of the workgroup, then a barrier
+  if (threadIdx.x <= ST_EXACT) wg_stats().v[threadIdx.x] = 0ull;
+  if (threadIdx.x == 0) wg_stats().waves = blockDim.x / 64u;
+}
+__device__ __forceinline__ void add_stat(StatIdx i, unsigned long long n) {
+  __hip_atomic_fetch_add(&wg_stats().v[i], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
 
 // x[idx] for a run-time idx in [0, NP), as an OR of masked elements: a select
 // chain is folded back into an indexed load by the compiler, which then moves
@@ -66,34 +79,39 @@ __device__ __forceinline__ float pick_f(const float (&x)[NP], int idx) {
   return __builtin_bit_cast(float, r);
 }
 
-// Lane groups (GROUP builds): the 64 lanes of a wavefront hold 64 / G
-// simulations, each replicated over G adjacent lanes that run in lock-step on
-// the same registers; lane r of the group computes what can be split (the
-// random blocks of the next SSA steps, the Poisson draws of reactions r, r +
-// G, ...) and the results are exchanged.  GROUP = false: G = 1.
-template <bool GROUP>
+// Lane groups: the 64 lanes of a wavefront hold 64 / G simulations, each
+// replicated over G adjacent lanes that run in lock-step on the same
+// registers; lane r of the group computes what can be split (the random blocks
+// of the next SSA steps, the Poisson draws of reactions r, r + G, ...) and the
+// results are exchanged.  Forms of a kernel:
+//   ONE       G = 1
+//   GROUPED   G > 1, fixed per job: launches with fewer than 64 simulations per
+//             wavefront (lanes_for in pst_capi.hip)
+//   WIDENING  G = 1 while there are simulations for every lane; grows once the
+//             queue is empty and most lanes of a wavefront are done (regroup)
+enum LaneForm { ONE = 0, GROUPED = 1, WIDENING = 2 };
+template <int FORM>
 struct LaneGroup {
   int G, r, base;  // size, position in the group, the group's first lane
   __device__ __forceinline__ void set(int lane, int sims_per_wave) {
-    G = GROUP ? 64 / sims_per_wave : 1;
-    r = GROUP ? (lane & (G - 1)) : 0;
-    base = GROUP ? (lane & ~(G - 1)) : lane;
+    // (in one scalar register where branches depend on it)
+    G = FORM == ONE ? 1 : 64 / (FORM == WIDENING ? __builtin_amdgcn_readfirstlane(sims_per_wave) : sims_per_wave);
+    r = FORM == ONE ? 0 : lane & (G - 1);
+    base = FORM == ONE ? lane : lane & ~(G - 1);
   }
-  __device__ __forceinline__ bool lead() const { return !GROUP || r == 0; }
-  __device__ __forceinline__ bool mine(int j) const { return !GROUP || (j & (G - 1)) == r; }
+  __device__ __forceinline__ bool grouped() const { return FORM == GROUPED || (FORM == WIDENING && G > 1); }
+  __device__ __forceinline__ bool lead() const { return FORM == ONE || r == 0; }
+  __device__ __forceinline__ bool mine(int j) const { return FORM == ONE || (j & (G - 1)) == r; }
   // p in any lane / in every lane of the group
   __device__ __forceinline__ unsigned long long mask() const { return (G == 64 ? ~0ull : (1ull << G) - 1ull) << base; }
   __device__ __forceinline__ bool any(bool p) const {
-    if constexpr (!GROUP) return p;
-    return (__builtin_amdgcn_ballot_w64(p) & mask()) != 0ull;
+    return FORM == ONE ? p : (__builtin_amdgcn_ballot_w64(p) & mask()) != 0ull;
   }
   __device__ __forceinline__ bool all(bool p) const {
-    if constexpr (!GROUP) return p;
-    return (~__builtin_amdgcn_ballot_w64(p) & mask()) == 0ull;
+    return FORM == ONE ? p : (~__builtin_amdgcn_ballot_w64(p) & mask()) == 0ull;
   }
   // reaction j's value, from the lane that owns it
   __device__ __forceinline__ int32_t owners(int32_t v, int j) const {
-    if constexpr (!GROUP) return v;
     return __builtin_amdgcn_ds_bpermute((base + (j & (G - 1))) * 4, v);
   }
 };
@@ -249,34 +267,36 @@ struct StateIO {
 
 // Engine interface (see EngineF64 / EngineF32):
 //   int  start(job, sim)            -> initial mode, state loaded
-//   int  decide<GROUP>(job, cnt, on, group), int ssa_step(job, cnt) -> next
+//   int  decide(job, cnt, on, group), int ssa_step(job, cnt) -> next
 //     mode (DONE may set flag)
 //   Draw1 ssa_draw(key, c), bool ssa_try(job, draw, tstop, sel, t1): one
 //     ordinary SSA step (ssa_run)
 //   int  flag
 template <class Engine, class Ref>
-__device__ __forceinline__ void finish_sim(const Ref& jr, const Engine& eng, int64_t sim, Counters& cnt,
-                                           unsigned long long ev_start) {
-  int32_t* fl = jr.p().flags;
+__device__ __forceinline__ void finish_sim(const Ref& jr, const Engine& eng, int64_t sim, const Counters& cnt,
+                                           unsigned long long ev_start, bool lead) {
+  int32_t* fl = jr.cold().flags;
   if (fl) glb(fl)[sim] = eng.flag;
-  cnt.flagged += (eng.flag != 0);
-  cnt.fevents += (eng.flag != 0) ? cnt.events - ev_start : 0ull;
+  if (eng.flag != 0 && lead) {
+    add_stat(ST_FLAGGED, 1ull);
+    add_stat(ST_FEVENTS, cnt.events - ev_start);
+  }
 }
 
 // After a step: record an ended simulation, or stop one that has recorded
 // the range's last sample.  Returns the lane's mode.
-template <class Engine, class Ref>
-__device__ __forceinline__ int settle(const Ref& jr, const Engine& eng, int64_t sim, Counters& cnt,
-                                      unsigned long long ev_start, int mode, int f_stop) {
+template <class Engine, class Ref, int FORM>
+__device__ __forceinline__ int settle(const Ref& jr, const Engine& eng, int64_t sim, const Counters& cnt,
+                                      unsigned long long ev_start, int mode, int f_stop, const LaneGroup<FORM>& g) {
   using SIO = StateIO<Engine>;
   if (mode == MODE_DONE) {
-    finish_sim(jr, eng, sim, cnt, ev_start);
-    if (SIO::fits(jr.p())) SIO::save(jr.p(), sim, eng, MODE_DONE, cnt.events - ev_start);
+    finish_sim(jr, eng, sim, cnt, ev_start, g.lead());
+    if (SIO::fits(jr.cold())) SIO::save(jr.cold(), sim, eng, MODE_DONE, cnt.events - ev_start);
     return MODE_DONE;
   }
   if (eng.F >= f_stop) {
-    if (SIO::fits(jr.p())) {
-      SIO::save(jr.p(), sim, eng, mode, cnt.events - ev_start);
+    if (SIO::fits(jr.cold())) {
+      SIO::save(jr.cold(), sim, eng, mode, cnt.events - ev_start);
       return MODE_DONE;
     }
   }
@@ -289,11 +309,11 @@ template <class Engine, class Ref>
 __device__ __forceinline__ int begin_sim(const Ref& jr, Engine& eng, int64_t sim, Counters& cnt,
                                          unsigned long long& ev_start, bool resume, int f_stop) {
   using SIO = StateIO<Engine>;
-  if (resume && SIO::fits(jr.p())) {
+  if (resume && SIO::fits(jr.cold())) {
     unsigned long long ev;
-    const int mode = SIO::load(jr.p(), sim, eng, ev);
+    const int mode = SIO::load(jr.cold(), sim, eng, ev);
     ev_start = cnt.events - ev;
-    eng.Ob = Engine::Out::base(jr.p(), sim);
+    eng.Ob = Engine::Out::base(jr.cold(), sim);
     if (mode == MODE_DONE || eng.F >= f_stop) return MODE_DONE;
     // Without tau-leaping a simulation is only ever in an SSA step (the
     // engines' start and step never return DECIDE then).  Saying so here
@@ -308,13 +328,13 @@ __device__ __forceinline__ int begin_sim(const Ref& jr, Engine& eng, int64_t sim
 
 template <class Ref>
 __device__ __forceinline__ int range_stop(const Ref& jr, int f_end) {
-  return f_end < jr.p().ita ? f_end : jr.p().ita;
+  return f_end < jr.cold().ita ? f_end : jr.cold().ita;
 }
 
 // time of the last sample of the range
 template <class Ref>
 __device__ __forceinline__ double stop_time(const Ref& jr, int f_stop) {
-  return (double)glb(jr.p().I)[f_stop > 0 ? f_stop - 1 : 0];
+  return (double)glb(jr.cold().I)[f_stop > 0 ? f_stop - 1 : 0];
 }
 
 // value of `v` in the lane with byte address `addr` (4 * lane)
@@ -342,9 +362,9 @@ __device__ __forceinline__ double lane_get(double v, int addr) {
 // general step, with about ten of them, takes 1,300 cycles for a single lane.
 // All lanes of the wavefront call this together.
 
-template <bool GROUP, class Engine, class Ref>
+template <class Engine, class Ref, int FORM>
 __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int mode, bool on, int cap, double tstop,
-                                       bool& general, const LaneGroup<GROUP>& g) {
+                                       bool& general, const LaneGroup<FORM>& g) {
   using Out = typename Engine::Out;
   constexpr int kBatch = 4;
   const auto& P = jr.p();
@@ -364,20 +384,20 @@ __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int 
   int n = 0;
   while (wave_any(go)) {
     typename Engine::Draw1 d[kBatch];
-    if constexpr (GROUP) {
-      // lane r of the group draws for step (n + r) % kBatch of the batch
-      const int q = g.G >= kBatch ? (g.r & (kBatch - 1)) : g.r;
-      typename Engine::Draw1 own = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + q));
-      typename Engine::Draw1 own2 = own;
-      if (g.G < kBatch) own2 = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + q + 2));
+    // lane r of the group draws for steps r, r + G, ... of the batch
+    d[0] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + (FORM == ONE ? 0 : g.r & (kBatch - 1))));
+    if (FORM != ONE && g.G >= kBatch) {
 #pragma unroll
-      for (int s = 0; s < kBatch; ++s) {
-        const int src = (g.base + (g.G >= kBatch ? s : (s & 1))) * 4;
-        d[s] = Engine::from_lane(g.G < kBatch && s >= 2 ? own2 : own, src);
-      }
+      for (int s = kBatch - 1; s >= 0; --s) d[s] = Engine::from_lane(d[0], (g.base + s) * 4);
+    } else if (g.grouped()) {
+      d[2] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + g.r + 2));
+      d[3] = Engine::from_lane(d[2], (g.base + 1) * 4);
+      d[2] = Engine::from_lane(d[2], g.base * 4);
+      d[1] = Engine::from_lane(d[0], (g.base + 1) * 4);
+      d[0] = Engine::from_lane(d[0], g.base * 4);
     } else {
 #pragma unroll
-      for (int s = 0; s < kBatch; ++s) d[s] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + s));
+      for (int s = 1; s < kBatch; ++s) d[s] = Engine::ssa_draw(uk, eng.bc + (uint64_t)(uint32_t)(n + s));
     }
     bool act = go, crossed = false;
     int csel = 0;
@@ -430,61 +450,142 @@ __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int 
   return mode;
 }
 
-// Up to `cap` SSA steps of every lane in SSA mode: ordinary ones in ssa_run,
-// and the one it leaves over, if any, through ssa_step.
-template <bool GROUP, class Engine, class Ref>
-__device__ __forceinline__ int ssa_slice(Ref& jr, Engine& eng, int64_t sim, Counters& cnt,
-                                         unsigned long long ev_start, int mode, int cap, int f_stop, double t_stop,
-                                         const LaneGroup<GROUP>& g) {
+// Up to `cap` SSA steps of the lanes with `on`: ordinary ones in ssa_run, and
+// the one it leaves over, if any, through ssa_step.
+template <class Engine, class Ref, int FORM>
+__device__ __forceinline__ int ssa_slice(Ref& jr, Engine& eng, Counters& cnt, int mode, bool on, int cap,
+                                         double t_stop, const LaneGroup<FORM>& g) {
   bool general;
-  mode = ssa_run<GROUP>(jr, eng, cnt, mode, mode == MODE_SSA, cap, t_stop, general, g);
+  mode = ssa_run(jr, eng, cnt, mode, on, cap, t_stop, general, g);
   if (wave_any(general)) {
-    if (general) {
-      mode = eng.ssa_step(jr, cnt);
-      mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-    }
+    if (general) mode = eng.ssa_step(jr, cnt);
   }
   return mode;
 }
 
-// One leap decision of every lane in DECIDE mode.
-template <bool GROUP, class Engine, class Ref>
-__device__ __forceinline__ int decide_pass(Ref& jr, Engine& eng, int64_t sim, Counters& cnt,
-                                           unsigned long long ev_start, int mode, int f_stop,
-                                           const LaneGroup<GROUP>& g) {
-  const bool on = mode == MODE_DECIDE;
-  const int next = eng.template decide<GROUP>(jr, cnt, on, g);
-  mode = on ? next : mode;
-  if (wave_any(on & ((mode == MODE_DONE) | (eng.F >= f_stop)))) {
-    if (on) mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
-  }
-  return mode;
-}
-
-// Adds a wavefront's counters to the launch's.  Lanes of a group count the
+// Adds a wavefront's counters and clears them.  Lanes of a group count the
 // same events: only the first lane's count, except for the Poisson draws,
 // which each lane counts for the reactions it drew.
-template <bool GROUP>
-__device__ __forceinline__ void add_stats(const Counters& cnt, const LaneGroup<GROUP>& g, int lane,
-                                          unsigned long long* __restrict__ stats) {
+template <int FORM>
+__device__ __forceinline__ void add_stats(Counters& cnt, const LaneGroup<FORM>& g) {
   const unsigned long long m = g.lead() ? ~0ull : 0ull;
-  const unsigned long long vals[ST_EXACT + 1] = {cnt.events & m, cnt.leaps & m, cnt.rejected & m, cnt.ssa & m,
-                                                 cnt.flagged & m, (cnt.w.uniforms & m) + cnt.w.draws, cnt.w.ptrs,
-                                                 cnt.w.inv, cnt.w.decisions & m, cnt.w.samples & m, cnt.fevents & m,
-                                                 cnt.w.asym, cnt.w.exact};
   // (32-bit per-lane counters: a lane's share of one launch stays far below 2^32)
+  add_stat(ST_EVENTS, cnt.events & m);
+  add_stat(ST_LEAPS, cnt.leaps & m);
+  add_stat(ST_REJECTED, cnt.rejected & m);
+  add_stat(ST_SSA, cnt.ssa & m);
+  add_stat(ST_UNIFORMS, (cnt.w.uniforms & m) + cnt.w.draws);
+  add_stat(ST_PTRS, cnt.w.ptrs);
+  add_stat(ST_INV, cnt.w.inv);
+  add_stat(ST_DECISIONS, cnt.w.decisions & m);
+  add_stat(ST_SAMPLES, cnt.w.samples & m);
+  add_stat(ST_ASYM, cnt.w.asym);
+  cnt = {};
+}
+__device__ __forceinline__ void leave_stats(int lane, unsigned long long* __restrict__ stats) {
+  uint32_t left = 0;
+  if (lane == 0)
+    left = __hip_atomic_fetch_add(&wg_stats().waves, 0xffffffffu, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+  left = __builtin_amdgcn_readfirstlane(left);
+  if (left == 1u && lane <= ST_EXACT) atomicAdd(&stats[lane], wg_stats().v[lane]);
+}
+
+// A simulation in transit: the engine state, its id, its events so far
+// (for the flagged-events counter), the job index and the next mode.
+template <class Engine, int STRIDE>
+struct SlotIO {
+  static constexpr int EW = (int)(sizeof(Engine) / 4);
+  static constexpr int WORDS = EW + 6;
+  static_assert(sizeof(Engine) % 4 == 0, "engine state is not whole words");
+  // word-major [word][slot]: consecutive lanes hit consecutive banks
+  static __device__ __forceinline__ void put(uint32_t* data, int slot, const Engine& eng, int64_t sim,
+                                             unsigned long long ev, int job, int mode) {
+    uint32_t w[EW];
+    __builtin_memcpy(w, &eng, sizeof(Engine));
 #pragma unroll
-  for (int i = 0; i <= ST_EXACT; ++i) {
-    const unsigned long long sum = wave_sum(vals[i]);
-    if (lane == 0) atomicAdd(&stats[i], sum);
+    for (int i = 0; i < EW; ++i) data[i * STRIDE + slot] = w[i];
+    data[(EW + 0) * STRIDE + slot] = (uint32_t)sim;
+    data[(EW + 1) * STRIDE + slot] = (uint32_t)((uint64_t)sim >> 32);
+    data[(EW + 2) * STRIDE + slot] = (uint32_t)ev;
+    data[(EW + 3) * STRIDE + slot] = (uint32_t)(ev >> 32);
+    data[(EW + 4) * STRIDE + slot] = (uint32_t)job;
+    data[(EW + 5) * STRIDE + slot] = (uint32_t)mode;
+  }
+  static __device__ __forceinline__ void get(const uint32_t* data, int slot, Engine& eng, int64_t& sim,
+                                             unsigned long long& ev, int& mode) {
+    uint32_t w[EW];
+#pragma unroll
+    for (int i = 0; i < EW; ++i) w[i] = data[i * STRIDE + slot];
+    __builtin_memcpy(&eng, w, sizeof(Engine));
+    sim = (int64_t)(((uint64_t)data[(EW + 1) * STRIDE + slot] << 32) | data[(EW + 0) * STRIDE + slot]);
+    ev = ((unsigned long long)data[(EW + 3) * STRIDE + slot] << 32) | data[(EW + 2) * STRIDE + slot];
+    mode = (int)data[(EW + 5) * STRIDE + slot];
+  }
+  static __device__ __forceinline__ int job(const uint32_t* data, int slot) {
+    return (int)data[(EW + 4) * STRIDE + slot];
+  }
+};
+
+// Once a job's queue is empty, the last simulations of a wavefront take more
+// lanes each: with at most 16 of them left they are moved to groups of four
+// or more lanes (up to `cap`), so a leap's draws and the random blocks of SSA
+// steps no longer run one after the other for the slowest simulations, which
+// end the launch.  The states go through LDS (`data`, slots first ..
+// first + 15, word-major); the counters so far are added to the launch's,
+// because which lanes count changes.
+__device__ __forceinline__ int group_cap(int n_reactions) {
+  int c = 4;  // the SSA batch
+  while (c < n_reactions && c < 32) c *= 2;
+  return c;
+}
+template <int FORM>
+__device__ __forceinline__ int wider_group(const LaneGroup<FORM>& g, unsigned long long leads, int cap) {
+  const int n = __builtin_popcountll(leads);
+  int G = g.G < 4 ? 4 : 2 * g.G;
+  if (n == 0 || G > cap || n * G > 64) return 0;
+  while (2 * G <= cap && n * 2 * G <= 64) G *= 2;
+  return G;
+}
+
+template <class Engine, int STRIDE, int FORM>
+__device__ __forceinline__ void regroup(uint32_t* data, int first, int G, LaneGroup<FORM>& g, int lane, Engine& eng,
+                                        int64_t& sim, unsigned long long& ev_start, Counters& cnt, int& mode,
+                                        bool blocks) {
+  using IO = SlotIO<Engine, STRIDE>;
+  using Out = typename Engine::Out;
+  constexpr int BW = Out::KS * OUT_BLOCK;
+  const bool moves = g.lead() & (mode != MODE_DONE);
+  const unsigned long long leads = __builtin_amdgcn_ballot_w64(moves);
+  if (moves) {
+    const int to = first + __builtin_popcountll(leads & ((1ull << lane) - 1ull));
+    IO::put(data, to, eng, sim, cnt.events - ev_start, lane, mode);
+  }
+  add_stats(cnt, g);
+  g.set(lane, 64 / G);
+  const int from = lane / G;
+  mode = MODE_DONE;
+  if (from < __builtin_popcountll(leads)) {
+    unsigned long long ev;
+    IO::get(data, first + from, eng, sim, ev, mode);
+    ev_start = 0ull - ev;
+    if (blocks) {  // the samples of the block in progress
+      const int32_t* old = Out::lds() + (Out::slot() & ~63) + IO::job(data, first + from);
+      int32_t w[BW];
+#pragma unroll
+      for (int i = 0; i < BW; ++i) w[i] = old[i * 256];
+#pragma unroll
+      for (int i = 0; i < BW; ++i) Out::lds()[i * 256 + Out::slot()] = w[i];
+    }
   }
 }
 
-template <class Engine, class Ref, bool GROUP>
+template <class Engine, class Ref, int FORM>
 __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__ jobs, int n_jobs,
                                            unsigned int* __restrict__ queue, unsigned long long* __restrict__ stats,
                                            int f_end, int resume) {
   const int lane = (int)(threadIdx.x & 63u);
+  init_stats();
+  __syncthreads();  // the only barrier: every lane of the workgroup reaches it
   Counters cnt = {};
   Engine eng;
   int mode = MODE_DONE;
@@ -497,13 +598,15 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
   jr.load(jobs);
   int f_stop = range_stop(jr, f_end);
   double t_stop = stop_time(jr, f_stop);
-  LaneGroup<GROUP> g;
-  g.set(lane, jr.p().lanes);
+  LaneGroup<FORM> g;
+  g.set(lane, jr.cold().lanes);
+  constexpr int kSlots = 64;  // sixteen per wavefront
+  __shared__ uint32_t s_move[SlotIO<Engine, kSlots>::WORDS * kSlots];
 
   for (;;) {
     // ---- refill lanes whose simulation ended from the job's queue (the lanes
     // of a group are in lock-step: they end together and take one simulation) ----
-    const bool want = (mode == MODE_DONE) && !exhausted && (GROUP || lane < jr.p().lanes);
+    const bool want = (mode == MODE_DONE) && !exhausted && (FORM != ONE || lane < jr.cold().lanes);
     const unsigned long long wmask = __builtin_amdgcn_ballot_w64(want & g.lead());
     if (wmask != 0ull) {
       const int n = __builtin_popcountll(wmask);
@@ -511,7 +614,7 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
       unsigned int base = 0;
       if (lane == leader) base = atomicAdd(&queue[job], (unsigned int)n);
       base = __shfl(base, leader, 64);
-      const int n_sims = jr.p().n_sims;
+      const int n_sims = jr.cold().n_sims;
       if ((int64_t)base + n >= (int64_t)n_sims) exhausted = true;
       if (want) {
         const int rank = __builtin_popcountll(wmask & ((1ull << g.base) - 1ull));
@@ -522,39 +625,54 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
         }
       }
     }
+    if (FORM == WIDENING && exhausted) {
+      const int G = wider_group(g, __builtin_amdgcn_ballot_w64((mode != MODE_DONE) & g.lead()), group_cap(jr.n_reactions()));
+      if (G != 0)
+        regroup<Engine, kSlots>(s_move, (int)(threadIdx.x >> 6) * 16, G, g, lane, eng, sim, ev_start, cnt, mode,
+                                jr.p().layout == LAYOUT_BLOCKS);
+    }
     if (!wave_any(mode != MODE_DONE)) {
       // this wavefront is idle and its job has no work left: next job
       job += 1;
       if (job >= n_jobs) break;
+      add_stats(cnt, g);
       jr.load(jobs + job);
       f_stop = range_stop(jr, f_end);
       t_stop = stop_time(jr, f_stop);
-      g.set(lane, jr.p().lanes);
+      g.set(lane, jr.cold().lanes);
       exhausted = false;
       continue;
     }
 
-    // (only tau-leaping decides: a compile-time fact in network kernels)
-    if (jr.method() == 0 && wave_any(mode == MODE_DECIDE)) {
-      mode = decide_pass<GROUP>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
+    // ---- passes until a simulation ends.  (A loop of its own: in the one
+    // above, the engine's registers were copied on its several ways round,
+    // 40 moves and a wait for the next sample time per pass.  One call of each
+    // function: the code of a step and of the saved-state record exists once.)
+    const bool ran = mode != MODE_DONE;
+    do {
+      // (only tau-leaping decides: a compile-time fact in network kernels)
+      if (jr.method() == 0 && wave_any(mode == MODE_DECIDE)) {
+        const int next = eng.decide(jr, cnt, mode == MODE_DECIDE, g);
+        mode = mode == MODE_DECIDE ? next : mode;
+      }
       // SSA steps of the lanes inside a burst: more of them the more lanes are
       // in one than deciding (a burst of 100 steps taken 8 at a time waits
-      // through 13 decisions of the others)
-      const unsigned long long ssa = __builtin_amdgcn_ballot_w64(mode == MODE_SSA);
+      // through 13 decisions of the others); most if no lane decides (pure SSA,
+      // or every live lane inside a burst)
+      const bool burst = mode == MODE_SSA && eng.F < f_stop;
+      const unsigned long long ssa = __builtin_amdgcn_ballot_w64(burst);
       if (ssa != 0ull) {
         const int n_ssa = __builtin_popcountll(ssa);
         const int n_dec = __builtin_popcountll(__builtin_amdgcn_ballot_w64(mode == MODE_DECIDE));
         const int times = n_ssa >= 8 * n_dec ? 8 : n_ssa >= 4 * n_dec ? 4 : n_ssa >= 2 * n_dec ? 2 : 1;
-        mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, times * (jr.p().ssa_slice + 1), f_stop, t_stop, g);
+        mode = ssa_slice(jr, eng, cnt, mode, burst, times * (jr.p().ssa_slice + 1), t_stop, g);
       }
-    } else {
-      // no lane decides (pure SSA, or every live lane inside a burst): up to
-      // 8 (1 + ssa_slice) SSA steps before the next refill
-      mode = ssa_slice<GROUP>(jr, eng, sim, cnt, ev_start, mode, 8 * (jr.p().ssa_slice + 1), f_stop, t_stop, g);
-    }
+    } while (!wave_any(ran & ((mode == MODE_DONE) | (eng.F >= f_stop))));
+    if (ran) mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
   }
 
-  add_stats(cnt, g, lane, stats);
+  add_stats(cnt, g);
+  leave_stats(lane, stats);
 }
 
 // ---------------------------------------------------------------------------
@@ -580,7 +698,6 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
 // its partner except while it has nothing to run, and it leaves once the
 // partner has finished every job (DONE flag), when no slot can be SENT.
 // ---------------------------------------------------------------------------
-enum { MODE_AWAY = 3 };
 enum { SLOT_FREE = 0u, SLOT_SENT = 1u, SLOT_BACK = 2u };
 constexpr int PAIR_SLOTS = 256;  // decide lanes per workgroup
 constexpr int BURST_SLICE = 8;   // SSA steps of a burst wavefront between two looks at its slots
@@ -592,50 +709,15 @@ __device__ __forceinline__ void lds_store_release(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// A simulation in transit: the engine state, its id, its events so far
-// (for the flagged-events counter), the job index and the next mode.
-template <class Engine>
-struct SlotIO {
-  static constexpr int EW = (int)(sizeof(Engine) / 4);
-  static constexpr int WORDS = EW + 6;
-  static_assert(sizeof(Engine) % 4 == 0, "engine state is not whole words");
-  // word-major [word][slot]: consecutive lanes hit consecutive banks
-  static __device__ __forceinline__ void put(uint32_t* data, int slot, const Engine& eng, int64_t sim,
-                                             unsigned long long ev, int job, int mode) {
-    uint32_t w[EW];
-    __builtin_memcpy(w, &eng, sizeof(Engine));
-#pragma unroll
-    for (int i = 0; i < EW; ++i) data[i * PAIR_SLOTS + slot] = w[i];
-    data[(EW + 0) * PAIR_SLOTS + slot] = (uint32_t)sim;
-    data[(EW + 1) * PAIR_SLOTS + slot] = (uint32_t)((uint64_t)sim >> 32);
-    data[(EW + 2) * PAIR_SLOTS + slot] = (uint32_t)ev;
-    data[(EW + 3) * PAIR_SLOTS + slot] = (uint32_t)(ev >> 32);
-    data[(EW + 4) * PAIR_SLOTS + slot] = (uint32_t)job;
-    data[(EW + 5) * PAIR_SLOTS + slot] = (uint32_t)mode;
-  }
-  static __device__ __forceinline__ void get(const uint32_t* data, int slot, Engine& eng, int64_t& sim,
-                                             unsigned long long& ev, int& mode) {
-    uint32_t w[EW];
-#pragma unroll
-    for (int i = 0; i < EW; ++i) w[i] = data[i * PAIR_SLOTS + slot];
-    __builtin_memcpy(&eng, w, sizeof(Engine));
-    sim = (int64_t)(((uint64_t)data[(EW + 1) * PAIR_SLOTS + slot] << 32) | data[(EW + 0) * PAIR_SLOTS + slot]);
-    ev = ((unsigned long long)data[(EW + 3) * PAIR_SLOTS + slot] << 32) | data[(EW + 2) * PAIR_SLOTS + slot];
-    mode = (int)data[(EW + 5) * PAIR_SLOTS + slot];
-  }
-  static __device__ __forceinline__ int job(const uint32_t* data, int slot) {
-    return (int)data[(EW + 4) * PAIR_SLOTS + slot];
-  }
-};
-
-template <class Engine, class Ref, bool GROUP>
+template <class Engine, class Ref, int FORM>
 __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __restrict__ jobs, int n_jobs,
                                                   unsigned int* __restrict__ queue,
                                                   unsigned long long* __restrict__ stats, int f_end, int resume) {
-  using IO = SlotIO<Engine>;
+  using IO = SlotIO<Engine, PAIR_SLOTS>;
   __shared__ uint32_t s_data[IO::WORDS * PAIR_SLOTS];
   __shared__ uint32_t s_state[PAIR_SLOTS];
   __shared__ uint32_t s_done[4];
+  __shared__ uint32_t s_lanes[4];  // simulations per wavefront of the pair (64 / G)
   const int tid = (int)threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;  // wave-uniform
@@ -643,6 +725,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
   const int slot = pair * 64 + lane;
   if (tid < PAIR_SLOTS) s_state[tid] = SLOT_FREE;
   if (tid < 4) s_done[tid] = 0u;
+  init_stats();
   __syncthreads();  // the only barrier: every lane of the workgroup reaches it
 
   Counters cnt = {};
@@ -650,7 +733,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
   int64_t sim = -1;
   unsigned long long ev_start = 0;  // cnt.events when this lane's simulation began (here)
   Ref jr;
-  LaneGroup<GROUP> g;
+  LaneGroup<FORM> g;
   g.set(lane, 1);
 
   if (wave < 4) {
@@ -660,7 +743,8 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     bool exhausted = false;
     jr.load(jobs);
     int f_stop = range_stop(jr, f_end);
-    g.set(lane, jr.p().lanes);
+    g.set(lane, jr.cold().lanes);
+    if (lane == 0) s_lanes[pair] = (uint32_t)(64 / g.G);
     for (;;) {
       // a burst handed back (ended simulations were recorded by the burst
       // lane); the lanes of a group take it together
@@ -669,9 +753,8 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         IO::get(s_data, slot, eng, sim, ev, mode);
         ev_start = cnt.events - ev;
         s_state[slot] = SLOT_FREE;
-        if (mode != MODE_DONE) mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop);
       }
-      const bool want = (mode == MODE_DONE) && !exhausted && (GROUP || lane < jr.p().lanes);
+      const bool want = (mode == MODE_DONE) && !exhausted && (FORM != ONE || lane < jr.cold().lanes);
       const unsigned long long wmask = __builtin_amdgcn_ballot_w64(want & g.lead());
       if (wmask != 0ull) {
         const int n = __builtin_popcountll(wmask);
@@ -679,7 +762,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         unsigned int base = 0;
         if (lane == leader) base = atomicAdd(&queue[job], (unsigned int)n);
         base = __shfl(base, leader, 64);
-        const int n_sims = jr.p().n_sims;
+        const int n_sims = jr.cold().n_sims;
         if ((int64_t)base + n >= (int64_t)n_sims) exhausted = true;
         if (want) {
           const int rank = __builtin_popcountll(wmask & ((1ull << g.base) - 1ull));
@@ -690,22 +773,42 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
           }
         }
       }
+      // regroup when no simulation is away (its slot belongs to its lane): bursts
+      // that start meanwhile wait
+      bool hold = false;
+      if (FORM == WIDENING && exhausted) {
+        const int G = wider_group(g, __builtin_amdgcn_ballot_w64((mode != MODE_DONE) & g.lead()), group_cap(jr.n_reactions()));
+        hold = G != 0 && wave_any(mode == MODE_AWAY);
+        if (G != 0 && !hold) {
+          regroup<Engine, PAIR_SLOTS>(s_data, pair * 64, G, g, lane, eng, sim, ev_start, cnt, mode,
+                                      jr.p().layout == LAYOUT_BLOCKS);
+          if (lane == 0) s_lanes[pair] = (uint32_t)(64 / G);
+        }
+      }
       if (!wave_any(mode != MODE_DONE)) {
         job += 1;
         if (job >= n_jobs) break;
+        add_stats(cnt, g);
         jr.load(jobs + job);
         f_stop = range_stop(jr, f_end);
-        g.set(lane, jr.p().lanes);
+        g.set(lane, jr.cold().lanes);
+        if (lane == 0) s_lanes[pair] = (uint32_t)(64 / g.G);
         exhausted = false;
         continue;
       }
-      if (wave_any(mode == MODE_DECIDE)) {
-            mode = decide_pass<GROUP>(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
-      } else if (!wave_any(mode == MODE_SSA)) {
-        __builtin_amdgcn_s_sleep(2);  // every live lane is away: wait for a burst to come back
+      const bool ran = (mode == MODE_DECIDE) | (mode == MODE_SSA);
+      const bool on = mode == MODE_DECIDE && eng.F < f_stop;
+      if (wave_any(on)) {
+        const int next = eng.decide(jr, cnt, on, g);
+        mode = on ? next : mode;
+      } else if (hold || !wave_any(mode == MODE_SSA)) {
+        __builtin_amdgcn_s_sleep(2);  // every live lane is away or held: wait for a burst to come back
+      }
+      if (wave_any(ran & ((mode == MODE_DONE) | (eng.F >= f_stop)))) {
+        if (ran) mode = settle(jr, eng, sim, cnt, ev_start, mode, f_stop, g);
       }
       // a burst starts (or a forced-SSA simulation starts): hand it over
-      if (mode == MODE_SSA) {
+      if (mode == MODE_SSA && !hold) {
         IO::put(s_data, slot, eng, sim, cnt.events - ev_start, job, MODE_SSA);
         lds_store_release(&s_state[slot], SLOT_SENT);
         mode = MODE_AWAY;
@@ -733,7 +836,13 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
           bjob = pj;
           f_stop = range_stop(jr, f_end);
           t_stop = stop_time(jr, f_stop);
-          g.set(lane, jr.p().lanes);
+        }
+        // ... and hold its present group size (it changes only while this
+        // wavefront has nothing in hand)
+        const int sims = (int)s_lanes[pair];
+        if (64 / g.G != sims) {
+          add_stats(cnt, g);
+          g.set(lane, sims);
         }
       }
       const bool pick = g.all(sent);
@@ -752,13 +861,9 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         __builtin_amdgcn_s_sleep(4);
         continue;
       }
-      bool general;
-      int m = ssa_run<GROUP>(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, general, g);
-      if (wave_any(general)) {
-            if (general) m = eng.ssa_step(jr, cnt);
-      }
+      int m = ssa_slice(jr, eng, cnt, (int)MODE_SSA, busy, BURST_SLICE, t_stop, g);
       if (busy) {
-        if (m == MODE_DONE) m = settle(jr, eng, sim, cnt, ev_start, m, f_stop);
+        if (m == MODE_DONE) m = settle(jr, eng, sim, cnt, ev_start, m, f_stop, g);
         // back to the decide lane at the burst's end, or at the range's
         // last sample (the decide lane saves it)
         if (m != MODE_SSA || eng.F >= f_stop) {
@@ -770,7 +875,8 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     }
   }
 
-  add_stats(cnt, g, lane, stats);
+  add_stats(cnt, g);
+  leave_stats(lane, stats);
 }
 
 }  // namespace pst

@@ -153,8 +153,7 @@ struct EngineF32 {
   // of the sampler: one copy per reaction came to 320 KB of code for 16 x 16.
   static constexpr bool kWorklist = Ref::kTable && MP > 4;
   // blocks generated beside the decision (the one-by-one draws generate theirs)
-  template <bool GROUP>
-  static constexpr int ahead() { return (GROUP || kWorklist) && NB > 1 ? 1 : NB; }
+  static constexpr int NA = kWorklist ? 1 : NB;
   float k[Ref::kKP];  // rates row: per-reaction constants, or hazard parameters
   int32_t x[NP];
   Key key;
@@ -192,7 +191,7 @@ struct EngineF32 {
   }
 
   __device__ __forceinline__ int start(const Ref& jr, int64_t sim) {
-    const auto& P = jr.p();
+    const JobParams& P = jr.cold();
     const int64_t set = sim / P.sims_per_set;
 #pragma unroll
     for (int j = 0; j < Ref::kKP; ++j) k[j] = (j < P.n_rates) ? (float)glb(P.rates)[set * P.n_rates + j] : 0.0f;
@@ -207,7 +206,7 @@ struct EngineF32 {
     burst = 0;
     nsteps = 0;
     Ob = Out::base(P, sim);
-    return P.method == 0 ? MODE_DECIDE : MODE_SSA;
+    return jr.p().method == 0 ? MODE_DECIDE : MODE_SSA;
   }
 
   // One direct-method SSA step in its general form -- see EngineF64::ssa_step;
@@ -305,8 +304,8 @@ struct EngineF32 {
 
   // One P1_P2 body (P1_P2.py:96-294) of the lanes with `on` -- see
   // EngineF64::decide.
-  template <bool GROUP>
-  __device__ __forceinline__ int decide(Ref& tab, Counters& cnt, bool on, const LaneGroup<GROUP>& g) {
+  template <int FORM>
+  __device__ __forceinline__ int decide(Ref& tab, Counters& cnt, bool on, const LaneGroup<FORM>& g) {
     const auto& P = tab.p();
     constexpr int ABSORBED = -1;
     int end = 0;  // ABSORBED, or the flag that ends the simulation
@@ -320,10 +319,12 @@ struct EngineF32 {
     // the decision's.  The first Poisson attempt takes the NB blocks from bc,
     // or those from bc + 1 when the critical draw took block bc.
     const Key uk = key.scalar_seed(P.seed);
-    constexpr int NA = ahead<GROUP>();
     Words4 B[NB];
+    B[0] = uk.block(bc, 0);
+    if (NA > 1 && !g.grouped()) {
 #pragma unroll
-    for (int r = 0; r < NA; ++r) B[r] = uk.block(bc + (uint64_t)r, 0);
+      for (int r = 1; r < NA; ++r) B[r] = uk.block(bc + (uint64_t)r, 0);
+    }
     float a[MP];
     tab.template props<float>(x, k, a);
     float a0 = 0.0f;
@@ -389,7 +390,7 @@ struct EngineF32 {
     unsigned long long ev = 0;
     bool again = live;
     for (int h = 0;; ++h) {
-      const int st = attempt<GROUP>(tab, cnt, again, a, crit, tau, sel, B, xn, ev, uk, g);
+      const int st = attempt(tab, cnt, again, a, crit, tau, sel, B, xn, ev, uk, g);
       end = (again & (st > 0)) ? st : end;
       again = again & (st < 0);
       if (!wave_any(again)) break;
@@ -477,11 +478,11 @@ struct EngineF32 {
   // exact FP64 decisions near integer boundaries (both are inversions, so no
   // draw is rejected and repeated); lambda >= 2^16 by PTRS on blocks of its own
   // (ptrs_wide).
-  template <bool GROUP>
+  template <int FORM>
   __device__ __forceinline__ int attempt(Ref& tab, Counters& cnt, bool on, const float (&a)[MP],
                                          unsigned crit, float tau, int sel, const Words4 (&W)[NB],
                                          int32_t (&xn)[NP], unsigned long long& ev, const Key& uk,
-                                         const LaneGroup<GROUP>& g) {
+                                         const LaneGroup<FORM>& g) {
     const auto& P = tab.p();
     const int M = P.M;
     const uint64_t grp = bc;
@@ -495,7 +496,7 @@ struct EngineF32 {
       K[j] = (sel == j) ? 1 : 0;
       bad = bad | (lam[j] >= (float)LAMBDA_LIMIT);
     }
-    if constexpr (GROUP || kWorklist) {
+    if (kWorklist || g.grouped()) {
       // the lane's own reactions, one after the other
       unsigned todo = 0;
 #pragma unroll
@@ -514,9 +515,11 @@ struct EngineF32 {
         for (int r = 0; r < MP; ++r) K[r] = (has & (r == j)) ? kk : K[r];
         todo = todo & (todo - 1u);
       }
+      if (g.grouped()) {
 #pragma unroll
-      for (int j = 0; j < MP; ++j) K[j] = g.owners(K[j], j);
-      fail = g.any(fail);
+        for (int j = 0; j < MP; ++j) K[j] = g.owners(K[j], j);
+        fail = g.any(fail);
+      }
     } else {
       float u[MP];
 #pragma unroll
@@ -560,7 +563,7 @@ struct EngineF32 {
       cnt.w.draws += asym ? 1u : 0u;
       const bool exact = asym & ex;
       if (wave_any(exact)) {
-        cnt.w.exact += exact ? 1u : 0u;
+        if (exact) add_stat(ST_EXACT, 1ull);
         if (exact) kk = poisson_exact_f64((double)l, (double)u, m);
       }
     }
@@ -589,7 +592,7 @@ struct EngineF32 {
     if (wave_any(wide)) {
       if (wide) {
         const Draw dr = ptrs_wide(key.k0, key.k1, key.s_lo, key.s_hi, c, slot, l);
-        cnt.w.ptrs += dr.iters;
+        add_stat(ST_PTRS, dr.iters);
         cnt.w.draws += 2 * dr.iters;
         fail = fail | (dr.k < 0);
         kk = (int32_t)dr.k;
@@ -598,7 +601,7 @@ struct EngineF32 {
     return kk;
   }
 
-  // Every reaction's draw by the simulation's own lane.
+  // Every reaction's draw by the simulation's own lane (G = 1).
   __device__ __forceinline__ void draw_all(Counters& cnt, bool bad, const float (&lam)[MP], const float (&u)[MP],
                                            uint64_t grp, int32_t (&K)[MP], bool& fail) const {
     unsigned inv = 0, exact = 0, wide = 0, nasym = 0;
@@ -622,7 +625,7 @@ struct EngineF32 {
     cnt.w.draws += nasym;
     // near an integer boundary, or in a far tail: decide exactly in FP64
     if (wave_any(exact != 0u)) {
-      cnt.w.exact += (unsigned int)__builtin_popcount(exact);
+      if (exact != 0u) add_stat(ST_EXACT, (unsigned long long)__builtin_popcount(exact));
 #pragma unroll
       for (int j = 0; j < MP; ++j)
         if ((exact >> j) & 1u) K[j] = poisson_exact_f64((double)lam[j], (double)u[j], mb[j]);
@@ -677,7 +680,7 @@ struct EngineF32 {
       for (int j = 0; j < MP; ++j) {
         if ((wide >> j) & 1u) {
           const Draw dr = ptrs_wide(key.k0, key.k1, key.s_lo, key.s_hi, grp + (uint64_t)(j >> 2), j & 3, lam[j]);
-          cnt.w.ptrs += dr.iters;
+          add_stat(ST_PTRS, dr.iters);
           cnt.w.draws += 2 * dr.iters;
           fail = fail | (dr.k < 0);
           K[j] = (int32_t)dr.k;

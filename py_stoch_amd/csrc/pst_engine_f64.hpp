@@ -123,7 +123,7 @@ struct EngineF64 {
   }
 
   __device__ __forceinline__ int start(const Ref& jr, int64_t sim) {
-    const auto& P = jr.p();
+    const JobParams& P = jr.cold();
     const int64_t set = sim / P.sims_per_set;
 #pragma unroll
     for (int j = 0; j < Ref::kKP; ++j) k[j] = (j < P.n_rates) ? glb(P.rates)[set * P.n_rates + j] : 0.0;
@@ -138,7 +138,7 @@ struct EngineF64 {
     burst = 0;
     nsteps = 0;
     Ob = Out::base(P, sim);
-    return P.method == 0 ? MODE_DECIDE : MODE_SSA;
+    return jr.p().method == 0 ? MODE_DECIDE : MODE_SSA;
   }
 
   // One direct-method SSA step (P3.py:73-149; gillespie.py:70-149 for pure
@@ -242,8 +242,8 @@ struct EngineF64 {
   // Rare outcomes (budget, absorbing state, flags) are collected in `end` and
   // handled once at the end instead of where they arise: each branch on a lane
   // mask costs 50-60 cycles of a step's chain.
-  template <bool GROUP>
-  __device__ __forceinline__ int decide(Ref& tab, Counters& cnt, bool on, const LaneGroup<GROUP>& g) {
+  template <int FORM>
+  __device__ __forceinline__ int decide(Ref& tab, Counters& cnt, bool on, const LaneGroup<FORM>& g) {
     const auto& P = tab.p();
     const int M = P.M;
     constexpr int ABSORBED = -1;
@@ -310,7 +310,7 @@ struct EngineF64 {
     unsigned long long ev = 0;
     bool again = live;
     for (int h = 0;; ++h) {
-      const int st = attempt<GROUP>(tab, cnt, again, a, crit, tau, sel, xn, ev, g);
+      const int st = attempt(tab, cnt, again, a, crit, tau, sel, xn, ev, g);
       end = (again & (st > 0)) ? st : end;
       again = again & (st < 0);
       if (!wave_any(again)) break;
@@ -418,10 +418,10 @@ struct EngineF64 {
   // others go on to their next reaction, and the sampler's code exists once.
   // (One inlined sampler per reaction and a retry loop after them came to 58
   // KB of code for Lotka-Volterra, about the instruction cache.)
-  template <bool GROUP>
+  template <int FORM>
   __device__ __forceinline__ int attempt(Ref& tab, Counters& cnt, bool on, const double (&a)[MP],
                                          unsigned crit, double tau, int sel, int32_t (&xn)[NP],
-                                         unsigned long long& ev, const LaneGroup<GROUP>& g) {
+                                         unsigned long long& ev, const LaneGroup<FORM>& g) {
     const auto& P = tab.p();
     const int M = P.M;
     const uint64_t grp = bc;
@@ -484,7 +484,7 @@ struct EngineF64 {
       fail = fail | ((todo != 0u) & (it >= (uint32_t)PTRS_MAX_ITERS));
       todo = fail ? 0u : acc ? todo & (todo - 1u) : todo;
     }
-    if constexpr (GROUP) {
+    if (g.grouped()) {
 #pragma unroll
       for (int j = 0; j < MP; ++j) K[j] = g.owners(K[j], j);
       fail = g.any(fail);

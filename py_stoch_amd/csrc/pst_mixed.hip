@@ -3,40 +3,40 @@
 
 namespace pst {
 
-// GROUP: a group of lanes per simulation (fewer than 64 simulations per wavefront)
-template <int NP, int MP, bool GROUP>
+template <int NP, int MP, int FORM>
 __global__ void __launch_bounds__(256) sim_mixed_kernel(const JobDev<NP, MP>* __restrict__ jobs, int n_jobs,
                                                         unsigned int* __restrict__ queue,
                                                         unsigned long long* __restrict__ stats, Range range) {
-  run_driver<EngineF32<JobRef<NP, MP>>, JobRef<NP, MP>, GROUP>(jobs, n_jobs, queue, stats, range.f_end, range.resume);
+  run_driver<EngineF32<JobRef<NP, MP>>, JobRef<NP, MP>, FORM>(jobs, n_jobs, queue, stats, range.f_end, range.resume);
 }
 
-template <int NP, int MP, bool GROUP>
+template <int NP, int MP, int FORM>
 static int launch_cls_m(const void* jobs, int n_jobs, unsigned int* queue, unsigned long long* stats, int waves, Range range,
                         hipStream_t stream) {
   const int block = 256;
   const int grid = (waves + 3) / 4;
   if (grid <= 0) return 0;
-  hipLaunchKernelGGL((sim_mixed_kernel<NP, MP, GROUP>), dim3(grid), dim3(block), 0, stream,
+  hipLaunchKernelGGL((sim_mixed_kernel<NP, MP, FORM>), dim3(grid), dim3(block), 0, stream,
                      (const JobDev<NP, MP>*)jobs, n_jobs, queue, stats, range);
   return (int)hipGetLastError();
 }
 
-template <int NP, int MP, bool GROUP>
+template <int NP, int MP, int FORM>
 static int occupancy_cls_m() {
   int blocks = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, sim_mixed_kernel<NP, MP, GROUP>, 256, 0) != hipSuccess) return 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, sim_mixed_kernel<NP, MP, FORM>, 256, 0) != hipSuccess) return 1;
   return blocks > 0 ? blocks : 1;
 }
 
 int launch_mixed(int cls, const void* jobs, int n_jobs, unsigned int* queue, unsigned long long* stats, int waves,
                  Range range, bool group, hipStream_t stream) {
-  switch (table_form(cls, group)) {
-    case 0: return launch_cls_m<4, 4, false>(jobs, n_jobs, queue, stats, waves, range, stream);
-    case 1: return launch_cls_m<4, 4, true>(jobs, n_jobs, queue, stats, waves, range, stream);
-    case 2: return launch_cls_m<8, 8, false>(jobs, n_jobs, queue, stats, waves, range, stream);
-    case 3: return launch_cls_m<8, 8, true>(jobs, n_jobs, queue, stats, waves, range, stream);
-    case 4: return launch_cls_m<16, 16, false>(jobs, n_jobs, queue, stats, waves, range, stream);
+  switch (2 * cls + (group ? 1 : 0)) {
+    case 0: return launch_cls_m<4, 4, ONE>(jobs, n_jobs, queue, stats, waves, range, stream);
+    case 1: return launch_cls_m<4, 4, GROUPED>(jobs, n_jobs, queue, stats, waves, range, stream);
+    case 2: return launch_cls_m<8, 8, ONE>(jobs, n_jobs, queue, stats, waves, range, stream);
+    case 3: return launch_cls_m<8, 8, GROUPED>(jobs, n_jobs, queue, stats, waves, range, stream);
+    case 4: return launch_cls_m<16, 16, ONE>(jobs, n_jobs, queue, stats, waves, range, stream);
+    case 5: return launch_cls_m<16, 16, GROUPED>(jobs, n_jobs, queue, stats, waves, range, stream);
     default: return -1;
   }
 }
@@ -93,12 +93,13 @@ int launch_poisson_probe(const float* lam, const uint32_t* words, int64_t n, int
 }
 
 int blocks_per_cu_mixed(int cls, bool group) {
-  switch (table_form(cls, group)) {
-    case 0: return occupancy_cls_m<4, 4, false>();
-    case 1: return occupancy_cls_m<4, 4, true>();
-    case 2: return occupancy_cls_m<8, 8, false>();
-    case 3: return occupancy_cls_m<8, 8, true>();
-    case 4: return occupancy_cls_m<16, 16, false>();
+  switch (2 * cls + (group ? 1 : 0)) {
+    case 0: return occupancy_cls_m<4, 4, ONE>();
+    case 1: return occupancy_cls_m<4, 4, GROUPED>();
+    case 2: return occupancy_cls_m<8, 8, ONE>();
+    case 3: return occupancy_cls_m<8, 8, GROUPED>();
+    case 4: return occupancy_cls_m<16, 16, ONE>();
+    case 5: return occupancy_cls_m<16, 16, GROUPED>();
     default: return 1;
   }
 }

@@ -29,7 +29,7 @@ const char* const kOptsFp64[] = {"--offload-arch=gfx950", "-O3", "-std=c++17",
                                  "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                                  "-ffp-contract=off"};
 
-const char* const kSuffix[] = {"", "_paired", "_group", "_paired_group"};  // kernel name suffix per RtcForm
+const char* const kSuffix[] = {"", "_group", "_paired", "_paired_group"};  // kernel name suffix per RtcForm
 
 void arr(std::string& s, const char* name, const int8_t* v, int n) {
   s += "  static constexpr int8_t ";
@@ -136,8 +136,7 @@ int compile(const std::string& source, int precision, std::vector<char>* code, s
 
 std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
                        const std::vector<std::string>& hazards, int waves_per_eu, RtcForm form) {
-  const bool paired = form == RTC_PAIRED || form == RTC_PAIRED_GROUP;
-  const bool group = form == RTC_GROUP || form == RTC_PAIRED_GROUP;
+  const bool paired = form >= RTC_PAIRED, group = form == RTC_GROUP || form == RTC_PAIRED_GROUP;
   const int N = net.N, M = net.M;
   std::vector<int8_t> v(N * M), ord(N * M), stp(N * M), E(N, 0);
   for (int i = 0; i < N * M; ++i) {
@@ -178,13 +177,22 @@ std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
   s += std::string("#define PST_KERNEL_NAME ") + (precision == PST_PRECISION_FP64 ? "pst_net_fp64" : "pst_net_mixed") +
        kSuffix[form] + "\n";
   s += paired ? "extern \"C\" __global__ void __launch_bounds__(512)" : "extern \"C\" __global__ void __launch_bounds__(256)";
+  // A paired workgroup has two wavefronts on each SIMD: 256 registers at most,
+  // or the hardware refuses the launch.
+  if (waves_per_eu == 0 && paired) waves_per_eu = 2;
   if (waves_per_eu > 0) s += " __attribute__((amdgpu_waves_per_eu(" + std::to_string(waves_per_eu) + ")))";
   s += "\n"
        "PST_KERNEL_NAME(const pst::JobParams* __restrict__ jobs, int n_jobs, unsigned int* __restrict__ queue,\n"
        "                 unsigned long long* __restrict__ stats, pst::Range range) {\n";
+  // One simulation per lane: the last ones of a wavefront share its lanes
+  // (WIDENING) where that pays: FP64 tau-leaping (Lotka-Volterra, 65,536
+  // simulations, 93 -> 86 ms) and the SSA methods (Schloegl SSA FP64, 100,003:
+  // 40.2 -> 36.4 ms); the mixed leap's draws are cheap next to what the two ways
+  // of drawing in one kernel cost (34.4 -> 35.2 ms).
+  const bool widening = c.method != 0 || (precision == PST_PRECISION_FP64 && !group);
   s += std::string("  pst::") + (paired ? "run_driver_paired" : "run_driver") +
-       "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>" +
-       (group ? ", true" : ", false") + ">(jobs, n_jobs, queue, stats, "
+       "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>, pst::" +
+       (widening ? "WIDENING" : group ? "GROUPED" : "ONE") + ">(jobs, n_jobs, queue, stats, "
        "range.f_end, range.resume);\n}\n";
   return s;
 }
@@ -243,10 +251,21 @@ int rtc_kernel(const std::string& source, int precision, RtcKernel* out, std::st
     *err = std::string("hipModuleGetFunction: ") + hipGetErrorString(e);
     return PST_EHIP;
   }
-  k.block = (form == RTC_PAIRED || form == RTC_PAIRED_GROUP) ? 512 : 256;
+  k.block = form >= RTC_PAIRED ? 512 : 256;
   int blocks = 0;
-  if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k.fn, k.block, 0) == hipSuccess && blocks > 0)
-    k.blocks_per_cu = blocks;
+  if ((e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k.fn, k.block, 0)) != hipSuccess) {
+    *err = std::string("occupancy of the network kernel: ") + hipGetErrorString(e);
+    return PST_EHIP;
+  }
+  int regs = 0, lds = 0;
+  (void)hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, k.fn);
+  (void)hipFuncGetAttribute(&lds, HIP_FUNC_ATTRIBUTE_SHARED_SIZE_BYTES, k.fn);
+  if (blocks < 1) {
+    *err = "the network kernel's workgroup of " + std::to_string(k.block) + " lanes does not fit a compute unit (" +
+           std::to_string(regs) + " registers per lane, " + std::to_string(lds) + " bytes of LDS)";
+    return PST_ETOOLARGE;
+  }
+  k.blocks_per_cu = blocks;
   g_cache.emplace(key, k);  // the module stays loaded for the life of the process
   *out = k;
   return PST_OK;

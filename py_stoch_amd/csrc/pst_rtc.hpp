@@ -36,11 +36,12 @@ struct RtcKernel {
 // C expression per reaction (X(i), C(k), R(v), see pst_network.hazards).
 // waves_per_eu > 0 asks the compiler for register use that fits that many
 // wavefronts per SIMD (the kernel's arithmetic, and so its results, do not
-// change).  RTC_PAIRED: the kernel runs run_driver_paired (workgroups of 512
-// lanes: four decide and four burst wavefronts), named pst_net_*_paired;
-// RTC_GROUP: run_driver with a group of lanes per simulation (fewer than 64
-// simulations per wavefront), named pst_net_*_group; RTC_PAIRED_GROUP: both.
-enum RtcForm { RTC_PLAIN = 0, RTC_PAIRED = 1, RTC_GROUP = 2, RTC_PAIRED_GROUP = 3 };
+// change).  Forms: RTC_PLAIN one simulation per lane, RTC_GROUP a group of
+// lanes per simulation (fewer than 64 simulations per wavefront), both in
+// run_driver; RTC_PAIRED and RTC_PAIRED_GROUP the same in run_driver_paired
+// (workgroups of 512 lanes: four decide and four burst wavefronts).  The kernel
+// is named pst_net_* with the suffix _group, _paired or _paired_group.
+enum RtcForm { RTC_PLAIN = 0, RTC_GROUP = 1, RTC_PAIRED = 2, RTC_PAIRED_GROUP = 3 };
 std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
                        const std::vector<std::string>& hazards, int waves_per_eu = 0, RtcForm form = RTC_PLAIN);
 

@@ -83,3 +83,30 @@ def test_group_size_changes_no_bit_in_mixed_precision(native, n_reactions, speci
         st.pop("kernel_ms")
         stats.append(st)
     assert stats[0] == stats[1] == stats[2]
+
+
+@pytest.mark.parametrize("method,burst_waves", [(0, 0), (0, 1), (2, 0)])
+@pytest.mark.parametrize("n_reactions", [3, 6])
+def test_lanes_shared_by_the_last_simulations(native, oracle_mod, n_reactions, method, burst_waves):
+    """One simulation per lane, more simulations than lanes on the chip for the
+    unpaired launch: wavefronts refill from the queue, then widen to groups of
+    four and eight lanes; the blocked layout carries a partial block along."""
+    n = 66003
+    a, tabs, rates, kw = _settings(n_reactions)
+    kw = dict(kw, n_sims=n, method=method, I=np.linspace(0, 0.4, 13).astype(np.float32), t_max=0.4)
+    Oc, Fc, sc = oracle_mod.simulate(tabs, rates, a.x_0, threads=16, **kw)
+    print("case: widening M=%d method=%d burst_waves=%d" % (n_reactions, method, burst_waves), flush=True)
+    plan = native.Plan(tabs, rates, a.x_0, precision=0, specialize=True, layout=native.LAYOUT_BLOCKS, **kw)
+    O, F = DeviceArray((2, 2, n, 8)), DeviceArray((n,))
+    try:
+        plan.set_launch(0, 7, 0, burst_waves)
+        plan.execute(O.ptr.value, n, F.ptr.value)
+        Og = O.get().transpose(0, 1, 3, 2).reshape(2, 16, n)
+        assert np.array_equal(Og[:, :13], Oc) and not Og[:, 13:].any() and np.array_equal(F.get(), Fc)
+        st = plan.stats()
+        for key in COUNTERS:
+            assert st[key] == sc[key], key
+    finally:
+        plan.close()
+        O.free()
+        F.free()
