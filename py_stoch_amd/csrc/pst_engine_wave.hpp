@@ -20,9 +20,10 @@
 //                        block (group + j, it) -- all draws of a leap in
 //                        parallel
 //   x' = x + V K         64-bit integer LDS atomics (order-independent)
-// State of the simulation (time, sample cursor, Philox counter, mode) is
-// wavefront-uniform.  Per wavefront LDS: x, x', propensities of non-critical
-// reactions and the critical flags (about 2 KB).
+// Ordinary SSA steps have a loop of their own (ssa_run).  State of the
+// simulation (time, sample cursor, Philox counter, mode) is wavefront-uniform.
+// Per wavefront LDS: x, x', propensities of non-critical reactions, the
+// critical flags and the net changes of every reaction (about 7 KB).
 #pragma once
 #include "pst_engine_f32.hpp"
 
@@ -34,6 +35,7 @@ constexpr int WAVE_R = WAVE_MAX_M / 64;  // reactions per lane
 constexpr int WAVE_MAX_REACT = 4;        // species with a propensity factor, per reaction
 constexpr int WAVE_MAX_V = 8;            // non-zero V entries per reaction
 constexpr int WAVE_MAX_T = 2048;         // non-zero V entries in total
+constexpr int WAVE_MAX_F = 4;            // propensity factors of a reaction in ssa_run
 
 // Network of one job in sparse form (built by the host library).
 struct WaveTab {
@@ -49,6 +51,13 @@ struct WaveTab {
   uint16_t tstart[WAVE_MAX_N + 1];         // column of V of species i: entries tstart[i] .. tstart[i+1]-1
   uint16_t tj[WAVE_MAX_T];                 // reaction of the entry
   int8_t tv[WAVE_MAX_T];                   // value of the entry
+  // the same for ssa_run: propensity factors (x_s - sub) one by one, a byte
+  // each (species | sub << 6), and how many; net changes as (species, value)
+  // byte pairs, species 255 past the last
+  uint32_t fw[WAVE_MAX_M];
+  uint8_t fn[WAVE_MAX_M];
+  uint32_t vrow[WAVE_MAX_M][4];
+  int32_t max_f;                           // most factors of a reaction; above WAVE_MAX_F: no ssa_run
 };
 
 struct WaveJob {
@@ -62,6 +71,7 @@ struct WaveLds {
   float anc[WAVE_MAX_M];     // propensity of non-critical reactions, 0 for critical ones
   int32_t K[WAVE_MAX_M];     // firings of the current leap attempt
   uint8_t crit[WAVE_MAX_M];
+  uint32_t vrow[WAVE_MAX_M][4];  // WaveTab::vrow of the current job
 };
 
 // LDS writes of some lanes visible to reads of others in the same wavefront
@@ -75,15 +85,69 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// v + (v of lane l ^ OFF): one step of a sum over the wavefront in the order of
+// a butterfly from 32 down to 1.  Lane exchanges inside the vector unit
+// (v_permlane*_swap, DPP) instead of 57-cycle trips through LDS.  A swap of v
+// with itself leaves, in every lane, its own value in one result and its
+// partner's in the other.  Below 16 the values repeat with the period of the
+// step before, so a rotation of the row is the exchange.
+template <int OFF>
+__device__ __forceinline__ void lane_pair(uint32_t v, uint32_t& x, uint32_t& y) {
+  if constexpr (OFF == 32 || OFF == 16) {
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(v, v, false, false)
+                             : __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    x = r[0];
+    y = r[1];
+  } else {
+    constexpr int ctrl = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4e : 0xb1;  // row_ror:8, :4, quad_perm
+    x = v;
+    y = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, ctrl, 0xf, 0xf, true);
+  }
+}
+template <int OFF>
+__device__ __forceinline__ float add_xor(float v) {
+  uint32_t x, y;
+  lane_pair<OFF>(__builtin_bit_cast(uint32_t, v), x, y);
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+template <int OFF>
+__device__ __forceinline__ double add_xor(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  uint32_t xl, yl, xh, yh;
+  lane_pair<OFF>((uint32_t)b, xl, yl);
+  lane_pair<OFF>((uint32_t)(b >> 32), xh, yh);
+  return __builtin_bit_cast(double, ((uint64_t)xh << 32) | xl) + __builtin_bit_cast(double, ((uint64_t)yh << 32) | yl);
+}
+template <class T>
+__device__ __forceinline__ T butterfly_sum(T v) {
+  return add_xor<1>(add_xor<2>(add_xor<4>(add_xor<8>(add_xor<16>(add_xor<32>(v))))));
+}
+__device__ __forceinline__ float wave_sum_f(float v) { return butterfly_sum(v); }
+__device__ __forceinline__ double wave_sum_d(double v) { return butterfly_sum(v); }
+
+// inclusive prefix sum over lanes by DPP row shifts and row broadcasts (its
+// order of additions is not wave_scan_d's)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double fast_scan_d(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
   return v;
 }
-__device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+__device__ __forceinline__ double read_lane_d(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 __device__ __forceinline__ float wave_min_f(float v) {
 #pragma unroll
@@ -109,6 +173,7 @@ __device__ __forceinline__ double wave_scan_d(double v, int lane) {
 // members are wavefront-uniform except the per-lane rate constants.
 struct EngineWave {
   float k[WAVE_R];  // rates of the lane's reactions
+  uint32_t fw[WAVE_R], fn;  // WaveTab::fw and fn (a byte each) of the lane's reactions
 
   Key key;
   uint64_t bc;
@@ -143,6 +208,20 @@ struct EngineWave {
     }
   }
 
+  // the parts of a job's table that ssa_run keeps at hand
+  __device__ __forceinline__ void load(const WaveJob& J, WaveLds& L, int lane) {
+    fn = 0;
+#pragma unroll
+    for (int r = 0; r < WAVE_R; ++r) {
+      const int j = lane + 64 * r;
+      fw[r] = J.t.fw[j];
+      fn |= (uint32_t)J.t.fn[j] << (8 * r);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) L.vrow[j][w] = J.t.vrow[j][w];
+    }
+    wave_lds_sync();
+  }
+
   __device__ __forceinline__ void start(const WaveJob& J, WaveLds& L, int lane, int64_t s) {
     const JobParams& P = J.p;
     const int64_t set = s / P.sims_per_set;
@@ -165,6 +244,121 @@ struct EngineWave {
     mode = P.method == 0 ? MODE_DECIDE : MODE_SSA;
   }
 
+  // propensities of the lane's reactions from the compact factors
+  __device__ __forceinline__ void props(const WaveLds& L, int M, int max_f, float (&a)[WAVE_R]) const {
+#pragma unroll
+    for (int r = 0; r < WAVE_R; ++r) {
+      float v = 0.0f;
+      if (64 * r < M) {  // whole slots past M are skipped by the wavefront
+        v = k[r];
+        const int nf = (int)((fn >> (8 * r)) & 0xffu);
+#pragma unroll
+        for (int e = 0; e < WAVE_MAX_F; ++e) {
+          if (e < max_f) {
+            const uint32_t b = (fw[r] >> (8 * e)) & 0xffu;
+            const int32_t f = L.x[b & 63u] - (int32_t)(b >> 6);
+            v = v * (e < nf ? (float)f : 1.0f);
+          }
+        }
+      }
+      a[r] = v;
+    }
+  }
+
+  // The ordinary SSA steps of a burst (or of SSA methods) until one needs
+  // step(): the end of the simulation, the last sample, the count limit, a
+  // step budget, a stuck clock, or a reaction choice too close to call.  The
+  // arithmetic is step()'s except for the prefix sums, whose additions come
+  // in another order; both are within 1e-13 of the exact sums relative to
+  // asum, so outside a band of 1e-12 asum they choose the same reaction.
+  // What the loop needs per reaction is in registers (rates, factors) or LDS
+  // (counts, net changes): step() reads the table's bytes from memory, one
+  // dependent load after the other, ~19,000 cycles a step at four wavefronts per
+  // SIMD.  Lane l draws the numbers of step l of the next 64.  Pure SSA of
+  // three networks of 17-40 species, 300 simulations each: 20.5 -> 4.2 ms; 16
+  // random networks by tau-leaping (57 M SSA steps, 0.7 M leaps) 162 -> 50 ms.
+  __device__ __forceinline__ void ssa_run(const WaveJob& J, WaveLds& L, int lane, Counters& cnt) {
+    const JobParams& P = J.p;
+    const WaveTab& T = J.t;
+    const int M = P.M, N = P.N, max_f = T.max_f;
+    const double tstop = (double)glb(P.I)[P.ita - 1];
+    const double tend = P.method == 2 ? (P.t_max < tstop ? P.t_max : tstop) : tstop;
+    int32_t xl = lane < N ? L.x[lane] : 0;
+    float nl = 0.0f, u = 0.0f;
+    int left = 0;  // drawn numbers not used yet
+    uint32_t n = 0;
+    const uint32_t budget = P.max_steps != 0u ? (nsteps < P.max_steps ? P.max_steps - nsteps : 0u) : 0xffffffffu;
+    const uint32_t lim = P.method == 0 && (uint32_t)burst < budget ? (uint32_t)burst : budget;
+    while (n < lim) {
+      if (left == 0) {
+        const Words4 w = key.block(bc + (uint64_t)(n + (uint32_t)lane), 0);
+        nl = -fast_log(u24(w.w0));
+        u = u24(w.w1);
+        left = 64;
+      }
+      const float nl1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, nl), 64 - left));
+      const float u1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, u), 64 - left));
+      float a[WAVE_R];
+      props(L, M, max_f, a);
+      double ad = 0.0;
+#pragma unroll
+      for (int r = 0; r < WAVE_R; ++r) ad += (double)a[r];
+      const double asum = wave_sum_d(ad);
+      const double t1 = t + (double)(nl1 * fast_rcp((float)asum));
+      const double target = (double)u1 * asum;
+      const double band = 1e-12 * asum;
+      bool near = false;
+      int sel = -1;
+      double carry = 0.0;
+#pragma unroll
+      for (int r = 0; r < WAVE_R; ++r) {
+        if (64 * r < M) {
+          const double cum = fast_scan_d((double)a[r]) + carry;
+          carry = read_lane_d(cum, 63);
+          near = near | (__builtin_fabs(cum - target) <= band);
+          const unsigned long long hit = __builtin_amdgcn_ballot_w64(cum >= target);
+          sel = (sel < 0 && hit != 0ull) ? 64 * r + (int)__builtin_ctzll(hit) : sel;
+        }
+      }
+      // (asum = 0 gives an infinite or undefined time, which fails here)
+      const bool ok = (t1 > t) & (t1 < tend) & !near & (sel >= 0);
+      if (__builtin_amdgcn_ballot_w64(!ok) != 0ull) break;
+      const uint32_t* row = L.vrow[sel];
+      int32_t dx = 0;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const uint32_t e2 = row[w];
+        dx += (int)(e2 & 0xffu) == lane ? __builtin_amdgcn_sbfe((int)e2, 8, 8) : 0;
+        dx += (int)((e2 >> 16) & 0xffu) == lane ? __builtin_amdgcn_sbfe((int)e2, 24, 8) : 0;
+      }
+      const int32_t xn = xl + dx;
+      if (__builtin_amdgcn_ballot_w64(xn >= COUNT_LIMIT) != 0ull) break;
+      while (t1 >= tnext) {  // sample-and-hold: the state before the step
+        if (lane < P.kappa) glb(P.O)[out_index(P, lane, F)] = L.x[T.E[lane]];
+        if (lane == 0) cnt.w.samples += 1;
+        F = F + 1;
+        tnext = (double)glb(P.I)[F];
+      }
+      xl = xn;
+      if (lane < N) L.x[lane] = xl;
+      wave_lds_sync();
+      t = t1;
+      n += 1;
+      left -= 1;
+    }
+    bc += (uint64_t)n;
+    nsteps += n;
+    if (lane == 0) {
+      cnt.w.uniforms += 2u * n;
+      cnt.ssa += n;
+      cnt.events += (unsigned long long)n;
+    }
+    if (P.method == 0) {
+      burst -= (int)n;
+      if (burst <= 0) mode = MODE_DECIDE;
+    }
+  }
+
   // one step (leap decision + leap, or one SSA step); returns true when the
   // simulation has ended
   __device__ bool step(const WaveJob& J, WaveLds& L, int lane, Counters& cnt) {
@@ -184,20 +378,24 @@ struct EngineWave {
     nsteps += 1;
     // propensities of the lane's reactions
     float a[WAVE_R];
+    if (T.max_f <= WAVE_MAX_F) {
+      props(L, M, T.max_f, a);
+    } else {
 #pragma unroll
-    for (int r = 0; r < WAVE_R; ++r) {
-      const int j = lane + 64 * r;
-      float v = 0.0f;
-      if (64 * r < M && j < M) {  // whole slots past M are skipped by the wavefront
-        v = k[r];
-        const int nr = T.nr[j];
-        for (int e = 0; e < nr; ++e) {
-          const int xi = L.x[T.rs[j][e]];
-          const int p = T.ro[j][e], st = T.rst[j][e];
-          for (int q = 0; q < p; ++q) v = v * (float)(xi - st * q);
+      for (int r = 0; r < WAVE_R; ++r) {
+        const int j = lane + 64 * r;
+        float v = 0.0f;
+        if (64 * r < M && j < M) {  // whole slots past M are skipped by the wavefront
+          v = k[r];
+          const int nr = T.nr[j];
+          for (int e = 0; e < nr; ++e) {
+            const int xi = L.x[T.rs[j][e]];
+            const int p = T.ro[j][e], st = T.rst[j][e];
+            for (int q = 0; q < p; ++q) v = v * (float)(xi - st * q);
+          }
         }
+        a[r] = v;
       }
-      a[r] = v;
     }
     float a_lane = 0.0f;
     double ad_lane = 0.0;
@@ -223,10 +421,11 @@ struct EngineWave {
         const int j = lane + 64 * r;
         bool c = false;
         if (64 * r < M && j < M) {
-          const int nv = T.nv[j];
-          for (int e = 0; e < nv; ++e) {
-            const int v = T.vv[j][e];
-            if (v < 0) c = c || ((-v) * P.n_c > L.x[T.vs[j][e]]);
+#pragma unroll
+          for (int e = 0; e < WAVE_MAX_V; ++e) {
+            const uint32_t b = L.vrow[j][e / 2] >> (16 * (e % 2));
+            const int v = __builtin_amdgcn_sbfe((int)b, 8, 8);
+            if (v < 0) c = c || ((-v) * P.n_c > L.x[b & 63u]);
           }
           L.anc[j] = c ? 0.0f : a[r];
           L.crit[j] = c ? 1 : 0;
@@ -260,6 +459,7 @@ struct EngineWave {
         ssa = true;
         mode = MODE_SSA;
         burst = P.ssa_burst;
+        if (T.max_f <= WAVE_MAX_F) return false;  // its steps run in ssa_run
         if (P.max_steps != 0u && nsteps >= P.max_steps) {
           fill_rest(J, L, lane, true, cnt);
           flag = FLAG_STEPS;
@@ -391,7 +591,6 @@ struct EngineWave {
   // so the sampler's code (and its registers) exists once.
   __device__ int leap(const WaveJob& J, WaveLds& L, int lane, Counters& cnt, int sel, float& tau, long long& ev) {
     const JobParams& P = J.p;
-    const WaveTab& T = J.t;
     const int M = P.M, N = P.N;
     for (int h = 0; h < MAX_HALVINGS; ++h) {
       const uint64_t grp = bc;
@@ -457,9 +656,12 @@ struct EngineWave {
         const int32_t kk = L.K[j];
         if (kk != 0) {
           ev_lane += kk;
-          const int nv = T.nv[j];
-          for (int e = 0; e < nv; ++e)
-            atomicAdd((unsigned long long*)&L.xn[T.vs[j][e]], (unsigned long long)((long long)kk * T.vv[j][e]));
+          for (int e = 0; e < WAVE_MAX_V; ++e) {
+            const uint32_t b = L.vrow[j][e / 2] >> (16 * (e % 2));
+            const int v = __builtin_amdgcn_sbfe((int)b, 8, 8);
+            if (v == 0) break;  // past the last entry
+            atomicAdd((unsigned long long*)&L.xn[b & 63u], (unsigned long long)((long long)kk * v));
+          }
         }
       }
       wave_lds_sync();

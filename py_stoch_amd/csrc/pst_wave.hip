@@ -4,6 +4,7 @@
 // Every wavefront takes simulations one at a time from the job's work queue
 // (one atomic per simulation) and runs each to its end; jobs are visited in
 // order.  LDS holds the state of the wavefront's current simulation.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 
@@ -13,7 +14,7 @@ namespace pst {
 
 // Four wavefronts per SIMD: 128 VGPRs and ~400 bytes of scratch spill per lane
 // instead of 227 VGPRs at two, which hides more latency than the spills cost
-// (first 48 random networks: 1,508 -> 1,264 ms; three: 1,339 ms; five: 1,622 ms).
+// (16 random networks: 50.4 ms; three wavefronts 57.2, five 56.1).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 sim_wave_kernel(const WaveJob* __restrict__ jobs, int n_jobs, unsigned int* __restrict__ queue,
                 unsigned long long* __restrict__ stats) {
@@ -24,6 +25,8 @@ sim_wave_kernel(const WaveJob* __restrict__ jobs, int n_jobs, unsigned int* __re
   EngineWave eng;
   for (int job = 0; job < n_jobs; ++job) {
     const WaveJob& J = jobs[job];
+    eng.load(J, L, lane);
+    const bool fast = J.t.max_f <= WAVE_MAX_F;
     for (;;) {
       unsigned int s = 0;
       if (lane == 0) s = atomicAdd(&queue[job], 1u);
@@ -31,8 +34,9 @@ sim_wave_kernel(const WaveJob* __restrict__ jobs, int n_jobs, unsigned int* __re
       if ((int64_t)s >= (int64_t)J.p.n_sims) break;
       const unsigned long long ev_start = cnt.events;
       eng.start(J, L, lane, (int64_t)s);
-      while (!eng.step(J, L, lane, cnt)) {
-      }
+      do {
+        if (fast && eng.mode == MODE_SSA) eng.ssa_run(J, L, lane, cnt);
+      } while (!eng.step(J, L, lane, cnt));
       const int fl = __shfl(eng.flag, 0, 64);
       cnt.fevents += (fl != 0) ? cnt.events - ev_start : 0ull;  // summed over lanes below
       if (lane == 0) {
@@ -104,6 +108,21 @@ bool make_wave_tab(const HostNet& h, WaveTab* t, char* why, size_t why_len) {
     }
     t->nr[j] = (uint8_t)nr;
     t->nv[j] = (uint8_t)nv;
+    // the compact form of ssa_run
+    int nf = 0;
+    for (int e = 0; e < nr; ++e) {
+      for (int q = 0; q < t->ro[j][e]; ++q, ++nf) {
+        const int sub = t->rst[j][e] ? q : 0;
+        if (nf < WAVE_MAX_F && sub < 4) t->fw[j] |= (uint32_t)(t->rs[j][e] | (sub << 6)) << (8 * nf);
+        if (sub >= 4) nf = WAVE_MAX_F;  // beyond the format
+      }
+    }
+    t->fn[j] = (uint8_t)(nf < 255 ? nf : 255);
+    t->max_f = std::max(t->max_f, (int32_t)t->fn[j]);
+    for (int e = 0; e < WAVE_MAX_V; ++e) {
+      const uint32_t b = e < nv ? (uint32_t)t->vs[j][e] | ((uint32_t)(uint8_t)t->vv[j][e] << 8) : 0xffu;
+      t->vrow[j][e / 2] |= b << (16 * (e % 2));
+    }
   }
   int e = 0;
   for (int i = 0; i < N; ++i) {
