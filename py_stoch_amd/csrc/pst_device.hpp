@@ -328,15 +328,25 @@ __device__ __forceinline__ int32_t poisson_asym_f32(float lam, float u, bool& ex
 // N is m - 1 if P(X <= m - 1) >= u and m otherwise (the FP32 root is within
 // the band of m); the CDF is a sum of pmf terms from p(m - 1) downwards, or
 // 1 minus a sum from p(m) upwards above the mean, to 1e-17 of the sum.  With
-// m = -1 (lambda < 60, u in a far tail) a search from n = 0.
+// m = -1 (u in a far tail: lambda < 60, or u = 1.0 at any lambda) a search from
+// n = 0, 100,000 at most.  u24 is 1.0 once in 2^24 draws, above every value the
+// FP64 sum takes for most means: the search ends as soon as the sum has, there
+// with the 100,000 it would count up to -- that many divisions one after the
+// other, 8-11 ms in which the wavefront does nothing else and, being the last,
+// holds the launch.  The sum has ended where it starts from an underflowed
+// e^-lambda, and past the mode where p is below half an ulp of S and every
+// later p smaller.  Schloegl, 20,000 simulations, 19.4 -> 12.8 ms; Lotka-
+// Volterra, 65,536, 34.9 -> 30.6 ms; 10 reactions, 20,011, 12.3 -> 4.9 ms.
 __device__ __noinline__ int32_t poisson_exact_f64(double lam, double u, int32_t m) {
   if (m < 0) {
     double p = exp_f64(-lam), S = p;
+    if (S == 0.0) return 100000;
     int32_t k = 0;
     while (u > S && k < 100000) {
       k += 1;
       p = p * lam / (double)k;
       S += p;
+      if ((double)k > lam && p < S * 0x1p-54) return (u > S) ? 100000 : k;
     }
     return k;
   }
