@@ -337,6 +337,17 @@ __device__ __forceinline__ int32_t poisson_asym_f32(float lam, float u, bool& ex
 // e^-lambda, and past the mode where p is below half an ulp of S and every
 // later p smaller.  Schloegl, 20,000 simulations, 19.4 -> 12.8 ms; Lotka-
 // Volterra, 65,536, 34.9 -> 30.6 ms; 10 reactions, 20,011, 12.3 -> 4.9 ms.
+//
+// The term-by-term sums are a chain of one division per term over ~8 sqrt(lambda)
+// terms (0.1 ms at lambda = 50,000), so a sum of four terms per trip goes first:
+// it shares the first term, takes the ratios' products side by side, and stops
+// where u lies outside [sum, sum + geometric bound of the rest] by more than
+// POIS_SUM_MARGIN of the sum.  Both sums are within 65,536 terms x 3 x 2^-53 =
+// 2.2e-11 of the exact one, so the margin of 1e-10 makes the decision that of
+// the term-by-term sum; where u lies closer the latter runs as well.  10
+// reactions with means up to 10^4..10^5, 20,011 simulations: 4.64 -> 4.19 ms;
+// Lotka-Volterra, Schloegl (means of 10..1000) 0..0.5 % faster.
+constexpr double POIS_SUM_MARGIN = 1e-10;
 __device__ __noinline__ int32_t poisson_exact_f64(double lam, double u, int32_t m) {
   if (m < 0) {
     double p = exp_f64(-lam), S = p;
@@ -355,6 +366,18 @@ __device__ __noinline__ int32_t poisson_exact_f64(double lam, double u, int32_t 
   if ((double)(m - 1) <= lam) {
     // P(X <= m - 1) = sum_{k <= m - 1} p(k), from p(m - 1) down
     double t = exp_f64(-lam + (double)(m - 1) * ll - lgamma_int_f64((double)m));
+    {
+      const double il = 1.0 / lam;
+      double k = (double)(m - 1), ts = t, Ss = t;
+      while (ts > 1e-17 * Ss) {
+        const double c1 = k * il, c2 = c1 * ((k - 1.0) * il), c3 = (k - 2.0) * il, c4 = c3 * ((k - 3.0) * il);
+        Ss += ts * ((c1 + c2) + c2 * (c3 + c4));  // (a factor of 0 at k = 0 ends the products)
+        ts = ts * (c2 * c4);
+        k -= 4.0;
+        if (u <= Ss * (1.0 - POIS_SUM_MARGIN)) return m - 1;
+        if ((u - Ss * (1.0 + POIS_SUM_MARGIN)) * (lam - k) > ts * k * (1.0 + POIS_SUM_MARGIN)) return m;
+      }
+    }
     double S = t;
     for (int32_t k = m - 1; k > 0 && t > 1e-17 * S; --k) {
       t = t * (double)k / lam;
@@ -364,6 +387,19 @@ __device__ __noinline__ int32_t poisson_exact_f64(double lam, double u, int32_t 
   }
   // P(X >= m) = sum_{k >= m} p(k), from p(m) up; P(X <= m - 1) = 1 - that
   double t = exp_f64(-lam + (double)m * ll - lgamma_int_f64((double)m + 1.0));
+  {
+    const double v = 1.0 - u, l2 = lam * lam;  // (v exact)
+    double k = (double)m, ts = t, Ts = t;
+    while (ts > 1e-17 * Ts) {
+      const double a1 = k + 1.0, a2 = k + 2.0, a3 = k + 3.0, a4 = k + 4.0;
+      const double a34 = a3 * a4, r = lam / ((a1 * a2) * a34);
+      Ts += ts * (r * (a34 * (a2 + lam) + l2 * (a4 + lam)));
+      ts = ts * (r * (lam * l2));
+      k += 4.0;
+      if (Ts * (1.0 - POIS_SUM_MARGIN) > v + 1e-15) return m;
+      if ((v - 1e-15 - Ts * (1.0 + POIS_SUM_MARGIN)) * (k + 1.0 - lam) > ts * lam * (1.0 + POIS_SUM_MARGIN)) return m - 1;
+    }
+  }
   double T = t;
   for (int32_t k = m + 1; t > 1e-17 * T; ++k) {
     t = t * lam / (double)k;

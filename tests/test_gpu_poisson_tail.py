@@ -1,6 +1,8 @@
 """The far tail of the mixed-precision Poisson sampler, the FP64 search that
-decides it, and where that search ends (marked gpu)."""
+decides it and where that search ends; the FP64 sums that decide draws next to a
+value of the CDF (marked gpu)."""
 import math
+import zlib
 
 import numpy as np
 import pytest
@@ -43,3 +45,20 @@ def test_uniform_just_below_one_is_the_exact_inverse(native):
     k, _ = native.poisson_probe_mixed(lam, np.full(lam.size, U_BELOW, np.uint32))
     for l, n in zip(lam.astype(np.float64), k):
         assert special.pdtrc(n, l) <= 2.0 ** -24 * (1 + 1e-6) and special.pdtrc(n - 1, l) > 2.0 ** -24 * (1 - 1e-6), (l, n)
+
+
+# crc32 of the draws (int32) as the term-by-term FP64 sums alone decide them
+TERM_BY_TERM = {10.0: 2101785422, 11.5: 2358396442, 57.25: 1646697598, 300.0: 1699955642, 900.5: 2218100682,
+                5000.0: 3973358506, 30000.75: 3706015999, 65535.0: 2201492289}
+
+
+def _draws(native, lam):
+    words = np.random.default_rng(int(lam)).integers(0, 2 ** 32, 1 << 19, dtype=np.uint32)
+    return native.poisson_probe_mixed(np.full(words.size, lam, np.float32), words)
+
+
+@pytest.mark.parametrize("lam", TERM_BY_TERM)
+def test_decisions_are_those_of_the_term_by_term_sums(native, lam):
+    k, path = _draws(native, lam)
+    assert (path == 3).sum() > 20
+    assert zlib.crc32(k.astype("<i4").tobytes()) == TERM_BY_TERM[lam]
