@@ -249,8 +249,8 @@ typedef struct pst_launch {
                                  decide and four burst wavefronts; a simulation's SSA
                                  fallback burst (P3.py:71-151) moves through LDS to the
                                  paired burst wavefront and back.  0: they do not.  A plan
-                                 without a launch shape of its own pairs while one wavefront
-                                 per SIMD holds all its simulations */
+                                 without a launch shape of its own pairs while two
+                                 wavefronts per SIMD hold all its simulations */
   double kernel_ms;           /* kernel time of the chosen shape on the tuning horizon */
   double default_ms;          /* same for the library's default shape */
 } pst_launch;

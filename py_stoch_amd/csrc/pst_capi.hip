@@ -345,14 +345,17 @@ int lanes_for(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int
 }
 
 // Whether a launch of a tau-leaping network kernel runs its SSA bursts on
-// paired wavefronts when the launch shape leaves it open: yes while one
-// wavefront per SIMD holds every simulation (the burst wavefront then takes
+// paired wavefronts when the launch shape leaves it open: yes while two
+// wavefronts per SIMD hold every simulation (the burst wavefronts then take
 // issue slots that would stay empty) and a wavefront holds several simulations
 // (alone it never waits for another's burst), if the hand-off slots fit LDS.
 // Measured, one role / paired: Schloegl mixed 2048 simulations 5.3 / 4.5 ms,
-// 20,000 8.6 / 6.4, 65,536 10.9 / 7.8, 262,144 (four wavefronts per SIMD)
-// 31.0 / 33.5; Lotka-Volterra FP64 16,411 53 / 43, 65,536 107 / 93, 131,072 (to
-// t = 6) 60 / 65; 128 Schloegl simulations, one per wavefront, 3.1 / 3.9.
+// 20,000 8.6 / 6.4, 72,000 20.6 / 19.2, 100,003 20.7 / 21.8, 131,072 (two
+// wavefronts per SIMD) 25.8 / 26.6, 262,144 31.0 / 33.5; Lotka-Volterra mixed
+// 72,000 44.6 / 34.8, 100,003 45.4 / 43.5, 131,072 48.8 / 48.4, FP64 16,411
+// 53 / 43, 65,536 107 / 93, 100,003 158 / 132, 131,072 159 / 157; Schloegl FP64
+// 100,003 55.3 / 46.4, 131,072 56.1 / 56.9; 128 Schloegl simulations, one per
+// wavefront, 3.1 / 3.9.
 bool pair_by_default(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int L, int simds, int precision) {
   const pst::JobParams& P = jobs[ids[0]].p;
   if (P.method != PST_METHOD_TAU_LEAPING || L < 2 || waves_at(jobs, ids, L) > 2 * (int64_t)simds) return false;
@@ -394,12 +397,12 @@ int kernel_kind(const pst_job& J, const pst::HostNet& h) {
 // first need, asking for register use that fits kOccupancyWaves wavefronts
 // per SIMD.  A launch that needs more wavefronts than the plain build holds
 // resident uses the second build if it holds more: Schloegl tau-leaping,
-// 262,144 simulations (238 VGPRs, two wavefronts per SIMD, against 168 VGPRs
-// with a few spills, three): mixed 63.0 -> 61.4 ms, FP64 164.3 -> 153.0 ms.
-// Launches the plain build holds at once keep it: Lotka-Volterra with 65,536
-// simulations (one wavefront per SIMD) takes 57.6 ms plain and 66.1 ms with
-// the request.  Asking for four wavefronts per SIMD was slower than three on
-// every case.  Both builds give identical results.  (Fewer resident
+// 262,144 simulations, two / three / four wavefronts per SIMD: FP64 (to t = 5)
+// 70.0 / 65.6 / 68.9 ms, mixed (to t = 10) 47.5 / 47.6 / 42.7.  Four is the
+// better only there: Lotka-Volterra mixed, 262,144 to t = 2, 5.9 -> 6.5 ms from
+// three to four, Schloegl SSA mixed, 300,000 to t = 5, 29.4 -> 34.1, FP64 with 4
+// species and 5 reactions, 262,144, 11.8 -> 22.4.  Launches the plain build
+// holds at once keep it.  Both builds give identical results.  (Fewer resident
 // wavefronts than the limit is the separate waves_trim of the launch shape.)
 constexpr int kOccupancyWaves = 3;
 

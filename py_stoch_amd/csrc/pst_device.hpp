@@ -108,8 +108,7 @@ struct Work {
 //   SSA step            1 block  rho1 = U(w0,w1), rho2 = U(w2,w3)
 //   critical tau2/pick  1 block  rho1 = U(w0,w1), rho  = U(w2,w3)
 //   Poisson attempt     FP64: block b+j for reaction j, U = U(w0,w1),
-//                       V = U(w2,w3); mixed: block b + j/2, words 2(j%2),
-//                       2(j%2)+1
+//                       V = U(w2,w3); mixed: block b + j/4, word j%4
 struct Key {
   uint32_t k0, k1, s_lo, s_hi;
   __device__ __forceinline__ void init(uint64_t seed, uint64_t sim) {

@@ -13,14 +13,23 @@
 //
 // Per lane the driver keeps a mode -- DECIDE (next step is a leap decision,
 // P1_P2.py:96-294), SSA (inside a P3 burst, P3.py:71-151, or pure SSA) or
-// DONE.  Every pass of its loop runs one step for every active lane (the
-// engine's step() serves both modes with shared code), then, while at least
-// SSA_LANES_MIN lanes are in an SSA burst, up to `ssa_slice` further SSA-only
-// steps for them: a wavefront lasts as long as its slowest simulation, and a
-// burst taken one step per pass would add 100 passes to that simulation's
-// path (8 steps per pass: Lotka-Volterra 81 -> 70 ms, Schlogl 110 -> 76 ms).
-// A pass in which no lane decides runs up to 1 + ssa_slice SSA steps (2 +
-// 2 ssa_slice for pure SSA: 68 -> 66 ms on Schlogl, 65,536 simulations).
+// DONE.  A pass of its loop decides for the lanes in DECIDE (Engine::decide),
+// then takes SSA steps for those in a burst: 1 + ssa_slice, and more the more
+// lanes are in a burst than deciding.  A wavefront lasts as long as its
+// slowest simulation, and a burst taken one step per pass would add 100
+// passes to that simulation's path.
+//
+// SSA steps that cross no sample time and meet no rare case -- nearly all --
+// run in ssa_run: four random blocks at a time, then four steps whose results
+// are committed by selects, no branch in between.  The step's chain of
+// dependent operations is what bounds it (a dependent operation takes 9
+// cycles, a branch on a lane mask 50): Schloegl pure SSA, 100,003
+// simulations, mixed 80 -> 40 ms.  Other steps end the run and go through
+// Engine::ssa_step, the same arithmetic in general form.
+//
+// A launch with fewer than 64 simulations per wavefront, and the last
+// simulations of a wavefront (LaneForm), replicate each over a group of
+// lanes that share its draws.
 // Every simulation executes exactly the reference's sequence
 // (decision, burst of ssa_burst SSA steps, decision, ...); only the
 // interleaving of different simulations within a wavefront changes.

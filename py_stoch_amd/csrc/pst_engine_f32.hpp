@@ -5,13 +5,16 @@
 // SSA fallback burst and sampling rules, same wavefront-uniform loop.
 // Precision:
 //   FP32: propensities, a0 for the leap decision, mu / sigma^2, the Cao tau
-//         bound, Poisson means and the whole Poisson sampler (PTRS log-density
-//         test in a cancellation-free Stirling form), uniforms (24-bit, one
-//         Philox word each)
+//         bound, Poisson means and the Poisson samplers (inversions; PTRS, for
+//         means of 2^16 and above, with its log-density test in a
+//         cancellation-free Stirling form), uniforms (24-bit, one Philox word
+//         each)
 //   FP64: the simulation clock t, and the reaction choice, done as "first j
 //         with sum_{r<=j} a_r >= rho2 * a0" accumulated in FP64 so that FP32
-//         round-off cannot bias which reaction fires.  Poisson means of 2^22
-//         and above use the FP64 sampler (FP32 cannot resolve the integers).
+//         round-off cannot bias which reaction fires.  Poisson draws whose
+//         FP32 root lies next to an integer are decided in FP64, and means of
+//         2^22 and above use the FP64 sampler (FP32 cannot resolve the
+//         integers).
 // Transcendentals use the hardware v_log_f32 / v_exp_f32 / v_rcp_f32.  The
 // launch loop, work queue and lane modes are in pst_driver.hpp.
 #pragma once

@@ -188,7 +188,7 @@ std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
   // (WIDENING) where that pays: FP64 tau-leaping (Lotka-Volterra, 65,536
   // simulations, 93 -> 86 ms) and the SSA methods (Schloegl SSA FP64, 100,003:
   // 40.2 -> 36.4 ms); the mixed leap's draws are cheap next to what the two ways
-  // of drawing in one kernel cost (34.4 -> 35.2 ms).
+  // of drawing in one kernel cost (29.4 -> 30.3 ms).
   const bool widening = c.method != 0 || (precision == PST_PRECISION_FP64 && !group);
   s += std::string("  pst::") + (paired ? "run_driver_paired" : "run_driver") +
        "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>, pst::" +
