@@ -239,7 +239,8 @@ int pst_batch_plan_execute(pst_plan* plan, int32_t* const* O_dev, const int64_t*
 typedef struct pst_launch {
   int32_t lanes_shift;        /* simulations per wavefront = library choice >> lanes_shift */
   int32_t ssa_slice;          /* SSA steps per pass while lanes decide: 1 + ssa_slice, more the more
-                                 lanes are in a burst than deciding (up to 8 times as many) */
+                                 lanes are in a burst than deciding (up to 8 times as many;
+                                 64 times where no lane decides: the SSA methods) */
   int32_t waves_trim;         /* resident wavefronts per SIMD held back from the kernel's
                                  occupancy limit (at least one stays): with fewer lanes
                                  than simulations, the work queue refills lanes and a

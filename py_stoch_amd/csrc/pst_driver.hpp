@@ -666,14 +666,17 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
       }
       // SSA steps of the lanes inside a burst: more of them the more lanes are
       // in one than deciding (a burst of 100 steps taken 8 at a time waits
-      // through 13 decisions of the others); most if no lane decides (pure SSA,
-      // or every live lane inside a burst)
+      // through 13 decisions of the others); most if every live lane is inside
+      // a burst.  Where no lane ever decides, 512 at the default slice: only a
+      // lane whose simulation has ended waits for the others' (64 -> 512:
+      // birth-death, 1024 simulations, mixed 0.374 -> 0.360 ms, FP64 0.617 ->
+      // 0.604; Schloegl, 200,000, mixed 13.7 -> 13.1, table-driven 33.1 -> 32.1)
       const bool burst = mode == MODE_SSA && eng.F < f_stop;
       const unsigned long long ssa = __builtin_amdgcn_ballot_w64(burst);
       if (ssa != 0ull) {
         const int n_ssa = __builtin_popcountll(ssa);
         const int n_dec = __builtin_popcountll(__builtin_amdgcn_ballot_w64(mode == MODE_DECIDE));
-        const int times = n_ssa >= 8 * n_dec ? 8 : n_ssa >= 4 * n_dec ? 4 : n_ssa >= 2 * n_dec ? 2 : 1;
+        const int times = jr.method() != 0 ? 64 : n_ssa >= 8 * n_dec ? 8 : n_ssa >= 4 * n_dec ? 4 : n_ssa >= 2 * n_dec ? 2 : 1;
         mode = ssa_slice(jr, eng, cnt, mode, burst, times * (jr.p().ssa_slice + 1), t_stop, g);
       }
     } while (!wave_any(ran & ((mode == MODE_DONE) | (eng.F >= f_stop))));
