@@ -224,6 +224,14 @@ struct JobRef {
 #pragma unroll
     for (int j = 0; j < MP; ++j) a[j] = av[j];
   }
+  // props and their FP32 sum, of rounded products (they come from a loop)
+  __device__ __forceinline__ float props_sum(const int32_t (&x)[NP], const float (&k)[MP], float (&a)[MP]) const {
+    props<float>(x, k, a);
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < MP; ++j) sum += a[j];
+    return sum;
+  }
 
   // critical reactions (P1_P2.py:314-327, on V) as a bit mask; mu and sigma^2
   // of every species over the non-critical reactions and whether it has any
@@ -380,6 +388,58 @@ struct FixedRef {
       }
     }
   }
+  // propensity factors of reaction j, counted with their order
+  static constexpr int factors(int j) {
+    int n = 0;
+    for (int i = 0; i < kNP; ++i) n += Net::ord[i * kMP + j];
+    return n;
+  }
+  // props and their FP32 sum, in which each reaction's last product enters
+  // unrounded (one fused operation).  The sum decides between a leap and an SSA
+  // burst, so a bit of it can send a simulation another way: it is fused here,
+  // not left to the compiler, which fuses only if it keeps sum and products in
+  // one basic block (and in decide moved the sum behind a branch wherever two
+  // species change: 1 simulation of 8192 took another path).  The sum of hazard
+  // expressions is held in their block by the volatile asm.
+  __device__ __forceinline__ static float props_sum(const int32_t (&x)[kNP], const float (&k)[kKP], float (&a)[kMP]) {
+    float sum = 0.0f;
+    if constexpr (kCustom) {
+      Net::template props<float>(x, k, a);
+#pragma unroll
+      for (int j = 0; j < kMP; ++j) sum += a[j];
+      asm volatile("" : "+v"(sum));
+    } else {
+#pragma unroll
+      for (int j = 0; j < kMP; ++j) {
+        float v = k[j];
+        int left = factors(j);
+        if (left == 0) sum += v;
+#pragma unroll
+        for (int i = 0; i < kNP; ++i)
+          for (int q = 0; q < Net::ord[i * kMP + j]; ++q) {
+            const float f = (float)(x[i] - Net::stp[i * kMP + j] * q);
+            if (--left == 0) sum = __builtin_fmaf(v, f, sum);
+            v = v * f;
+          }
+        a[j] = v;
+      }
+    }
+    return sum;
+  }
+  // s + w aj for a term of mu or sigma^2.  FP32: fused for a reaction that can
+  // never be critical, else the product is rounded first (again one form for
+  // every build; it matters from net changes of 3 on).
+  static constexpr bool never_critical(int j) {
+    for (int i = 0; i < kNP; ++i)
+      if (V(i, j) < 0) return false;
+    return true;
+  }
+  __device__ __forceinline__ static double add_term(double s, int w, double aj, bool, bool on) {
+    return s + (on ? (double)w * aj : 0.0);
+  }
+  __device__ __forceinline__ static float add_term(float s, int w, float aj, bool never, bool on) {
+    return never ? __builtin_fmaf((float)w, aj, s) : s + (on ? (float)w * aj : 0.0f);
+  }
   template <class R>
   __device__ __forceinline__ static void sums(const int32_t (&x)[kNP], const R (&a)[kMP], int n_c, unsigned& crit,
                                               R (&mu)[kNP], R (&s2)[kNP], unsigned& any) {
@@ -404,8 +464,8 @@ struct FixedRef {
         const int v = V(i, j);
         if (v != 0) {
           const bool nc = !cr[j];
-          m += nc ? (R)v * a[j] : (R)0;
-          s += nc ? (R)(v * v) * a[j] : (R)0;
+          m = add_term(m, v, a[j], never_critical(j), nc);
+          s = add_term(s, v * v, a[j], never_critical(j), nc);
           some = some | nc;
         }
       }

@@ -329,10 +329,7 @@ struct EngineF32 {
       for (int r = 1; r < NA; ++r) B[r] = uk.block(bc + (uint64_t)r, 0);
     }
     float a[MP];
-    tab.template props<float>(x, k, a);
-    float a0 = 0.0f;
-#pragma unroll
-    for (int j = 0; j < MP; ++j) a0 += a[j];
+    const float a0 = tab.props_sum(x, k, a);
     // (products already rounded to FP32: not to be contracted into the sums below)
 #pragma unroll
     for (int j = 0; j < MP; ++j) asm("" : "+v"(a[j]));
