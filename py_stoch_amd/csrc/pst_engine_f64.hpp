@@ -75,10 +75,14 @@ __device__ __forceinline__ bool ptrs_fast_f64(const PtrsF64& P, double U, double
 }
 
 // The log-density test after a failed squeeze (kf >= 0, 0 < V <= 1, us > 0).
+// Without a branch: where the lanes of one meet again, hipcc 7.2 has put
+// constants back into registers before it switches the other lanes on again.
+// Those lanes then draw with what the register held (the table-driven kernel
+// for 16 x 16 with its 434 registers; a simulation without end).
 __device__ __forceinline__ bool ptrs_slow_f64(const PtrsF64& P, double V, double kf, double us) {
   const double invalpha = 1.1239 + 1.1328 / (P.b - 3.4);
   const double lhs = log_normal_f64(V) + log_normal_f64(invalpha) - log_normal_f64(P.a / (us * us) + P.b);
-  const double rhs = -P.lam + kf * P.loglam - lgamma_int_f64(kf + 1.0);
+  const double rhs = -P.lam + kf * P.loglam - lgamma_int_flat_f64(kf + 1.0);
   return lhs <= rhs;
 }
 
