@@ -98,6 +98,14 @@ __device__ __forceinline__ void load_params_vgpr(JobParams* dst, const JobParams
   __builtin_memcpy(dst, w, sizeof(JobParams));
 }
 
+// LDS accesses of some lanes of a wavefront before those of others: the
+// hardware keeps a wavefront's LDS operations in order, the compiler only where
+// it is told that another lane may read or write the same word.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 #ifndef __HIPCC_RTC__
 template <int NP, int MP>
 struct JobDev {
@@ -158,7 +166,9 @@ struct JobRef {
     vrange = lane < MP ? jd->tab.vrange[lane] : 0u;
     species = lane < NP ? jd->tab.species[lane] : 0u;
     const uint32_t* d = reinterpret_cast<const uint32_t*>(jd->tab.vrow);
+    wave_lds_sync();  // the job before's rows have been read
     if (lane < NP * MP / 4) rows()[lane] = d[lane];  // NP * MP / 4 <= 64; read by this wavefront only
+    wave_lds_sync();
     jp = &jd->p;
     load_params_vgpr(&P, jp);
   }

@@ -493,9 +493,11 @@ __device__ __forceinline__ void add_stats(Counters& cnt, const LaneGroup<FORM>& 
 }
 __device__ __forceinline__ void leave_stats(int lane, unsigned long long* __restrict__ stats) {
   uint32_t left = 0;
+  wave_lds_sync();  // every lane's share is in
   if (lane == 0)
     left = __hip_atomic_fetch_add(&wg_stats().waves, 0xffffffffu, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
   left = __builtin_amdgcn_readfirstlane(left);
+  wave_lds_sync();
   if (left == 1u && lane <= ST_EXACT) atomicAdd(&stats[lane], wg_stats().v[lane]);
 }
 
@@ -569,22 +571,27 @@ __device__ __forceinline__ void regroup(uint32_t* data, int first, int G, LaneGr
     const int to = first + __builtin_popcountll(leads & ((1ull << lane) - 1ull));
     IO::put(data, to, eng, sim, cnt.events - ev_start, lane, mode);
   }
+  wave_lds_sync();  // records and sample blocks are read by other lanes
   add_stats(cnt, g);
   g.set(lane, 64 / G);
   const int from = lane / G;
+  const bool takes = from < __builtin_popcountll(leads);
   mode = MODE_DONE;
-  if (from < __builtin_popcountll(leads)) {
+  int32_t w[BW];
+  if (takes) {
     unsigned long long ev;
     IO::get(data, first + from, eng, sim, ev, mode);
     ev_start = 0ull - ev;
     if (blocks) {  // the samples of the block in progress
       const int32_t* old = Out::lds() + (Out::slot() & ~63) + IO::job(data, first + from);
-      int32_t w[BW];
 #pragma unroll
       for (int i = 0; i < BW; ++i) w[i] = old[i * 256];
-#pragma unroll
-      for (int i = 0; i < BW; ++i) Out::lds()[i * 256 + Out::slot()] = w[i];
     }
+  }
+  wave_lds_sync();  // ... before the blocks and slots are written again
+  if (takes && blocks) {
+#pragma unroll
+    for (int i = 0; i < BW; ++i) Out::lds()[i * 256 + Out::slot()] = w[i];
   }
 }
 
@@ -757,6 +764,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
     int f_stop = range_stop(jr, f_end);
     g.set(lane, jr.cold().lanes);
     if (lane == 0) s_lanes[pair] = (uint32_t)(64 / g.G);
+    wave_lds_sync();  // before any lane of this wavefront sends
     for (;;) {
       // a burst handed back (ended simulations were recorded by the burst
       // lane); the lanes of a group take it together
@@ -795,6 +803,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
           regroup<Engine, PAIR_SLOTS>(s_data, pair * 64, G, g, lane, eng, sim, ev_start, cnt, mode,
                                       jr.p().layout == LAYOUT_BLOCKS);
           if (lane == 0) s_lanes[pair] = (uint32_t)(64 / G);
+          wave_lds_sync();
         }
       }
       if (!wave_any(mode != MODE_DONE)) {
@@ -805,6 +814,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
         f_stop = range_stop(jr, f_end);
         g.set(lane, jr.cold().lanes);
         if (lane == 0) s_lanes[pair] = (uint32_t)(64 / g.G);
+        wave_lds_sync();
         exhausted = false;
         continue;
       }

@@ -74,12 +74,6 @@ struct WaveLds {
   uint32_t vrow[WAVE_MAX_M][4];  // WaveTab::vrow of the current job
 };
 
-// LDS writes of some lanes visible to reads of others in the same wavefront
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -210,6 +204,7 @@ struct EngineWave {
 
   // the parts of a job's table that ssa_run keeps at hand
   __device__ __forceinline__ void load(const WaveJob& J, WaveLds& L, int lane) {
+    wave_lds_sync();  // the job before's net changes have been read
     fn = 0;
 #pragma unroll
     for (int r = 0; r < WAVE_R; ++r) {
