@@ -384,10 +384,11 @@ __device__ __forceinline__ int ssa_run(Ref& jr, Engine& eng, Counters& cnt, int 
     lim = left < (uint32_t)lim ? (int)left : lim;
   }
   if (P.method == 2) tstop = P.t_max < tstop ? P.t_max : tstop;
-  // a batch cannot reach the count limit from here
+  // lim steps, each changing a count by 127 at most, cannot reach the count limit
   bool go = on & (lim > 0) & (eng.t < tstop);
+  const int safe = COUNT_LIMIT - 127 * lim;
 #pragma unroll
-  for (int i = 0; i < Engine::NP; ++i) go = go & (eng.x[i] < COUNT_LIMIT - 127 * 64);
+  for (int i = 0; i < Engine::NP; ++i) go = go & (eng.x[i] < safe);
   bool stop = on & !go;  // the next step is not for this loop
   const Key uk = eng.key.scalar_seed(P.seed);  // a lane without a simulation may hold any key
   int n = 0;
