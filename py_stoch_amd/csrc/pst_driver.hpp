@@ -641,6 +641,9 @@ __device__ __forceinline__ void run_driver(const typename Ref::Dev* __restrict__
           mode = begin_sim(jr, eng, s, cnt, ev_start, resume != 0, f_stop);
         }
       }
+      // in a resumed range a lane may have taken a simulation that had ended: no
+      // reason to wait for the others, or to leave the job
+      if (resume != 0 && !exhausted && wave_any(want & (mode == MODE_DONE))) continue;
     }
     if (FORM == WIDENING && exhausted) {
       const int G = wider_group(g, __builtin_amdgcn_ballot_w64((mode != MODE_DONE) & g.lead()), group_cap(jr.n_reactions()));
@@ -793,6 +796,7 @@ __device__ __forceinline__ void run_driver_paired(const typename Ref::Dev* __res
             mode = begin_sim(jr, eng, s, cnt, ev_start, resume != 0, f_stop);
           }
         }
+        if (resume != 0 && !exhausted && wave_any(want & (mode == MODE_DONE))) continue;  // as in run_driver
       }
       // regroup when no simulation is away (its slot belongs to its lane): bursts
       // that start meanwhile wait
