@@ -199,7 +199,8 @@ void pst_plan_destroy(pst_plan* plan);
 /*
  * Re-key a plan's random stream for its next executions: simulation s then
  * draws from (seed, sim_offset + s).  Runs with disjoint id ranges are
- * independent samples of the same workload.
+ * independent samples of the same workload.  Pending sample ranges
+ * (pst_plan_execute_range) go on with the stream they were started on.
  */
 int pst_plan_set_stream(pst_plan* plan, uint64_t seed, uint64_t sim_offset);
 

@@ -296,6 +296,7 @@ struct PlanJob {
   std::vector<std::string> hazards;  // compiled hazard expressions (empty: mass action)
   uint32_t* d_state = nullptr;  // saved simulations between sample ranges (allocated on first use)
   int32_t state_words = 0;
+  uint64_t range_seed = 0;  // seed of the pending sample ranges: that of their first
 };
 
 template <int NP, int MP>
@@ -1102,7 +1103,15 @@ int pst_plan_execute_range(pst_plan* p, int32_t* const* O_dev, const int64_t* o_
   int count[pst::NUM_CLASSES];
   int n_wave = 0;
   int64_t wave_sims = 0;
+  // simulations that were started on one stream go on with it: a resumed one
+  // has its key in its saved state, and the launch's settings hold the same seed
+  // whatever pst_plan_set_stream has set for the next run
+  for (PlanJob& pj : p->jobs) {
+    if (p->range_pos == 0) pj.range_seed = pj.p.seed;
+    std::swap(pj.range_seed, pj.p.seed);
+  }
   rc = prepare_plan(p, O_dev, o_strides, flags_dev, s, true, count, &n_wave, &wave_sims);
+  for (PlanJob& pj : p->jobs) std::swap(pj.range_seed, pj.p.seed);
   if (rc != PST_OK) return rc;
   const pst::Range r = {f_end, p->range_pos > 0 ? 1 : 0};
   rc = enqueue_plan(p, s, count, n_wave, wave_sims, r, false);
