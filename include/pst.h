@@ -250,8 +250,9 @@ typedef struct pst_launch {
   int32_t burst_waves;        /* 1: tau-leaping network kernels run in workgroups of four
                                  decide and four burst wavefronts; a simulation's SSA
                                  fallback burst (P3.py:71-151) moves through LDS to the
-                                 paired burst wavefront and back.  0: they do not.  A plan
-                                 without a launch shape of its own pairs while two
+                                 paired burst wavefront and back.  0: they do not.  -1:
+                                 the library's choice, launch by launch, as in a plan
+                                 without a launch shape of its own: paired while two
                                  wavefronts per SIMD hold all its simulations */
   double kernel_ms;           /* kernel time of the chosen shape on the tuning horizon */
   double default_ms;          /* same for the library's default shape */
@@ -260,7 +261,7 @@ int pst_plan_autotune(pst_plan* plan, int32_t* const* O_dev, const int64_t* o_st
                       int32_t* const* flags_dev, void* stream, double fraction, pst_launch* chosen);
 /* Set a launch shape directly (a pst_launch of an earlier autotune):
  * 0 <= lanes_shift <= 6, 0 <= ssa_slice <= 63, 0 <= waves_trim <= 7,
- * burst_waves 0 or 1.  No reference counterpart. */
+ * burst_waves -1, 0 or 1.  No reference counterpart. */
 int pst_plan_set_launch(pst_plan* plan, int32_t lanes_shift, int32_t ssa_slice, int32_t waves_trim,
                         int32_t burst_waves);
 

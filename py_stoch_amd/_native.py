@@ -438,7 +438,9 @@ class Plan(_RangeMixin):
         _check(load().pst_plan_set_stream(self._h, int(seed), int(sim_offset)), "pst_plan_set_stream")
 
     def set_launch(self, lanes_shift, ssa_slice, waves_trim=0, burst_waves=0):
-        """Use this launch shape (e.g. one an autotune returned) for later executions."""
+        """Use this launch shape (e.g. one an autotune returned) for later executions;
+        burst_waves=-1 leaves the pairing to the library, as in a plan without a
+        shape of its own."""
         _check(load().pst_plan_set_launch(self._h, int(lanes_shift), int(ssa_slice), int(waves_trim),
                                           int(burst_waves)),
                "pst_plan_set_launch")
@@ -529,7 +531,9 @@ class BatchPlan(_RangeMixin):
                "pst_batch_plan_execute")
 
     def set_launch(self, lanes_shift, ssa_slice, waves_trim=0, burst_waves=0):
-        """Use this launch shape (e.g. one an autotune returned) for later executions."""
+        """Use this launch shape (e.g. one an autotune returned) for later executions;
+        burst_waves=-1 leaves the pairing to the library, as in a plan without a
+        shape of its own."""
         _check(load().pst_plan_set_launch(self._h, int(lanes_shift), int(ssa_slice), int(waves_trim),
                                           int(burst_waves)),
                "pst_plan_set_launch")

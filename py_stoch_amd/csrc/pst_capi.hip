@@ -1299,7 +1299,9 @@ int pst_plan_autotune(pst_plan* p, int32_t* const* O_dev, const int64_t* o_strid
     paired = paired || g.pair;
     single = single || !g.pair;
   }
-  const int def_bw = paired ? 1 : 0;
+  // the default shape as a caller can set it again: where it pairs some groups
+  // and others not, only as the library's choice
+  const int def_bw = paired && single ? -1 : paired ? 1 : 0;
   for (const PlanJob& pj : p->jobs) others = others || pj.fixed < 0;
   const int slices[3] = {3, 7, 15};
   for (int bw = 0; bw <= (paired || single ? 1 : 0) && rc == PST_OK; ++bw) {
@@ -1354,7 +1356,7 @@ int pst_plan_set_launch(pst_plan* p, int32_t lanes_shift, int32_t ssa_slice, int
   if (lanes_shift < 0 || lanes_shift > 6) return fail(PST_EINVAL, "lanes_shift %d outside [0, 6]", lanes_shift);
   if (ssa_slice < 0 || ssa_slice > 63) return fail(PST_EINVAL, "ssa_slice %d outside [0, 63]", ssa_slice);
   if (waves_trim < 0 || waves_trim > 7) return fail(PST_EINVAL, "waves_trim %d outside [0, 7]", waves_trim);
-  if (burst_waves < 0 || burst_waves > 1) return fail(PST_EINVAL, "burst_waves %d outside [0, 1]", burst_waves);
+  if (burst_waves < -1 || burst_waves > 1) return fail(PST_EINVAL, "burst_waves %d outside [-1, 1]", burst_waves);
   p->lanes_shift = lanes_shift;
   p->ssa_slice = ssa_slice;
   p->waves_trim = waves_trim;
