@@ -488,11 +488,18 @@ static int fixed_kernel(FixedBuild& b, int precision, const char* what) {
 // The build of a network kernel for a launch at the jobs' lane counts: SSA
 // bursts of tau-leaping jobs on paired wavefronts if the launch shape says so
 // (or leaves it open and pair_by_default); the occupancy build if the plain
-// build cannot hold the launch resident at once.
+// build cannot hold the launch resident at once.  Groups of lanes only while two
+// wavefronts per SIMD hold a tau-leaping launch (always, but for a launch shape
+// that halves the lanes of a large one): beyond that the SIMDs have other
+// wavefronts to fill a simulation's gaps with.  32 simulations per wavefront,
+// groups / one lane each: Schloegl mixed 262,144 50.4 / 35.5 ms, FP64 24.6 /
+// 23.0, Lotka-Volterra mixed 262,144 6.3 / 4.6, FP64 131,072 9.1 / 8.7; Schloegl
+// SSA FP64 131,072 11.5 / 12.9.
 static int choose_build(pst_plan* p, FixedGroup& g, int simds) {
   const int L = p->jobs[g.jobs[0]].p.lanes;
   int rc;
-  g.pair = p->jobs[g.jobs[0]].p.method == PST_METHOD_TAU_LEAPING &&
+  const bool leaping = p->jobs[g.jobs[0]].p.method == PST_METHOD_TAU_LEAPING;
+  g.pair = leaping &&
            (p->burst_waves == 1 ||
             (p->burst_waves < 0 && !g.pair_failed && pair_by_default(p->jobs, g.jobs, L, simds, p->precision)));
   if (g.pair) {
@@ -503,7 +510,7 @@ static int choose_build(pst_plan* p, FixedGroup& g, int simds) {
     g.pair = false;
     g_err[0] = 0;
   }
-  g.use = L < 64 ? BUILD_GROUP : BUILD_PLAIN;
+  g.use = L < 64 && !(leaping && waves_at(p->jobs, g.jobs, L) > 2 * (int64_t)simds) ? BUILD_GROUP : BUILD_PLAIN;
   if ((rc = fixed_kernel(g.build[g.use], p->precision, "network kernel: ")) != PST_OK) return rc;
   if (g.use == BUILD_GROUP) return PST_OK;
   const int plain = g.build[BUILD_PLAIN].k.blocks_per_cu;

@@ -121,3 +121,32 @@ def test_occupancy_build_takes_the_same_way(native):
     print("case: pinned lotka_volterra, occupancy build", flush=True)
     O, F = _run(native, case, (0, 7, 0, 0), 3 * U)
     assert _crc(O[:, :, :U], F[:U]) == PINNED["lotka_volterra"]
+
+
+def test_a_large_launch_at_half_the_lanes(native):
+    """Twice as many wavefronts as the launch needs, none of them with lanes to
+    share: no groups (which took 1.6 times the time), and the same way."""
+    case = _case("lotka_volterra")
+    tabs, rates, x0, kw = case
+    n = 4 * U
+    kw = dict(kw, n_sims=n, t_max=2.0, I=np.linspace(0, 2.0, 11).astype(np.float32))
+    plan = native.Plan(tabs, rates, x0, precision=native.PRECISION_MIXED, specialize=True, **kw)
+    O, F = DeviceArray((2, 11, n)), DeviceArray((n,))
+    try:
+        got, ms = [], []
+        for shift in (0, 1):
+            print("case: lotka_volterra %d, lanes_shift %d" % (n, shift), flush=True)
+            plan.set_launch(shift, 7, 0, 0)
+            times = []
+            for _ in range(4):
+                plan.execute(O.ptr.value, n, F.ptr.value)
+                times.append(plan.stats()["kernel_ms"])
+            got.append((O.get(), F.get()))
+            ms.append(min(times[1:]))
+        print("kernel ms", ms, flush=True)
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+        assert ms[1] < 1.4 * ms[0]
+    finally:
+        plan.close()
+        O.free()
+        F.free()
