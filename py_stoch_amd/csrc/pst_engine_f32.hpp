@@ -454,8 +454,10 @@ struct EngineF32 {
   static __device__ __forceinline__ Draw1 from_lane(const Draw1& d, int addr) { return {lane_get(d.nl, addr), lane_get(d.u, addr)}; }
 
   // One SSA step from state (x, t) with draw d: the reaction and the new time;
-  // false if the step needs step<true> (see ssa_run).  step<true>'s
-  // arithmetic; a0 = 0 gives an infinite or undefined time, which fails.
+  // false if the step needs ssa_step (see ssa_run).  ssa_step's arithmetic; a
+  // sum of 0 gives an infinite or undefined time, which fails.  A hazard
+  // expression may be negative: then the FP32 sum, which ends a simulation where
+  // it is 0, can be 0 where this one is not, and ssa_step decides.
   __device__ __forceinline__ bool ssa_try(const Ref& tab, const Draw1& d, double tstop, int& sel, double& t1) const {
     float a[MP];
     tab.template props<float>(x, k, a);
@@ -466,9 +468,14 @@ struct EngineF32 {
     t1 = t + (double)(d.nl * fast_rcp((float)asum));
     const double target = (double)d.u * asum;  // <= asum: the last sum always reaches it
     sel = 0;
+    bool ok = (t1 > t) & (t1 < tstop);
 #pragma unroll
     for (int j = 0; j < MP - 1; ++j) sel += (cum[j] < target) ? 1 : 0;
-    return (t1 > t) & (t1 < tstop);
+    if constexpr (Ref::kCustom) {
+#pragma unroll
+      for (int j = 0; j < MP; ++j) ok = ok & (a[j] >= 0.0f);
+    }
+    return ok;
   }
 
   // One attempt of the leap for the lanes with `on` -- see EngineF64::attempt

@@ -150,3 +150,18 @@ def test_a_large_launch_at_half_the_lanes(native):
         plan.close()
         O.free()
         F.free()
+
+
+def test_propensities_that_cancel_end_a_simulation(native):
+    """A hazard may turn negative.  A simulation ends where the FP32 sum of the
+    propensities is 0, here 1 + 1e8 - 1e8, also where the FP64 sum of the
+    reaction choice is not."""
+    spn = models._spn(1, [({0: 1}, {0: 2}, "parameter_0*species_0"), ({0: 1}, {0: 3}, "parameter_1*species_0"),
+                          ({0: 1}, {}, "parameter_1*species_0")], [1], [1.0, 1e8])
+    a = models.make_args(spn, E=[0], t_max=5.0, ita=6, U=200)
+    tabs = dict(tables_of(a), hazard_c=["C(0)*X(0)", "C(1)*X(0)", "-C(1)*X(0)"], n_params=2)
+    for method in (1, 2):
+        print("case: cancelling propensities, method %d" % method, flush=True)
+        O, F, st = native.simulate(tabs, np.array([1.0, 1e8]), a.x_0, method=method, precision=native.PRECISION_MIXED,
+                                   specialize=True, t_max=5.0, I=a.I, E=a.E, n_sims=200, seed=1, max_steps=50)
+        assert np.all(O == 1) and not F.any() and st["ssa_steps"] == 0
