@@ -24,7 +24,8 @@ struct NetTab {
   uint16_t vent[NP * MP];  // net changes V = Post - Pre (d_V, P1_P2.py:8): species | (uint8) value << 8
   uint32_t vrange[MP];     // reaction j's net changes: first | end << 16
   uint32_t species[NP];    // H (d_H, P1_P2.py:9) | H_type << 8 (P1_P2.py:10) | 1 << 16 if the species has any
-                           // Pre entry (I_rs, P1_P2.py:338-346) | recorded species E[i] << 24 (d_E, P1_P2.py:13)
+                           // Pre entry (I_rs, P1_P2.py:338-346)
+  uint32_t recorded[2];    // recorded species (d_E, P1_P2.py:13), four bits each
   int8_t vrow[MP * NP];    // V once more, dense and reaction-major: the change of every species by reaction j
 };
 
@@ -135,6 +136,10 @@ __device__ __forceinline__ T at(const T (&v)[N], int i) {
 // of code for 4 x 4 and 300 KB for 16 x 16, beyond the 64 KB instruction
 // cache, and walked the zero entries too.)  The net changes of a reaction
 // chosen per lane are read from a dense copy in LDS.
+// v_readlane reads lanes whether they are on or not, and a copy the register
+// allocator makes where some are off leaves theirs undefined: lists are read
+// only where the whole wavefront is on.  What branches on a lane mask need (the
+// recorded species, net changes) is the same in every lane, or in LDS.
 template <int NP, int MP>
 struct JobRef {
   static constexpr int kNP = NP, kMP = MP;
@@ -145,6 +150,7 @@ struct JobRef {
   using Dev = JobDev<NP, MP>;
   static constexpr int EW = (NP * MP / 2 + 63) / 64;  // registers of an entry list
   uint32_t fac[EW], vent[EW], vrange, species;
+  uint64_t recorded;
   JobParams P;
   const JobParams* jp;
   __device__ __forceinline__ const JobParams& cold() const { return cold_params(jp); }
@@ -165,6 +171,7 @@ struct JobRef {
     }
     vrange = lane < MP ? jd->tab.vrange[lane] : 0u;
     species = lane < NP ? jd->tab.species[lane] : 0u;
+    recorded = jd->tab.recorded[0] | ((uint64_t)jd->tab.recorded[1] << 32);
     const uint32_t* d = reinterpret_cast<const uint32_t*>(jd->tab.vrow);
     wave_lds_sync();  // the job before's rows have been read
     if (lane < NP * MP / 4) rows()[lane] = d[lane];  // NP * MP / 4 <= 64; read by this wavefront only
@@ -187,7 +194,7 @@ struct JobRef {
   __device__ __forceinline__ int Hv(int i) const { return (int)(word(species, i) & 0xffu); }
   __device__ __forceinline__ int Htv(int i) const { return (int)((word(species, i) >> 8) & 0xffu); }
   __device__ __forceinline__ bool Irs(int i) const { return (word(species, i) >> 16) & 1u; }
-  __device__ __forceinline__ int Ev(int q) const { return (int)(word(species, q) >> 24); }
+  __device__ __forceinline__ int Ev(int q) const { return (int)((uint32_t)(recorded >> (4 * q)) & 15u); }
 
   // body(i) for every species, rolled (i is wavefront-uniform: index arrays with at())
   template <class F>
@@ -540,8 +547,8 @@ inline NetTab<NP, MP> make_tab(const HostNet& h) {
     t.vrange[j] = (uint32_t)v0 | ((uint32_t)nv << 16);
   }
   for (int i = 0; i < h.N; ++i)
-    t.species[i] = (uint32_t)h.H[i] | ((uint32_t)h.Ht[i] << 8) | ((uint32_t)(h.irs[i] != 0) << 16) |
-                   (i < h.kappa ? (uint32_t)h.E[i] << 24 : 0u);
+    t.species[i] = (uint32_t)h.H[i] | ((uint32_t)h.Ht[i] << 8) | ((uint32_t)(h.irs[i] != 0) << 16);
+  for (int q = 0; q < h.kappa; ++q) t.recorded[q / 8] |= (uint32_t)h.E[q] << (4 * (q % 8));
   return t;
 }
 

@@ -276,8 +276,8 @@ struct StateIO {
 
 // Engine interface (see EngineF64 / EngineF32):
 //   int  start(job, sim)            -> initial mode, state loaded
-//   int  decide(job, cnt, on, group), int ssa_step(job, cnt) -> next
-//     mode (DONE may set flag)
+//   int  decide(job, cnt, on, group), int ssa_step(job, cnt, propensities) ->
+//     next mode (DONE may set flag)
 //   Draw1 ssa_draw(key, c), bool ssa_try(job, draw, tstop, sel, t1): one
 //     ordinary SSA step (ssa_run)
 //   int  flag
@@ -468,7 +468,9 @@ __device__ __forceinline__ int ssa_slice(Ref& jr, Engine& eng, Counters& cnt, in
   bool general;
   mode = ssa_run(jr, eng, cnt, mode, on, cap, t_stop, general, g);
   if (wave_any(general)) {
-    if (general) mode = eng.ssa_step(jr, cnt);
+    typename Engine::Real a[Engine::MP];
+    jr.template props<typename Engine::Real>(eng.x, eng.k, a);  // (with every lane on: JobRef)
+    if (general) mode = eng.ssa_step(jr, cnt, a);
   }
   return mode;
 }

@@ -150,6 +150,7 @@ __device__ __noinline__ Draw ptrs_wide(uint32_t k0, uint32_t k1, uint32_t s_lo, 
 // Per-lane state and steps of one mixed-precision simulation.
 template <class Ref>
 struct EngineF32 {
+  using Real = float;
   static constexpr int NP = Ref::kNP, MP = Ref::kMP;
   static constexpr int NB = (MP + 3) / 4;  // Philox blocks of a leap attempt
   // The larger tables take their draws one after the other through one copy
@@ -215,7 +216,7 @@ struct EngineF32 {
   // One direct-method SSA step in its general form -- see EngineF64::ssa_step;
   // the arithmetic is FP32 except the clock and the cumulative sum of the
   // reaction choice.
-  __device__ __forceinline__ int ssa_step(const Ref& tab, Counters& cnt) {
+  __device__ __forceinline__ int ssa_step(const Ref& tab, Counters& cnt, const float (&a)[MP]) {
     const auto& P = tab.p();
     if (P.method == 2 && !(t < P.t_max)) {
       fill_rest(tab, true, cnt);
@@ -228,8 +229,6 @@ struct EngineF32 {
       return MODE_DONE;
     }
     nsteps += 1;
-    float a[MP];
-    tab.template props<float>(x, k, a);
     float a0 = 0.0f;
 #pragma unroll
     for (int j = 0; j < MP; ++j) a0 += a[j];

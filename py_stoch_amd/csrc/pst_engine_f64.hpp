@@ -89,6 +89,7 @@ __device__ __forceinline__ bool ptrs_slow_f64(const PtrsF64& P, double V, double
 // Per-lane state and steps of one FP64 simulation.
 template <class Ref>
 struct EngineF64 {
+  using Real = double;
   static constexpr int NP = Ref::kNP, MP = Ref::kMP;
   double k[Ref::kKP];  // rates row: per-reaction constants, or hazard parameters
   int32_t x[NP];
@@ -146,9 +147,9 @@ struct EngineF64 {
   }
 
   // One direct-method SSA step (P3.py:73-149; gillespie.py:70-149 for pure
-  // SSA) in its general form; ordinary steps run in ssa_run (pst_driver.hpp).
-  // Returns the next mode.
-  __device__ __forceinline__ int ssa_step(const Ref& tab, Counters& cnt) {
+  // SSA) in its general form, from the propensities of the present state;
+  // ordinary steps run in ssa_run (pst_driver.hpp).  Returns the next mode.
+  __device__ __forceinline__ int ssa_step(const Ref& tab, Counters& cnt, const double (&a)[MP]) {
     const auto& P = tab.p();
     const int M = P.M;
     if (P.method == 2 && !(t < P.t_max)) {
@@ -163,8 +164,6 @@ struct EngineF64 {
       return MODE_DONE;
     }
     nsteps += 1;
-    double a[MP];
-    tab.template props<double>(x, k, a);
     double a0 = 0.0;
 #pragma unroll
     for (int j = 0; j < MP; ++j) a0 = a0 + a[j];
