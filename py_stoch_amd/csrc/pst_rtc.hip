@@ -6,6 +6,7 @@
 #include <sys/stat.h>
 #include <unistd.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -189,7 +190,14 @@ std::string rtc_source(const HostNet& net, const JobParams& c, int precision,
   // simulations, 93 -> 86 ms) and the SSA methods (Schloegl SSA FP64, 100,003:
   // 40.2 -> 36.4 ms); the mixed leap's draws are cheap next to what the two ways
   // of drawing in one kernel cost (29.4 -> 30.3 ms).
-  const bool widening = c.method != 0 || (precision == PST_PRECISION_FP64 && !group);
+  // The states on the move need LDS, 256 bytes a word (rates, counts, 23 more)
+  // beside the gathered samples; with more of it than lets two workgroups on a
+  // compute unit the lanes stay as they are (beyond 62 FP64 rates with four
+  // recorded species; with 256 the kernel would not fit at all).  Paired
+  // wavefronts have their hand-off slots for it.
+  const int words = c.n_rates * (precision == PST_PRECISION_FP64 ? 2 : 1) + N + 23;
+  const bool fits = paired || words * 256 + std::min(net.kappa, 4) * 8192 <= 64 * 1024;
+  const bool widening = fits && (c.method != 0 || (precision == PST_PRECISION_FP64 && !group));
   s += std::string("  pst::") + (paired ? "run_driver_paired" : "run_driver") +
        "<pst::PST_ENGINE<pst::FixedRef<pst::NetGen>>, pst::FixedRef<pst::NetGen>, pst::" +
        (widening ? "WIDENING" : group ? "GROUPED" : "ONE") + ">(jobs, n_jobs, queue, stats, "
