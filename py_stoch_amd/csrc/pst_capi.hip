@@ -840,10 +840,11 @@ int pst_batch_plan_create(const pst_job* jobs, int32_t n_jobs, pst_plan** out) {
     for (int q : g.jobs) p->jobs[q].p.lanes = L;
     const int rc2 = choose_build(p, g, cu * 4);
     if (rc2 != PST_OK) {
-      pst_plan_destroy(p);
+      const int job = g.jobs[0];
       char msg[sizeof(g_err)];
       std::snprintf(msg, sizeof(msg), "%s", g_err);
-      return fail(rc2, "job %d: %.480s", g.jobs[0], msg);
+      pst_plan_destroy(p);
+      return fail(rc2, "job %d: %.480s", job, msg);
     }
   }
   if ((e = hipEventCreate(&p->ev0)) != hipSuccess || (e = hipEventCreate(&p->ev1)) != hipSuccess) {
