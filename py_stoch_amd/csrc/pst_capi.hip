@@ -405,7 +405,14 @@ int kernel_kind(const pst_job& J, const pst::HostNet& h) {
 // species and 5 reactions, 262,144, 11.8 -> 22.4.  Launches the plain build
 // holds at once keep it.  Both builds give identical results.  (Fewer resident
 // wavefronts than the limit is the separate waves_trim of the launch shape.)
+// Mixed tau-leaping kernels of networks so large that the plain build holds one
+// wavefront per SIMD ask for two: at three most of a decision's values are
+// spilled.  Two / three, 70,000 and 262,144 simulations: 10 reactions 5.5 / 20.5
+// and 11.3 / 51.1 ms, 12 reactions 1.7 / 3.2 and 2.9 / 5.4, 9 reactions 1.0 / 1.7
+// and 2.0 / 3.7; with 7 reactions 0.42 / 0.48 and 1.00 / 0.95.  Their FP64
+// kernels spill less: 10 reactions 13.5 / 13.5 and 30.3 / 23.3.
 constexpr int kOccupancyWaves = 3;
+constexpr int kOccupancyWavesLarge = 2;
 
 // A plan with several kernel launches (size classes, network groups, the
 // large-network kernel) spreads them over the caller's stream and up to
@@ -418,9 +425,9 @@ constexpr int kOccupancyWaves = 3;
 constexpr int kSideStreams = 3;
 
 // builds of a specialised kernel: one simulation per lane, the same compiled
-// for kOccupancyWaves wavefronts per SIMD, a group of lanes per simulation, and
+// for kOccupancyWaves or kOccupancyWavesLarge wavefronts per SIMD, a group of lanes per simulation, and
 // decide + burst wavefronts with one simulation or a group
-enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_GROUP, BUILD_PAIR, BUILD_PAIR_GROUP, NUM_BUILDS };
+enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_OCC_LARGE, BUILD_GROUP, BUILD_PAIR, BUILD_PAIR_GROUP, NUM_BUILDS };
 struct FixedBuild {
   std::string source;
   pst::RtcForm form = pst::RTC_PLAIN;
@@ -515,8 +522,9 @@ static int choose_build(pst_plan* p, FixedGroup& g, int simds) {
   if (g.use == BUILD_GROUP) return PST_OK;
   const int plain = g.build[BUILD_PLAIN].k.blocks_per_cu;
   if (waves_at(p->jobs, g.jobs, L) <= (int64_t)plain * simds) return PST_OK;
-  if ((rc = fixed_kernel(g.build[BUILD_OCC], p->precision, "network kernel (occupancy build): ")) != PST_OK) return rc;
-  if (g.build[BUILD_OCC].k.blocks_per_cu > plain) g.use = BUILD_OCC;
+  const int occ = leaping && p->precision == PST_PRECISION_MIXED && plain == 1 ? BUILD_OCC_LARGE : BUILD_OCC;
+  if ((rc = fixed_kernel(g.build[occ], p->precision, "network kernel (occupancy build): ")) != PST_OK) return rc;
+  if (g.build[occ].k.blocks_per_cu > plain) g.use = occ;
   return PST_OK;
 }
 
@@ -823,6 +831,7 @@ int pst_batch_plan_create(const pst_job* jobs, int32_t n_jobs, pst_plan** out) {
         FixedBuild* b = p->fixed[g].build;
         b[BUILD_PLAIN].source = std::move(src);
         b[BUILD_OCC].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, kOccupancyWaves);
+        b[BUILD_OCC_LARGE].source = pst::rtc_source(pj.net, P, p->precision, pj.hazards, kOccupancyWavesLarge);
         const pst::RtcForm forms[] = {pst::RTC_GROUP, pst::RTC_PAIRED, pst::RTC_PAIRED_GROUP};
         for (int i = 0; i < 3; ++i) {
           b[BUILD_GROUP + i].form = forms[i];
