@@ -251,17 +251,21 @@ __device__ __forceinline__ double lgamma_int_f64(double x) {  // x = k + 1
   return (x - 0.5) * log_f64(x) - x + 0.9189385332046727417803297 + ser;
 }
 
-// lgamma_int_f64 for finite x, the same bits without a branch (both sides
-// computed): see ptrs_slow_f64.
+// lgamma_int_f64 for finite x, the same bits without a branch on a lane mask:
+// see ptrs_slow_f64.  Values below 10.5, rare at large means, only where the
+// wavefront has one.
 __device__ __forceinline__ double lgamma_int_flat_f64(double x) {
   const double r = 1.0 / x;
   const double r2 = r * r;
   const double ser = r * (1.0 / 12.0 - r2 * (1.0 / 360.0 - r2 * (1.0 / 1260.0 - r2 * (1.0 / 1680.0))));
-  const double big = (x - 0.5) * log_normal_f64(x) - x + 0.9189385332046727417803297 + ser;
-  double small = 0.0;
+  double v = (x - 0.5) * log_normal_f64(x) - x + 0.9189385332046727417803297 + ser;
+  const bool low = x < 10.5;
+  if (__builtin_amdgcn_ballot_w64(low) != 0ull) {
+    v = low ? 0.0 : v;
 #pragma unroll
-  for (int k = 2; k < 10; ++k) small = x == (double)(k + 1) ? logfact_small(k) : small;
-  return x < 10.5 ? small : big;
+    for (int k = 2; k < 10; ++k) v = x == (double)(k + 1) ? logfact_small(k) : v;
+  }
+  return v;
 }
 
 // __float2int_rn (P1_P2.py:572): round half to even; NaN -> 0, clamped.
