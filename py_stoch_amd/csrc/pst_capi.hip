@@ -317,22 +317,28 @@ void pack_jobs(const std::vector<PlanJob>& jobs, int cls, std::vector<unsigned c
 
 // Simulations per wavefront when `need(L)` wavefronts hold L each: 64 unless
 // the launch holds fewer than 64 simulations per SIMD, then the smallest power
-// of two that needs (up to a tenth more) no more wavefronts than the chip has
-// SIMDs.  A wavefront issues the same instructions whatever its lane count, so
+// of two that needs no more wavefronts than the chip has SIMDs (for tau-leaping
+// without a step budget, up to a tenth more).  A wavefront issues the same instructions whatever its lane count, so
 // spreading a small launch over every SIMD costs nothing per wavefront and
 // leaves each with fewer divergent paths, a shorter slowest-lane tail and
 // lanes that share one simulation's work.  The tenth keeps a launch just
 // beyond a power of two from running on half the SIMDs: Lotka-Volterra,
 // 16,411 simulations, 32 -> 16 per wavefront (513 -> 1026 wavefronts on 1024
-// SIMDs): FP64 72 -> 53 ms, mixed 35.6 -> 27.6 ms; at twice as many wavefronts
-// as SIMDs the second one per SIMD costs as much as it hides (Schloegl SSA,
-// 8192 simulations, 8 -> 4: 3.6 -> 4.1 ms).
+// SIMDs): FP64 72 -> 53 ms, mixed 35.6 -> 27.6 ms.  The few simulations beyond
+// the SIMDs start when others end, which costs little where run lengths differ
+// and a whole run where a step budget makes them equal (300 steps of the same,
+// 16,400 simulations, mixed 0.87 ms with the tenth and 0.63 without; table-
+// driven, 8 reactions, 1000 steps, 33,000: 8.8 / 5.3); the SSA methods gain
+// nothing from more than four lanes (Schloegl SSA, 17,900, mixed 3.9 / 3.5,
+// FP64 6.6 / 5.7; birth-death, table-driven, 33,000, mixed 0.43 / 0.28).
 template <class Need>
-int spread_lanes(Need need, int simds) {
+int spread_lanes(Need need, int simds, bool tenth) {
+  const int64_t limit = (int64_t)simds * (tenth ? 11 : 10);
   int L = 64;
-  while (L > 1 && need(L / 2) * 10 <= (int64_t)simds * 11) L /= 2;
+  while (L > 1 && need(L / 2) * 10 <= limit) L /= 2;
   return L;
 }
+bool spread_tenth(const pst::JobParams& P) { return P.method == PST_METHOD_TAU_LEAPING && P.max_steps == 0; }
 
 // wavefronts of the jobs `ids` at L simulations each
 int64_t waves_at(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int L) {
@@ -342,7 +348,9 @@ int64_t waves_at(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, 
 }
 
 int lanes_for(const std::vector<PlanJob>& jobs, const std::vector<int>& ids, int simds) {
-  return spread_lanes([&](int L) { return waves_at(jobs, ids, L); }, simds);
+  bool tenth = true;
+  for (int q : ids) tenth = tenth && spread_tenth(jobs[q].p);
+  return spread_lanes([&](int L) { return waves_at(jobs, ids, L); }, simds, tenth);
 }
 
 // Whether a launch of a tau-leaping network kernel runs its SSA bursts on
@@ -1542,8 +1550,6 @@ int pst_run_noalloc(const pst_network* net, const pst_config* cfg, const double*
   if ((rc = scratch_on_device(dev, &base)) != PST_OK) return rc;
 
   const int simds = cu * 4;
-  // simulations per wavefront, as for a plan
-  const int L = spread_lanes([&](int l) { return ((int64_t)c.n_sims + l - 1) / l; }, simds);
   pst::JobParams P;
   std::memset(&P, 0, sizeof(P));
   P.N = h.N;
@@ -1556,9 +1562,11 @@ int pst_run_noalloc(const pst_network* net, const pst_config* cfg, const double*
   P.n_sims = c.n_sims;
   P.sims_per_set = c.sims_per_set;
   P.ssa_slice = kSsaSlice;
-  P.lanes = L;
   P.n_rates = h.M;
   P.max_steps = (uint32_t)c.max_steps;
+  // simulations per wavefront, as for a plan
+  const int L = spread_lanes([&](int l) { return ((int64_t)c.n_sims + l - 1) / l; }, simds, spread_tenth(P));
+  P.lanes = L;
   P.eta = c.eta;
   P.t_max = c.t_max;
   P.seed = c.seed;
