@@ -219,24 +219,26 @@ struct JobRef {
     for (int j = 0; j < MP; ++j) av[j] = (R)0;
     const int n = n_reactions();
     R v = k[0];
-    // one trip per listed factor
+    // one trip per listed species, with a branch only for orders above 1 (a
+    // uniform branch costs ~50 cycles, a select 9): with branches for order 0 and
+    // for the last of a reaction too, 8 reactions, 262,144 simulations, took 34.2
+    // ms mixed and 35.7 FP64, now 31.3 and 31.1; Schloegl 39.7 / 40.1, now 38.0 /
+    // 38.0.  One entry per factor instead of the inner loop: 47.5 / 45.4.
 #pragma unroll 1
     for (int e = 0, j = 0; j < n; ++e) {
       const uint32_t w = entry(fac, e);
       const int order = (int)(w >> 8);
-      if (order > 0) {
-        const int32_t xi = at<int32_t, NP>(x, (int)(w & 31u));
-        v = v * (R)xi;
-        if (order > 1) {
-          const int step = (int)((w >> 5) & 1u);
-          for (int q = 1; q < order; ++q) v = v * (R)(xi - step * q);
-        }
+      const int32_t xi = at<int32_t, NP>(x, (int)(w & 31u));
+      v = v * (R)(order > 0 ? xi : 1);
+      if (order > 1) {
+        const int step = (int)((w >> 5) & 1u);
+        for (int q = 1; q < order; ++q) v = v * (R)(xi - step * q);
       }
-      if (w & 64u) {
-        av[j] = v;
-        j += 1;
-        v = at<R, MP>(k, j & (MP - 1));
-      }
+      av[j] = v;
+      const bool last = (w & 64u) != 0u;
+      j += last ? 1 : 0;
+      const R kj = at<R, MP>(k, j & (MP - 1));
+      v = last ? kj : v;
     }
 #pragma unroll
     for (int j = 0; j < MP; ++j) a[j] = av[j];
