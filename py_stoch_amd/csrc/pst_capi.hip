@@ -318,10 +318,11 @@ void pack_jobs(const std::vector<PlanJob>& jobs, int cls, std::vector<unsigned c
 // Simulations per wavefront when `need(L)` wavefronts hold L each: 64 unless
 // the launch holds fewer than 64 simulations per SIMD, then the smallest power
 // of two that needs no more wavefronts than the chip has SIMDs (for tau-leaping
-// without a step budget, up to a tenth more).  A wavefront issues the same instructions whatever its lane count, so
-// spreading a small launch over every SIMD costs nothing per wavefront and
-// leaves each with fewer divergent paths, a shorter slowest-lane tail and
-// lanes that share one simulation's work.  The tenth keeps a launch just
+// without a step budget, up to a tenth more).  A wavefront issues the same
+// instructions whatever its lane count, so spreading a small launch over every
+// SIMD costs nothing per wavefront and leaves each with fewer divergent paths,
+// a shorter slowest-lane tail and lanes that share one simulation's work.  The
+// tenth keeps a launch just
 // beyond a power of two from running on half the SIMDs: Lotka-Volterra,
 // 16,411 simulations, 32 -> 16 per wavefront (513 -> 1026 wavefronts on 1024
 // SIMDs): FP64 72 -> 53 ms, mixed 35.6 -> 27.6 ms.  The few simulations beyond
@@ -433,8 +434,9 @@ constexpr int kOccupancyWavesLarge = 2;
 constexpr int kSideStreams = 3;
 
 // builds of a specialised kernel: one simulation per lane, the same compiled
-// for kOccupancyWaves or kOccupancyWavesLarge wavefronts per SIMD, a group of lanes per simulation, and
-// decide + burst wavefronts with one simulation or a group
+// for kOccupancyWaves or kOccupancyWavesLarge wavefronts per SIMD, a group of
+// lanes per simulation, and decide + burst wavefronts with one simulation or a
+// group
 enum { BUILD_PLAIN = 0, BUILD_OCC, BUILD_OCC_LARGE, BUILD_GROUP, BUILD_PAIR, BUILD_PAIR_GROUP, NUM_BUILDS };
 struct FixedBuild {
   std::string source;
